@@ -185,14 +185,12 @@ int64_t hif8_k_pad(int64_t K) { return (K + 7) / 8 * 8; }
 
 size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// int8 / fp8 B given [K, N]: for large problems the whole org B is transposed to [N, K] in the workspace first,
-// so the GEMM copies both operands straight into LDS (the transpose costs 2 K N bytes of traffic; the in-loop byte
-// transpose of the [K, N] path roughly halves the GEMM's rate).  Below the 256 x 256 tile sizes (M or N < 1024) an
-// int8 B [K, N] with N % 16 == 0 is not transposed: its GEMM copies the K rows into LDS and reads them with LDS
-// transpose reads.
-bool bytes_transposes_b(const ascq_matmul_s* h)
+// int8 / fp8 B given [K, N] is read in place, but ascq_matmul_workspace_size keeps the N K bytes that it has always
+// reported at these sizes (earlier kernels transposed B there), and a handle holds them as before: callers' checks,
+// buffers and the scratch limit of the allocation-free form rely on the figure.
+bool bytes_reserves_b(const ascq_matmul_s* h)
 {
-    if (h->ty.b_format == ASCQ_FORMAT_NZ) return false;  // converted from NZ instead (bytes_nz_b)
+    if (h->ty.b_format == ASCQ_FORMAT_NZ) return false;
     if (kind_of(h->ty) == K_INT8 && h->N % 16 == 0 && (h->M < 1024 || h->N < 1024)) return false;
     return !h->trans_b && h->M >= 512 && h->N % 16 == 0 && h->K % 16 == 0;
 }
@@ -204,10 +202,10 @@ bool bytes_transposes_a(const ascq_matmul_s* h) { return h->trans_a != 0; }
 // int8 / fp8 B in the NZ fractal layout: converted to a K-contiguous [N, K] copy in the workspace at every IterateAll
 bool bytes_nz_b(const ascq_matmul_s* h) { return h->ty.b_format == ASCQ_FORMAT_NZ; }
 
-// the operand copies of an int8 / fp8 Matmul (transposed or NZ-converted B, transposed A)
+// the operand copies of an int8 / fp8 Matmul (NZ-converted B, transposed A)
 size_t bytes_operands(const ascq_matmul_s* h)
 {
-    size_t need = bytes_transposes_b(h) || bytes_nz_b(h) ? align256((size_t)h->N * (size_t)h->K) : 0;
+    size_t need = bytes_nz_b(h) ? align256((size_t)h->N * (size_t)h->K) : 0;
     if (bytes_transposes_a(h)) need += align256((size_t)h->M * (size_t)h->K);
     return need;
 }
@@ -215,7 +213,8 @@ size_t bytes_operands(const ascq_matmul_s* h)
 // ... then, for decode-sized batches, the accumulators of the K split across workgroups
 size_t bytes_workspace(const ascq_matmul_s* h)
 {
-    const int tb = h->trans_b || bytes_transposes_b(h) || bytes_nz_b(h);  // B as the GEMM sees it
+    if (bytes_reserves_b(h)) return align256((size_t)h->N * (size_t)h->K) + bytes_operands(h);  // (M >= 512: no split)
+    const int tb = h->trans_b || bytes_nz_b(h);  // B as the GEMM sees it
     return bytes_operands(h) + align256(ascq::decode_split_ws_bytes(h->M, h->N, h->K, tb));
 }
 
@@ -273,7 +272,7 @@ ascq_status split_region(ascq_matmul_s* h, int64_t m, int64_t n, int64_t k, uint
 {
     *ws = nullptr;
     *bytes = 0;
-    const int tb = h->trans_b || bytes_transposes_b(h) || bytes_nz_b(h);  // B as the GEMM sees it
+    const int tb = h->trans_b || bytes_nz_b(h);  // B as the GEMM sees it
     const size_t need = ascq::decode_split_ws_bytes(m, n, k, tb);
     if (need == 0 || en_atomic != 0) return ASCQ_OK;
     const size_t off = bytes_operands(h);
@@ -306,8 +305,8 @@ ascq_status prepare_byte_operands(ascq_matmul_s* h, hipStream_t st, ByteOperands
     o.ldb = h->trans_b ? h->K : h->N;
     o.trans_a = h->trans_a;
     o.trans_b = h->trans_b;
-    const bool tb = bytes_transposes_b(h), ta = bytes_transposes_a(h), nz = bytes_nz_b(h);
-    if (!tb && !ta && !nz) return ASCQ_OK;
+    const bool ta = bytes_transposes_a(h), nz = bytes_nz_b(h);
+    if (!ta && !nz && !bytes_reserves_b(h)) return ASCQ_OK;
     ascq_status s = ensure_workspace(h);
     if (s != ASCQ_OK) return s;
     uint8_t* ws = (uint8_t*)h->ws;
@@ -315,14 +314,6 @@ ascq_status prepare_byte_operands(ascq_matmul_s* h, hipStream_t st, ByteOperands
         hipError_t e = h->trans_b ? ascq::launch_nz_to_nd(ws, h->b, 1, 1, h->N, h->K, 0, st)
                                   : ascq::launch_nz_to_nd(ws, h->b, 1, 1, h->K, h->N, 1, st);
         if (e != hipSuccess) return hip_status(e, "NZ B to ND");
-        o.B = ws;
-        o.ldb = h->K;
-        o.trans_b = 1;
-        ws += align256((size_t)h->N * (size_t)h->K);
-    }
-    if (tb) {  // B [K, N] -> [N, K]
-        hipError_t e = ascq::launch_transpose_i8(ws, (const uint8_t*)h->b, h->K, h->N, st);
-        if (e != hipSuccess) return hip_status(e, "transpose B");
         o.B = ws;
         o.ldb = h->K;
         o.trans_b = 1;

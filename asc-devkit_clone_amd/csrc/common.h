@@ -57,6 +57,28 @@ __device__ __forceinline__ uint16_t f32_to_bf16_sat(float x)
     b = (b & 0x7fffu) == 0x7f80u ? ((b & 0x8000u) | 0x7f7fu) : b;
     return (u & 0x7fffffffu) > 0x7f800000u ? (uint16_t)((u >> 16) | 0x40u) : (uint16_t)b;
 }
+// Two fp32 -> two f16 / bf16 (rne, saturating as f32_to_f16_sat / f32_to_bf16_sat) in one gfx950 conversion, as one
+// dword; `top` keeps the largest magnitude bits of both halves seen, so a caller converts many pairs and looks once for
+// the rare ones the conversion alone does not saturate (an exponent of all ones: overflow, infinity, NaN).
+typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bf2_t __attribute__((ext_vector_type(2)));
+typedef float f2_t __attribute__((ext_vector_type(2)));
+typedef uint16_t us2_t __attribute__((ext_vector_type(2)));
+template <bool BF>
+__device__ __forceinline__ uint32_t cvt_pair(float a, float b, us2_t& top)
+{
+    uint32_t d;
+    if constexpr (BF) d = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2_t){a, b}, bf2_t));
+    else d = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2_t){a, b}, h2_t));
+    top = __builtin_elementwise_max(top, __builtin_bit_cast(us2_t, d & 0x7fff7fffu));
+    return d;
+}
+template <bool BF>
+__device__ __forceinline__ bool cvt_special(us2_t top)
+{
+    constexpr uint32_t INF = BF ? 0x7f80u : 0x7c00u;
+    return top[0] >= INF || top[1] >= INF;
+}
 __device__ __forceinline__ float bf16_to_f32(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
 // fp32 -> bf16 value (kept in an fp32 register): rne, overflow to inf, NaN kept
 __device__ __forceinline__ float bf16_round(float x)  // rne to bf16, overflow to inf, NaN kept
@@ -367,6 +389,14 @@ __device__ __forceinline__ void c_atomic(uint8_t* p, uint32_t v, int op)
             old = prev;
         }
     }
+}
+
+// a 1-byte C element: (V)QF322B8_PRE for int8 / uint8, (V)QF322FP8_PRE, (V)QF322HIF8_PRE
+__device__ __forceinline__ uint8_t byte_out(float v, uint64_t w, int c_type)
+{
+    if (c_type == DT_INT8 || c_type == DT_UINT8) return requant8(v, w);
+    if (c_type == DT_HIF8) return (uint8_t)hif8_code_rna_sat(v);
+    return f32_to_fp8(v, c_type == DT_FP8_E5M2 ? 1 : 0);
 }
 
 }  // namespace ascq

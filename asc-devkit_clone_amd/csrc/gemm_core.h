@@ -1,9 +1,7 @@
 // gemm_core.h -- the LDS-staged MFMA main loop shared by the int8 and fp8 Matmuls, the MoE group matmul and
 // the MX (FP4 / FP8 element) Matmuls (gfx950).
 //
-// MFMA: the 32x32 forms, v_mfma_i32_32x32x32_i8 and v_mfma_[scale_]f32_32x32x64_f8f6f4 -- on gfx950 they issue
-// at the full int8 / fp8 / fp4 rate, the 16x16 forms at about half of it (measured: 4.80 vs 2.71 int8 POPS,
-// 9.34 vs 4.80 fp4 POPS on one MI355X).  A k-step (one instruction) covers 32 int8, 64 fp4 or 64 fp8 of K per
+// MFMA: the 32x32 forms, v_mfma_i32_32x32x32_i8 and v_mfma_[scale_]f32_32x32x64_f8f6f4.  A k-step (one instruction) covers 32 int8, 64 fp4 or 64 fp8 of K per
 // row: 32, 32 or 64 bytes.  Lane l holds row l % 32.  int8 / fp4: 16 bytes, the K half l / 32 of the step (fp4:
 // 32 elements, one MX block).  fp8: 32 bytes in two register quads; the instruction's K order is [quad 0 of
 // lanes 0-31, quad 0 of lanes 32-63, quad 1 of lanes 0-31, quad 1 of lanes 32-63], so lane l takes K bytes
@@ -220,6 +218,7 @@ struct GemmCore {
     static constexpr int CBSZ = OP == OP_MXFP4 ? F8F6F4_E2M1 : (IS_FP6 ? F8F6F4_E2M3 : (FMT & 7));
     static constexpr int BLGP = OP == OP_MXFP4 ? F8F6F4_E2M1 : (IS_FP6 ? F8F6F4_E2M3 : ((FMT >> 3) & 7));
     static constexpr int TBM = BM, TBN = BN, TWN = WN;  // the tile shape, for code outside the template
+    static constexpr int AR = 16;                       // registers of an accumulator fragment
     static constexpr int NW = WM * WN;
     static constexpr int NT = NW * 64;
     static constexpr int WTM = BM / WM, WTN = BN / WN;
@@ -299,6 +298,10 @@ struct GemmCore {
         return wm * WTM + i * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
     }
     __device__ __forceinline__ static int frag_col(int wn, int j, int lane) { return wn * WTN + j * 32 + (lane & 31); }
+    // where register r of fragment (i, j) lies in the tile (without CT), and the first row of fragment row i
+    __device__ __forceinline__ static int el_row(int wm, int i, int r, int lane) { return frag_row(wm, i, r, lane); }
+    __device__ __forceinline__ static int el_col(int wn, int j, int, int lane) { return frag_col(wn, j, lane); }
+    __device__ __forceinline__ static int block_row(int wm, int i) { return wm * WTM + i * 32; }
     // CT layout: the row of fragment (i, *) and the first of the four columns of register quad q of fragment (*, j)
     __device__ __forceinline__ static int ct_row(int wm, int i, int lane) { return wm * WTM + i * 32 + (lane & 31); }
     __device__ __forceinline__ static int ct_col(int wn, int j, int q, int lane)
@@ -898,14 +901,15 @@ __device__ __forceinline__ uint32_t acc_bits(int x) { return (uint32_t)x; }
 // the main loop -- and a rolled loop then takes one element per thread per step and hands put(tile row, tile
 // column, accumulator bits) the element.  Rolling the loop keeps the per-element code (a compare-and-swap, a software
 // encoder) and its registers out of an unrolled store path.  A tile that does not fit the LDS at once goes in NCH
-// chunks of rows: in chunk ch every wave writes the 32-row fragments that lie in it.
+// chunks of rows: in chunk ch every wave writes the 32-row fragments that lie in it.  Column c of row r is parked at
+// c ^ (r % 32), so neither a layout with one column per lane nor one with one row per lane meets on one bank.
 template <class T, class F>
 __device__ __forceinline__ void rolled_epilogue(uint8_t* smem, const typename T::acc_t (&acc)[T::FM][T::FN], int rows,
                                                 int cols, F put)
 {
     constexpr int NCH = (size_t)T::TBM * T::TBN * 4 <= T::LDS_BYTES ? 1 : (size_t)T::TBM * T::TBN * 2 <= T::LDS_BYTES ? 2 : 4;
     constexpr int CHR = T::TBM / NCH;  // rows per chunk
-    static_assert((size_t)CHR * T::TBN * 4 <= T::LDS_BYTES && CHR % 32 == 0 && (T::TBN & (T::TBN - 1)) == 0,
+    static_assert((size_t)CHR * T::TBN * 4 <= T::LDS_BYTES && CHR % 16 == 0 && T::TBN % 32 == 0,
                   "rolled epilogue chunks");
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wm = wave / T::TWN, wn = wave % T::TWN;
@@ -914,20 +918,21 @@ __device__ __forceinline__ void rolled_epilogue(uint8_t* smem, const typename T:
         __syncthreads();  // the main loop's last LDS reads (or the previous chunk's) are done
 #pragma unroll
         for (int i = 0; i < T::FM; ++i) {
-            if ((wm * T::WTM + i * 32) / CHR != ch) continue;  // 32-row fragment i lies in chunk ch or not at all
+            if (T::block_row(wm, i) / CHR != ch) continue;  // fragment row i lies in chunk ch or not at all
 #pragma unroll
             for (int j = 0; j < T::FN; ++j)
 #pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    *(uint32_t*)(smem + ((T::frag_row(wm, i, r, lane) - ch * CHR) * T::TBN + T::frag_col(wn, j, lane)) * 4) =
-                        acc_bits(acc[i][j][r]);
+                for (int r = 0; r < T::AR; ++r) {
+                    const int row = T::el_row(wm, i, r, lane), col = T::el_col(wn, j, r, lane);
+                    *(uint32_t*)(smem + ((row - ch * CHR) * T::TBN + (col ^ (row & 31))) * 4) = acc_bits(acc[i][j][r]);
+                }
         }
         __syncthreads();
 #pragma unroll 1
         for (int e = threadIdx.x; e < CHR * T::TBN; e += T::NT) {
             const int rr = ch * CHR + e / T::TBN, cc = e % T::TBN;
             if (rr >= rows || cc >= cols) continue;
-            put(rr, cc, *(const uint32_t*)(smem + e * 4));
+            put(rr, cc, *(const uint32_t*)(smem + (e ^ (rr & 31)) * 4));
         }
     }
 }

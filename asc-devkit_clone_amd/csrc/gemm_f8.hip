@@ -11,15 +11,15 @@
 // The float bias seeds the accumulator in the reference (MmadCompute with isBias, mmad_compute.h:40-90); adding
 // it to the finished fp32 sum differs only by fp32 rounding.
 //
-// gfx950 design: the gemm_core.h main loop with v_mfma_f32_32x32x64_f8f6f4 (the f8f6f4 MFMA with zero scale
+// gfx950 design: aligned problems above decode size run the pipelined 16x16x128 tiles of gemm_pipe.h
+// (gemm_pipe_f8.hip); here the gemm_core.h main loop with v_mfma_f32_32x32x64_f8f6f4 (the f8f6f4 MFMA with zero scale
 // operands), cbsz / blgp selecting e4m3 (0) or e5m2 (1) per operand: per lane 32 fp8 of one row in two
 // register quads, 64 K per instruction (K order in gemm_core.h).  The instruction sums each group of 16
 // consecutive K products (one register quad) aligned to the group's largest product and drops what falls below
 // 2^(e_max - 13) (measured: 1 + 2^-15 gives 1 within a group and 1 + 2^-15 across groups or k-steps), so
 // results differ from an fp32-accumulated sum by up to ~2^-13 of the group maxima.  gfx950's fp8 formats are
 // the OCP ones: e4m3 with no infinities and S.1111.111 as NaN (fp8_e4m3fn_t) and IEEE-like e5m2 (fp8_e5m2_t).
-// Tiles, stages and the [K, N] B register transpose are those of the int8 GEMM (fp8 operands are bytes like
-// int8).
+// Tiles and stages are those of the int8 GEMM (fp8 operands are bytes like int8).
 // hifloat8 operands (the sample's default scenario, MatmulFp8Kernel<hifloat8_t, hifloat8_t, float, float>,
 // matmul_fp8.asc:229; A and B both hifloat8, README_en.md) have no gfx950 MFMA format, but every HiF8 value (a
 // significand of at most 4 bits, 2^-22 .. 2^15, +-inf, NaN) is a bf16 value -- a normal one, where f16 would need
@@ -40,14 +40,6 @@ __device__ __forceinline__ float fp8_to_f32(uint8_t v, int fmt) { return fp8_bit
 __device__ __forceinline__ float op_elem(const uint8_t* p, int64_t idx, int fmt)
 {
     return fmt == FMT_BF16 ? bf16_to_f32(((const uint16_t*)p)[idx]) : fp8_to_f32(p[idx], fmt);
-}
-
-// a 1-byte C element: (V)QF322B8_PRE for int8 / uint8, (V)QF322FP8_PRE, (V)QF322HIF8_PRE
-__device__ __forceinline__ uint8_t byte_out(float v, uint64_t w, int c_type)
-{
-    if (c_type == DT_INT8 || c_type == DT_UINT8) return requant8(v, w);
-    if (c_type == DT_HIF8) return (uint8_t)hif8_code_rna_sat(v);
-    return f32_to_fp8(v, c_type == DT_FP8_E5M2 ? 1 : 0);
 }
 
 // w: the column's QUANT_PRE word (offset and sign flag of QF322B8); atomic: IterateAll's enAtomic (f32 / f16 /
@@ -358,7 +350,6 @@ static hipError_t launch_f8_fmt(const GemmF8Args& a, bool ua, hipStream_t st)
                                                                   : launch_f8_tiled<128, 128, 2, 2, 2, true, 64, FMT, true>(a, st);
     }
     if (ua) return hipErrorInvalidValue;
-    const bool big = a.M >= 1024 && a.N >= 1024;
     // decode-sized batches (B streamed once) with a K-contiguous B and f32 / f16 / bf16 C stored: 32 x 32 tiles,
     // each tile's K split over four waves of one workgroup, up to 32 rows, and up to 64 while 64 x 64 tiles would
     // leave fewer than 160 workgroups (the int8 Matmul's rule; 33-64 rows take 64 x 32 tiles where those make one
@@ -393,21 +384,14 @@ static hipError_t launch_f8_fmt(const GemmF8Args& a, bool ua, hipStream_t st)
                    : m64x32   ? launch_f8_tiled<64, 32, 1, 1, 4, false, 64, FMT, false, 4, true>(a, st)
                                 : launch_f8_tiled<32, 32, 1, 1, 4, false, 64, FMT, false, 4, true>(a, st);
     }
-    if (a.trans_b) {
+    if constexpr (ES == 1) {
+        return launch_gemm_f8_pipe(a, st);
+    } else {  // (the bf16 operands of a hifloat8 Matmul are always K-contiguous)
+        const bool big = a.M >= 1024 && a.N >= 1024;
         if (big) return (a.K * ES) % 128 == 0 ? launch_f8_tiled<256, 256, 4, 2, 2, true, 128, FMT>(a, st)
                                               : launch_f8_tiled<256, 256, 4, 2, 4, true, 64, FMT>(a, st);
         return launch_f8_tiled<64, 64, 2, 2, 4, true, 64, FMT>(a, st);
     }
-    // a large [K, N] B is transposed by the host layer first; this in-loop transpose serves the rest (fp8 only: the
-    // bf16 operands of a hifloat8 Matmul are always K-contiguous)
-    // (16-byte K rows: staged like A's and read by LDS transpose reads, as the int8 Matmul does -- K = 4096,
-    // N = 11008, M = 64: 37.8 -> 23.6 us; otherwise the in-register byte transpose)
-    if constexpr (ES == 1) {
-        if (a.ldb % 16 == 0 && (uintptr_t)a.B % 16 == 0)
-            return launch_f8_tiled<64, 128, 2, 2, 4, false, 64, FMT, false, 1, true>(a, st);
-        return launch_f8_tiled<64, 128, 2, 2, 4, false, 64, FMT>(a, st);
-    }
-    return hipErrorInvalidValue;
 }
 
 hipError_t launch_gemm_f8(const GemmF8Args& a, hipStream_t st)

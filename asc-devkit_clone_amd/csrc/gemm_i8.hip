@@ -4,9 +4,10 @@
 // stage/compute/mmad_compute.h:40-90 Mmad int8 -> int32 L0C; stage/copy_cube_out/copy_cube_out_fixpipe.h:339-357
 // and quant/quant_processor_fixpipe.h:74-234 for the DEQF16 / QS322BF16_PRE / REQ8 epilogues).
 //
-// gfx950 design: the v_mfma_i32_32x32x32_i8 main loop of gemm_core.h (a ring of LDS stages filled by
-// global->LDS buffer copies, XOR-swizzled LDS, in-flight byte transpose of a row-major [K, N] B), XCD-aware
-// tile order, and the fixpipe epilogue in registers:
+// gfx950 design: aligned problems above decode size run the pipelined 16x16x64 tiles of gemm_pipe.h (gemm_pipe_i8.hip,
+// B [N, K] or [K, N] as it lies); here are the decode-sized K-split tiles, the any-alignment tiles and the group matmul
+// on the v_mfma_i32_32x32x32_i8 main loop of gemm_core.h (a ring of LDS stages filled by global->LDS buffer copies,
+// XOR-swizzled LDS), XCD-aware tile order, and the fixpipe epilogue in registers:
 //   acc (+ int32 bias) -> f32 (rne) x M1[n] -> f16 / bf16 (rne, saturating), or -> requant8 (int8 / uint8 C:
 //   clamp, rint, + offset, saturate by the word's sign flag); M1 = QUANT_PRE bits [31:13]
 //   (accompanying_quantization.md:79-103).
@@ -531,7 +532,6 @@ hipError_t launch_gemm_i8(const GemmI8Args& a, hipStream_t st)
                                 : (a.ldb % 4 == 0 && a.N % 4 == 0 && ((uintptr_t)a.B % 4 == 0) && a.ldb * a.K < (1ll << 31));
     // the tiled epilogue addresses a 256-row output tile with 32-bit offsets
     if (a_ok && b_ok && a.K % 16 == 0 && a.ldc < (1ll << 21)) {
-        const bool big = a.M >= 1024 && a.N >= 1024;
         // small problems (the W8A8 sample, 128 x 256 x 512: 4 tiles of 64 x 128) take 32 x 32 single-wave tiles so
         // that at least 32 workgroups share the work
         const bool tiny = ((a.M + 63) / 64) * ((a.N + 127) / 128) < 32;
@@ -573,18 +573,7 @@ hipError_t launch_gemm_i8(const GemmI8Args& a, hipStream_t st)
             return a.N >= 10240 ? launch_tiled<32, 64, 1, 1, 4, false, 64, true, 4>(a, st)
                    : m64x32   ? launch_tiled<64, 32, 1, 1, 4, false, 64, true, 4>(a, st)
                                 : launch_tiled<32, 32, 1, 1, 4, false, 64, true, 4>(a, st);
-        if (a.trans_b)
-            return big ? (a.K % 128 == 0 ? launch_tiled<256, 256, 4, 2, 2, true, 128>(a, st)
-                                         : launch_tiled<256, 256, 4, 2, 4, true>(a, st))
-                       : (tiny ? launch_tiled<32, 32, 1, 1, 4, true>(a, st) : launch_tiled<64, 64, 2, 2, 4, true>(a, st));
-        // B [K, N] with 16-byte K rows (small and medium problems; the host transposes a large one first): the K
-        // rows are copied like A's and read by LDS transpose reads.  For 256 x 256 tiles that measured slower than
-        // the transpose plus the K-contiguous kernel (632.7 against 602 us at 8192^3: the 128-byte-stage form spills)
-        if (!big && a.ldb % 16 == 0 && (uintptr_t)a.B % 16 == 0)
-            return tiny ? launch_tiled<32, 32, 1, 1, 4, false, 64, true>(a, st)
-                        : launch_tiled<64, 128, 2, 2, 4, false, 64, true>(a, st);
-        if (tiny) return launch_tiled<32, 32, 1, 1, 4, false>(a, st);
-        return big ? launch_tiled<256, 256, 4, 2, 4, false>(a, st) : launch_tiled<64, 128, 2, 2, 4, false>(a, st);
+        return launch_gemm_i8_pipe(a, st);
     }
     // K not a multiple of 16, or operands / leading dimensions not 16-byte (A, K-contiguous B) or 4-byte ([K, N] B)
     // aligned: the any-alignment tiles (GemmCoreUA), 64 x 64 while that leaves fewer than 256 workgroups of 128 x 128

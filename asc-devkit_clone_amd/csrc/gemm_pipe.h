@@ -1,0 +1,569 @@
+// gemm_pipe.h -- the half-tile pipelined MFMA main loop of the medium and large int8 / fp8 / MX Matmuls (gfx950),
+// for K-contiguous operands with 128-byte multiples of K.
+//
+// What bounds a large tile is the feed from L2 / HBM into LDS.  GemmCore's two-stage loop waits for a whole stage
+// (64 KiB at 256 x 256) that was requested less than one stage of MFMAs earlier, and reads each k-step's fragments
+// right in front of the MFMAs that take them, so every barrier starts with the matrix cores idle.  Here a stage (128 K
+// bytes of every tile row) is four halves -- the upper and lower half of A's rows and of B's -- and the loop runs in
+// phases of a quarter stage.  A phase multiplies one A half by one B half (a quadrant of the wave's accumulators)
+// out of registers, reads the half that the phase after next needs first from LDS into registers, and requests one
+// half from memory into the slot whose half went to registers in the phase before.  Requests so run 4 ST - 2 phases
+// ahead of their reads (1.5 stages of MFMAs at ST = 2: 96 KiB in flight of a 128 KiB ring), no MFMA waits for an LDS
+// read issued in front of it, and a barrier has MFMA operands ready in registers on its far side.
+//
+// Order of the halves: H(4k) = A0(k), H(4k+1) = B0(k), H(4k+2) = B1(k), H(4k+3) = A1(k).  Phase t = 4k + p:
+//   p = 0: A0 B0, p = 1: A0 B1, p = 2: A1 B1, p = 3: A1 B0 -- each half is read once and consecutive phases share one;
+//   it reads H(t + 2) and requests H(t + 1 + 4 ST).  Each wave's quadrant rows are (half) x (wave row) x 32-row blocks.
+// B0(k + 1) is read while B0(k) is still multiplied: it goes to the registers B1(k) has left, so the two register sets
+// of B swap roles from stage to stage.
+//
+// MFMA: the 16x16 forms, v_mfma_i32_16x16x64_i8 and v_mfma_[scale_]f32_16x16x128_f8f6f4.  On operands that vary like
+// data the matrix cores run at a power limit, and the 16x16 forms do more within it than the 32x32 ones (256
+// workgroups of 8 waves multiplying out of registers, normal data, on one MI355X: int8 4.00 against 3.23 POPS, fp8 e4m3
+// 4.40 against 3.85, fp4 7.44 against 6.79 PFLOP/s).  Lane l holds row l % 16; with g = l / 16, int8 and fp4 take the
+// 16 bytes 16 g .. of a k-step's 64 (fp4: one MX block of 32), fp8 the 16 bytes 16 g .. and 64 + 16 g .. of its 128.
+// The MFMAs take the B fragment first, so an accumulator holds the transposed 16 x 16 block: lane l holds columns
+// 4 g .. 4 g + 3 of row l % 16.
+//
+// LDS rows of a K-contiguous operand are 128 bytes, 16-byte chunk c of row r at c ^ (r / 2 % 8): the 16 rows of a
+// fragment read hit 16 distinct 16-byte bank groups, and a copy writes 1 KiB contiguous (the swizzle is applied on the
+// global side).
+// B given [K, N] (BTR): a half of B is its columns' 128 K rows, copied as they lie, and read with ds_read_b64_tr_b8: a
+// 16-lane group g reads 8 K rows x 16 columns and lane j receives the 8 K of column j, so two reads (K rows 16 g ..
+// + 7 and 16 g + 8 .. + 15) give the lane's 16 K bytes.  Chunk c of K row k lies at c ^ swz_tr(k), which spreads the 16
+// pieces that two lane groups read together over 16 distinct 16-byte bank groups.
+// K is a multiple of 16 bytes: a lane's chunks at or past the end of K are not read (zeros), nor are a [K, N] B's rows.
+#pragma once
+
+#include "gemm_core.h"
+
+namespace ascq {
+
+// A buffer resource as four dwords, and its copy of 16 bytes per lane into LDS at `lds` (a byte address, wave-uniform)
+// + 16 * lane.  Written in assembly because through the builtin the compiler takes every later LDS transpose read for a
+// possible reader of the copy's destination and drains all copies in flight (s_waitcnt vmcnt(0)) in front of it; the
+// copies are ordered by the pipeline's own counted waits and barriers.  It has no register outputs.
+typedef uint32_t rsrc4_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ rsrc4_t make_rsrc4(const void* base, uint32_t bytes)
+{
+    const uint64_t a = (uint64_t)base;
+    rsrc4_t r = {(uint32_t)a, (uint32_t)(a >> 32) & 0xffffu, bytes, 0x00020000u};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = (uint32_t)__builtin_amdgcn_readfirstlane((int)r[i]);
+    return r;
+}
+__device__ __forceinline__ void dma16(const rsrc4_t& r, uint32_t lds, uint32_t off)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                 :
+                 : "s"(lds), "v"(off), "s"(r)
+                 : "memory", "m0");
+}
+__device__ __forceinline__ uint32_t lds_addr(const void* p)
+{
+    return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p;
+}
+
+struct PipeArgs {
+    rsrc4_t a, b;       // A: [rows][lda] bytes; B: [columns][ldb] bytes, or (BTR) [K][ldb]; ranges end with the operand
+    uint32_t lda, ldb;
+    uint32_t a0, b0;    // byte offsets of the tile origin
+    int32_t kbytes;     // K, a multiple of 16
+};
+
+template <int BM, int BN, int WM, int WN, int ST, int OP, int FMT = 0, bool BTR = false>
+struct GemmPipe {
+    static constexpr bool IS_F8 = OP == OP_F8;
+    static_assert(OP == OP_I8 || OP == OP_F8, "int8 or fp8");
+    static constexpr int CBSZ = FMT & 7, BLGP = (FMT >> 3) & 7;  // f8f6f4 formats of A and B
+    static constexpr int TBM = BM, TBN = BN, TWN = WN;
+    static constexpr int ROWB = 128;
+    static constexpr int KPS = IS_F8 ? 1 : 2;        // k-steps per stage
+    static constexpr int AR = 4;                     // registers of an accumulator fragment
+    static constexpr int NW = WM * WN, NT = NW * 64;
+    // rows of half h (192 rows: 128 and 64), of a wave in it, and their 16-row fragments
+    static constexpr int hm(int h) { return BM % 128 == 0 || BM == 64 ? BM / 2 : (h ? BM / 3 : BM / 3 * 2); }
+    static constexpr int hn(int h) { return BN % 128 == 0 || BN == 64 ? BN / 2 : (h ? BN / 3 : BN / 3 * 2); }
+    static constexpr int whm(int h) { return hm(h) / WM; }
+    static constexpr int whn(int h) { return hn(h) / WN; }
+    static constexpr int fmh(int h) { return whm(h) / 16; }
+    static constexpr int fnh(int h) { return whn(h) / 16; }
+    static constexpr int FM = fmh(0) + fmh(1), FN = fnh(0) + fnh(1);
+    static constexpr int ca(int h) { return hm(h) / 8 / NW; }  // 1 KiB copies per wave of an A / B half
+    static constexpr int cb(int h) { return hn(h) / 8 / NW; }
+    static constexpr int A_REG = ST * BM * ROWB, B_REG = ST * BN * ROWB;
+    static constexpr size_t LDS_BYTES = (size_t)A_REG + B_REG;
+    typedef typename std::conditional<OP == OP_I8, v4i, v4f>::type acc_t;
+    typedef typename std::conditional<IS_F8, v8i, v4i>::type frag_t;
+    static_assert(whm(0) % 16 == 0 && whm(1) % 16 == 0 && whn(0) % 32 == 0 && whn(1) % 32 == 0, "wave quadrants");
+    static_assert(hm(0) % (8 * NW) == 0 && hm(1) % (8 * NW) == 0 && hn(0) % (8 * NW) == 0 && hn(1) % (8 * NW) == 0,
+                  "copies split evenly over the waves");
+    static_assert(NW == 4 || NW == 8, "the swizzles of a lane's copies agree");
+    static_assert(ST == 2 || ST == 4, "the stage loop is unrolled by the ring");
+    static_assert(A_REG <= 65536 && B_REG <= 65536, "LDS read offsets are 16 bits");
+    static_assert(LDS_BYTES <= 160 * 1024, "LDS");
+    static_assert(!BTR || ((hn(0) == 128 || hn(0) == 64) && (hn(1) == 128 || hn(1) == 64)), "[K, N] halves");
+
+    // copies of half H(i)
+    static constexpr int half_copies(int i) { return i % 4 == 0 ? ca(0) : i % 4 == 1 ? cb(0) : i % 4 == 2 ? cb(1) : ca(1); }
+    // copies a wave may have outstanding at the barrier in front of phase p: H(t + 3) .. H(t + 4 ST)
+    static constexpr int outstanding(int p)
+    {
+        int n = 0;
+        for (int i = p + 3; i <= p + 4 * ST; ++i) n += half_copies(i);
+        return n;
+    }
+    static constexpr int RING = ST * (ca(0) + ca(1) + cb(0) + cb(1));  // copies of the whole ring
+    static_assert(RING < 64, "vmcnt");
+
+    // the tile row of fragment row i, and the first of the four columns of fragment column j
+    __device__ __forceinline__ static int block_row(int wm, int i)
+    {
+        return i < fmh(0) ? wm * whm(0) + i * 16 : hm(0) + wm * whm(1) + (i - fmh(0)) * 16;
+    }
+    __device__ __forceinline__ static int block_col(int wn, int j)
+    {
+        return j < fnh(0) ? wn * whn(0) + j * 16 : hn(0) + wn * whn(1) + (j - fnh(0)) * 16;
+    }
+    __device__ __forceinline__ static int ct_row(int wm, int i, int lane) { return block_row(wm, i) + (lane & 15); }
+    __device__ __forceinline__ static int ct_col(int wn, int j, int lane) { return block_col(wn, j) + 4 * (lane >> 4); }
+    __device__ __forceinline__ static int el_row(int wm, int i, int, int lane) { return ct_row(wm, i, lane); }
+    __device__ __forceinline__ static int el_col(int wn, int j, int r, int lane) { return ct_col(wn, j, lane) + r; }
+
+    // BTR: chunks per K row of half h, and the chunk swizzle of K row k in it
+    static constexpr int tch(int h) { return hn(h) / 16; }
+    __device__ __forceinline__ static int swz_tr(int h, int k)
+    {
+        return tch(h) == 8 ? ((k >> 1) & 3) | (((k >> 4) & 1) << 2) : ((k >> 2) & 1) | (((k >> 4) & 1) << 1);
+    }
+
+    // s_waitcnt vmcnt(N) lgkmcnt(0)
+    template <int N>
+    __device__ __forceinline__ static void wait_half()
+    {
+        __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | ((N >> 4) << 14));
+    }
+
+    __device__ __forceinline__ static void run(const PipeArgs& p, uint8_t* smem, acc_t (&acc)[FM][FN])
+    {
+        const int t = (int)threadIdx.x, lane = t & 63;
+        const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+        const int wm = wave / WN, wn = wave % WN;
+        const int r16 = lane & 15, g = lane >> 4;
+        uint8_t* sA = smem;
+        uint8_t* sB = smem + A_REG;
+        const uint32_t lA = lds_addr(sA), lB = lds_addr(sB);
+
+        // copy u of this wave in a half covers 1 KiB of it at u * NW + wave; the chunk swizzles repeat from copy to copy,
+        // so one lane offset per operand (BTR: per half of B) serves them all
+        const int nk = (p.kbytes + ROWB - 1) / ROWB;
+        const int kchunk = (int)((lane & 7) ^ ((wave * 4 + (lane >> 4)) & 7)) * 16;
+        const uint32_t va = p.a0 + (uint32_t)(lane >> 3) * p.lda + (uint32_t)kchunk;
+        uint32_t vb[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            if constexpr (BTR) {
+                const int kr = lane / tch(h), k = wave * (64 / tch(h)) + kr;
+                vb[h] = p.b0 + (uint32_t)kr * p.ldb + (uint32_t)((lane % tch(h)) ^ swz_tr(h, k)) * 16u;
+            } else {
+                vb[h] = p.b0 + (uint32_t)(lane >> 3) * p.ldb + (uint32_t)kchunk;
+            }
+        }
+        // half HI (0: A0, 1: B0, 2: B1, 3: A1) of stage kt into `slot`; nothing is read past K.  (Rows past the operand's
+        // last lie past its resource's range; rows past the tile's own are read, their products dropped.)
+        auto request = [&](auto HI, int kt, int slot) {
+            constexpr int hi = decltype(HI)::value;
+            constexpr bool isa = hi == 0 || hi == 3;
+            constexpr int h = hi >= 2 ? 1 : 0;
+            const uint32_t dst = isa ? lA + slot * (BM * ROWB) + h * hm(0) * ROWB : lB + slot * (BN * ROWB) + h * hn(0) * ROWB;
+            uint32_t v = isa ? va : vb[h], s = (uint32_t)kt * ROWB;
+            if constexpr (BTR && !isa) s = kt < nk ? s * p.ldb : OOB;
+            else v += kt * ROWB + kchunk < p.kbytes ? 0u : OOB;
+#pragma unroll
+            for (int u = 0; u < (isa ? ca(h) : cb(h)); ++u) {
+                const int c = u * NW + wave;
+                uint32_t row;
+                if constexpr (isa) row = (uint32_t)(h * hm(0) + c * 8) * p.lda;
+                else if constexpr (BTR) row = (uint32_t)(c * (64 / tch(h))) * p.ldb + (uint32_t)(h * hn(0));
+                else row = (uint32_t)(h * hn(0) + c * 8) * p.ldb;
+                dma16(isa ? p.a : p.b, dst + c * 1024, v + (s + row));
+            }
+        };
+
+        // lane offsets of the fragment reads: 16-byte chunk 4 c + g of the lane's row (within a half, wave row 0); BTR: the
+        // lane's 8-byte piece of fragment column j
+        constexpr int FA = fmh(0) > fmh(1) ? fmh(0) : fmh(1), FB = fnh(0) > fnh(1) ? fnh(0) : fnh(1);
+        uint32_t rl[2], rt[2][FB];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) rl[c] = (uint32_t)(r16 * ROWB + (((4 * c + g) ^ ((r16 >> 1) & 7)) * 16));
+        if constexpr (BTR) {
+            const int k = 16 * g + (r16 >> 1);
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int j = 0; j < fnh(h); ++j)
+                    rt[h][j] = (uint32_t)(k * hn(h) + ((wn * fnh(h) + j) ^ swz_tr(h, k)) * 16 + (r16 & 1) * 8);
+        }
+        const uint32_t wa[2] = {(uint32_t)(wm * whm(0) * ROWB), (uint32_t)((hm(0) + wm * whm(1)) * ROWB)};
+        const uint32_t wb[2] = {(uint32_t)(wn * whn(0) * ROWB), (uint32_t)((hn(0) + wn * whn(1)) * ROWB)};
+        frag_t fa[2][FA][KPS], fb[2][FB][KPS];
+        auto read_frag = [&](const uint8_t* base, int s) -> frag_t {
+            if constexpr (IS_F8) {
+                const v4i x = *(const v4i*)(base + rl[0]);
+                const v4i y = *(const v4i*)(base + rl[1]);
+                return (v8i){x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+            } else {
+                return *(const v4i*)(base + rl[s]);
+            }
+        };
+        auto read_a = [&](auto HH, int slot) {
+            constexpr int h = decltype(HH)::value;
+#pragma unroll
+            for (int i = 0; i < fmh(h); ++i)
+#pragma unroll
+                for (int s = 0; s < KPS; ++s) fa[h][i][s] = read_frag(sA + wa[h] + slot * (BM * ROWB) + i * 16 * ROWB, s);
+        };
+        typedef int v2i_t __attribute__((ext_vector_type(2)));
+        auto read_tr = [&](const uint8_t* base, int h, int j, int s) -> v4i {  // K rows 64 s + 16 g .. + 15
+            typedef __attribute__((address_space(3))) v2i_t* lp;
+            const v2i_t x = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lp)(base + rt[h][j] + s * 64 * hn(h)));
+            const v2i_t y = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lp)(base + rt[h][j] + (s * 64 + 8) * hn(h)));
+            return (v4i){x[0], x[1], y[0], y[1]};
+        };
+        auto read_b = [&](auto HH, int set, int slot) {
+            constexpr int h = decltype(HH)::value;
+#pragma unroll
+            for (int j = 0; j < fnh(h); ++j)
+#pragma unroll
+                for (int s = 0; s < KPS; ++s) {
+                    if constexpr (BTR) {
+                        const uint8_t* base = sB + slot * (BN * ROWB) + h * hn(0) * ROWB;
+                        if constexpr (IS_F8) {
+                            const v4i x = read_tr(base, h, j, 0), y = read_tr(base, h, j, 1);
+                            fb[set][j][s] = (v8i){x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+                        } else {
+                            fb[set][j][s] = read_tr(base, h, j, s);
+                        }
+                    } else {
+                        fb[set][j][s] = read_frag(sB + wb[h] + slot * (BN * ROWB) + j * 16 * ROWB, s);
+                    }
+                }
+        };
+        // MFMAs x0 .. x1 - 1 (k-step, then B fragment, then A fragment) of the quadrant (A half HA, B half HB held in
+        // register set `set`)
+        auto multiply = [&](auto HA, auto HB, int set, int x0, int x1) {
+            constexpr int ha = decltype(HA)::value, hb = decltype(HB)::value, fm = fmh(ha), fn = fnh(hb);
+#pragma unroll
+            for (int x = 0; x < KPS * fn * fm; ++x) {
+                if (x < x0 || x >= x1) continue;
+                const int s = x / (fn * fm), j = x / fm % fn, i = x % fm;
+                acc_t& c = acc[ha * fmh(0) + i][hb * fnh(0) + j];
+                if constexpr (OP == OP_I8)
+                    c = __builtin_amdgcn_mfma_i32_16x16x64_i8(fb[set][j][s], fa[ha][i][s], c, 0, 0, 0);
+                else
+                    c = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fb[set][j][s], fa[ha][i][s], c, BLGP, CBSZ, 0, 0, 0,
+                                                                         0);
+            }
+        };
+
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) acc[i][j] = (acc_t){};
+
+        using I0 = std::integral_constant<int, 0>;
+        using I1 = std::integral_constant<int, 1>;
+        using I2 = std::integral_constant<int, 2>;
+        using I3 = std::integral_constant<int, 3>;
+        // prologue: the ring's halves in flight, H(0) and H(1) into registers, then H(4 ST) into the slot of H(0)
+#pragma unroll
+        for (int k = 0; k < ST; ++k) {
+            request(I0{}, k, k);
+            request(I1{}, k, k);
+            request(I2{}, k, k);
+            request(I3{}, k, k);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        wait_vmcnt<RING - ca(0) - cb(0)>();
+        stage_barrier();
+        read_a(I0{}, 0);
+        read_b(I0{}, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        wait_half<RING - ca(0) - cb(0)>();
+        stage_barrier();
+        request(I0{}, ST, 0);
+        __builtin_amdgcn_sched_barrier(0);
+
+        // phase P of stage kt, which lies in slot SL of the ring (kt = SL modulo ST)
+        auto phase = [&](auto PP, auto SS, int kt) {
+            constexpr int P = decltype(PP)::value, SL = decltype(SS)::value, SN = (SL + 1) % ST;
+            constexpr int set0 = SL & 1, set1 = 1 - set0;  // register sets of B0(kt), B1(kt)
+            using HA = std::integral_constant<int, P >= 2>;
+            using HB = std::integral_constant<int, P == 1 || P == 2>;
+            constexpr int set = HB::value ? set1 : set0;
+            constexpr int NX = KPS * fnh(HB::value) * fmh(HA::value);
+            constexpr int LEAD = NX >= 8 ? NX / 4 : 1;  // MFMAs issued ahead of the reads
+            __builtin_amdgcn_sched_barrier(0);
+            wait_half<outstanding(P)>();
+            stage_barrier();
+            multiply(HA{}, HB{}, set, 0, LEAD);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (P == 0) read_b(I1{}, set1, SL);
+            if constexpr (P == 1) read_a(I1{}, SL);
+            if constexpr (P == 2) read_a(I0{}, SN);
+            if constexpr (P == 3) read_b(I0{}, set1, SN);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (P == 0) request(I1{}, kt + ST, SL);
+            if constexpr (P == 1) request(I2{}, kt + ST, SL);
+            if constexpr (P == 2) request(I3{}, kt + ST, SL);
+            if constexpr (P == 3) request(I0{}, kt + 1 + ST, SN);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(HA{}, HB{}, set, LEAD, NX);
+        };
+        auto stage = [&](auto SS, int kt) {
+            phase(I0{}, SS, kt);
+            phase(I1{}, SS, kt);
+            phase(I2{}, SS, kt);
+            phase(I3{}, SS, kt);
+        };
+        int kt = 0;
+        for (; kt + ST <= nk; kt += ST) {
+            stage(I0{}, kt);
+            stage(I1{}, kt + 1);
+            if constexpr (ST == 4) {
+                stage(I2{}, kt + 2);
+                stage(I3{}, kt + 3);
+            }
+        }
+        if (kt < nk) stage(I0{}, kt);
+        if constexpr (ST == 4) {
+            if (kt + 1 < nk) stage(I1{}, kt + 1);
+            if (kt + 2 < nk) stage(I2{}, kt + 2);
+        }
+        // drain: no copy may still target LDS when the caller reuses it or the wave ends
+        wait_vmcnt<0>();
+    }
+};
+
+// The tile of a problem: the one whose rounds over the 256 CUs cost least.  Measured per tile shape (int8, DEQF16 out,
+// K = 4096, one MI355X): microseconds per 128-byte stage of K with few CUs at work (`solo`) and with all of them
+// (`full`: the matrix cores and the memory system then share a power and a bandwidth limit), and what a tile costs
+// beyond its stages when all write at once (`tail`: first stage's latency, epilogue).  A CU runs c = ceil(tiles / 256)
+// tiles, one after the other or side by side (128 x 128 two at a time, 64 x 128 three: no gain per tile, so the same
+// sum), a fraction of the CUs one fewer.  E.g. K = 4096, N = 11008 (start: this layout's tiles before these kernels):
+// M = 2048 192 x 256 in 78 us against 91 (256 x 256), 84 (128 x 256), 88 (128 x 128); M = 512 128 x 192 in 25.0 against
+// 25.6 (128 x 256), 27.8 (128 x 128), 30.2 (64 x 128); M = 256 128 x 128 in 16.6 against 20.3 (128 x 192), 20.6
+// (64 x 128); M = 128 64 x 128 in 12.5 against 16.0 (128 x 128).
+enum PipeTile { PIPE_256x256, PIPE_192x256, PIPE_256x192, PIPE_128x256, PIPE_128x192, PIPE_128x128, PIPE_64x128, PIPE_TILES };
+inline PipeTile pick_pipe_tile(int64_t M, int64_t N, int64_t kbytes)
+{
+    static const struct {
+        int bm, bn;
+        float solo, full, tail;
+    } T[PIPE_TILES] = {{256, 256, 1.08f, 1.45f, 6.0f}, {192, 256, 0.86f, 1.16f, 4.0f}, {256, 192, 0.86f, 1.16f, 4.0f},
+                       {128, 256, 0.59f, 0.90f, 4.0f}, {128, 192, 0.50f, 0.67f, 3.5f}, {128, 128, 0.375f, 0.47f, 1.9f},
+                       {64, 128, 0.25f, 0.30f, 0.65f}};
+    const float stages = (float)((kbytes + 127) / 128);
+    PipeTile best = PIPE_256x256;
+    float least = 0.0f;
+    for (int t = 0; t < PIPE_TILES; ++t) {
+        const int64_t tiles = ((M + T[t].bm - 1) / T[t].bm) * ((N + T[t].bn - 1) / T[t].bn);
+        const float c = (float)((tiles + 255) / 256), fill = (float)tiles / (256.0f * c);
+        const float cost = c * ((T[t].solo + (T[t].full - T[t].solo) * fill) * stages + T[t].tail * fill);
+        if (t == 0 || cost < least) {
+            best = (PipeTile)t;
+            least = cost;
+        }
+    }
+    return best;
+}
+
+// XCD-aware tile order of the pipelined kernels: consecutive workgroup ids go round-robin over the 8 XCDs, so XCD x
+// gets the x-th of 8 contiguous runs (equal within one tile) of a raster that walks GM tile rows at a time: the tiles
+// that one XCD runs together share A rows and B columns through its L2.
+__device__ __forceinline__ void pipe_tile(int pid, int tiles_m, int tiles_n, int& tm, int& tn)
+{
+    const int total = tiles_m * tiles_n, q = total / 8, r = total % 8, x = pid % 8;
+    pid = x * q + (x < r ? x : r) + pid / 8;
+    constexpr int GM = 8;
+    const int width = GM * tiles_n;
+    const int first_m = (pid / width) * GM;
+    const int gm = (tiles_m - first_m) < GM ? (tiles_m - first_m) : GM;
+    const int in_group = pid % width;
+    tm = first_m + in_group % gm;
+    tn = in_group / gm;
+}
+
+// Store epilogue of transposed accumulators.  Lane l = 16 g + r holds columns 4 g .. 4 g + 3 of row r of each 16 x 16
+// fragment.  v_permlane16_swap trades the odd lane rows of fragment j's registers for the even ones of fragment
+// j + 1's, after which a lane owns eight consecutive columns -- 8 (g / 2) .. of fragment j + g % 2: one 16-byte
+// (2-byte elements), 8-byte (1-byte) or 4-byte (int4 codes, ES 0) store where there were eight of one element.  4-byte
+// elements leave as they are, one 16-byte store per fragment.
+// cols4(tile column) gives the parameters of four columns; conv(accumulator, parameters, e) the element's bits, or, for
+// the 2-byte types (OUT_F16, OUT_BF16), its fp32 value, which is converted here two at a time.
+// vec: the output's base and row pitch are multiples of four bytes; otherwise, and in runs that cross the tile's last
+// column, elements are stored one by one.
+enum { OUT_I4 = 0, OUT_1 = 1, OUT_F16 = 2, OUT_BF16 = 3, OUT_4 = 4 };
+template <class T, int OUT, class Cols, class Conv>
+__device__ __forceinline__ void ct_store(const TileOut& out, bool vec, int cols, const typename T::acc_t (&acc)[T::FM][T::FN],
+                                         int wm, int wn, int lane, Cols cols4, Conv conv)
+{
+    constexpr bool HALF = OUT == OUT_F16 || OUT == OUT_BF16;
+    const int g = lane >> 4;
+#pragma unroll
+    for (int j = 0; j < T::FN; j += 2) {
+        const int c0 = T::ct_col(wn, j, lane), c1 = c0 + 16;
+        const auto p0 = cols4(c0), p1 = cols4(c1);
+#pragma unroll
+        for (int i = 0; i < T::FM; ++i) {
+            const uint32_t roff = (uint32_t)T::ct_row(wm, i, lane) * out.pitch;
+            const int c = T::block_col(wn, j + (g & 1)) + 8 * (g >> 1);  // this lane's eight columns after the swap
+            if constexpr (OUT == OUT_4) {
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    uint32_t x[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) x[e] = conv(acc[i][j + q][e], q ? p1 : p0, e);
+                    const int cq = q ? c1 : c0;
+                    if (cq + 4 <= cols) {
+                        __builtin_amdgcn_raw_buffer_store_b128((u32x4){x[0], x[1], x[2], x[3]}, out.r,
+                                                               roff + (uint32_t)cq * 4, 0, 0);
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            __builtin_amdgcn_raw_buffer_store_b32(x[e], out.r,
+                                                                  cq + e < cols ? roff + (uint32_t)(cq + e) * 4 : OOB, 0, 0);
+                    }
+                }
+            } else {
+                constexpr int PER = HALF ? 2 : (OUT == OUT_1 ? 4 : 8);  // elements per dword
+                constexpr int SH = 32 / PER;                            // bits per element
+                uint32_t lo[2], hi[2], d[8 / PER];                      // fragment j's four elements, j + 1's
+                if constexpr (HALF) {
+                    float v[8];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        v[e] = conv(acc[i][j][e], p0, e);
+                        v[4 + e] = conv(acc[i][j + 1][e], p1, e);
+                    }
+                    us2_t top = {0, 0};
+                    lo[0] = cvt_pair<OUT == OUT_BF16>(v[0], v[1], top);
+                    lo[1] = cvt_pair<OUT == OUT_BF16>(v[2], v[3], top);
+                    hi[0] = cvt_pair<OUT == OUT_BF16>(v[4], v[5], top);
+                    hi[1] = cvt_pair<OUT == OUT_BF16>(v[6], v[7], top);
+                    if (__builtin_expect(cvt_special<OUT == OUT_BF16>(top), 0)) {
+                        auto one = [](float x) { return (uint32_t)(OUT == OUT_BF16 ? f32_to_bf16_sat(x) : f32_to_f16_sat(x)); };
+#pragma unroll
+                        for (int e = 0; e < 2; ++e) {
+                            lo[e] = one(v[2 * e]) | (one(v[2 * e + 1]) << 16);
+                            hi[e] = one(v[4 + 2 * e]) | (one(v[4 + 2 * e + 1]) << 16);
+                        }
+                    }
+                    const auto s0 = __builtin_amdgcn_permlane16_swap(lo[0], hi[0], false, false);
+                    const auto s1 = __builtin_amdgcn_permlane16_swap(lo[1], hi[1], false, false);
+                    d[0] = s0[0];
+                    d[1] = s1[0];
+                    d[2] = s0[1];
+                    d[3] = s1[1];
+                } else {
+                    constexpr uint32_t MASK = (1u << SH) - 1u;
+                    lo[0] = hi[0] = 0u;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        lo[0] |= (conv(acc[i][j][e], p0, e) & MASK) << (SH * e);
+                        hi[0] |= (conv(acc[i][j + 1][e], p1, e) & MASK) << (SH * e);
+                    }
+                    const auto sw = __builtin_amdgcn_permlane16_swap(lo[0], hi[0], false, false);
+                    if constexpr (OUT == OUT_I4) {
+                        d[0] = sw[0] | (sw[1] << 16);
+                    } else {
+                        d[0] = sw[0];
+                        d[1] = sw[1];
+                    }
+                }
+                if (vec && c + 8 <= cols) {
+                    if constexpr (OUT == OUT_I4)
+                        __builtin_amdgcn_raw_buffer_store_b32(d[0], out.r, roff + (uint32_t)(c / 2), 0, 0);
+                    else if constexpr (OUT == OUT_1)
+                        __builtin_amdgcn_raw_buffer_store_b64((u32x2){d[0], d[1]}, out.r, roff + (uint32_t)c, 0, 0);
+                    else
+                        __builtin_amdgcn_raw_buffer_store_b128((u32x4){d[0], d[1], d[2], d[3]}, out.r,
+                                                               roff + (uint32_t)c * 2, 0, 0);
+                } else if constexpr (OUT == OUT_I4) {  // two codes per byte (an even number of columns)
+#pragma unroll
+                    for (int e = 0; e < 8; e += 2)
+                        __builtin_amdgcn_raw_buffer_store_b8((uint8_t)(d[0] >> (4 * e)), out.r,
+                                                             c + e < cols ? roff + (uint32_t)((c + e) / 2) : OOB, 0, 0);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const uint32_t v = d[e / PER] >> (SH * (e % PER));
+                        const uint32_t o = c + e < cols ? roff + (uint32_t)((c + e) * (HALF ? 2 : 1)) : OOB;
+                        if constexpr (HALF) __builtin_amdgcn_raw_buffer_store_b16((uint16_t)v, out.r, o, 0, 0);
+                        else __builtin_amdgcn_raw_buffer_store_b8((uint8_t)v, out.r, o, 0, 0);
+                    }
+                }
+            }
+        }
+    }
+}
+
+// The per-channel words of an epilogue, four columns at a time: the int32 / f32 bias and the QUANT_PRE words of the
+// tile's columns go to LDS before the main loop (copies older than the loop's, whose first wait covers them), so the
+// epilogue starts without a trip to memory.  Absent vectors give `no_bias` (0, or -0.0f: adding it changes no fp32
+// value) and the scalar word (the bits of 1.0f where nothing is to be multiplied), so the arithmetic has no branches.
+struct ColWords {
+    uint32_t bias[4];
+    float m1[4];
+    uint32_t lo[4], hi[4];
+};
+struct ColLds {
+    static constexpr int BYTES = 3072;  // up to 256 columns
+    const uint8_t* base;
+    bool has_bias, has_words;
+    uint32_t no_bias;
+    uint64_t scalar;
+    // waves 0, 1 and 2 issue one 1 KiB copy each (modulo the workgroup's waves)
+    __device__ __forceinline__ void request(uint8_t* lds, int nw, const void* bias, uint32_t none, const uint64_t* words,
+                                            uint64_t qscalar, int64_t n0, int cols)
+    {
+        base = lds;
+        has_bias = bias != nullptr;
+        has_words = words != nullptr;
+        no_bias = none;
+        scalar = qscalar;
+        const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
+        if (has_bias && wave == 0)
+            dma16(make_rsrc4((const uint32_t*)bias + n0, (uint32_t)cols * 4u), lds_addr(lds), (uint32_t)lane * 16u);
+        if (has_words) {
+            const rsrc4_t r = make_rsrc4(words + n0, (uint32_t)cols * 8u);
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                if (wave == (1 + h) % nw) dma16(r, lds_addr(lds) + 1024 + h * 1024, (uint32_t)(h * 1024 + lane * 16));
+        }
+    }
+    // one column's
+    __device__ __forceinline__ uint32_t bias(int c) const { return has_bias ? *(const uint32_t*)(base + c * 4) : no_bias; }
+    __device__ __forceinline__ uint64_t word(int c) const
+    {
+        return has_words ? *(const uint64_t*)(base + 1024 + c * 8) : scalar;
+    }
+    __device__ __forceinline__ ColWords operator()(int c) const
+    {
+        ColWords w;
+        const u32x4 b = has_bias ? *(const u32x4*)(base + c * 4) : (u32x4){no_bias, no_bias, no_bias, no_bias};
+        const u32x4 s = {(uint32_t)scalar, (uint32_t)(scalar >> 32), (uint32_t)scalar, (uint32_t)(scalar >> 32)};
+        const u32x4 x = has_words ? *(const u32x4*)(base + 1024 + c * 8) : s;
+        const u32x4 y = has_words ? *(const u32x4*)(base + 1024 + c * 8 + 16) : s;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            w.bias[e] = b[e];
+            w.lo[e] = e < 2 ? x[2 * e] : y[2 * e - 4];
+            w.hi[e] = e < 2 ? x[2 * e + 1] : y[2 * e - 3];
+            w.m1[e] = quant_pre_m1(w.lo[e]);
+        }
+        return w;
+    }
+};
+
+}  // namespace ascq

@@ -107,6 +107,9 @@ struct GemmI8Args {
     int splits;           // (set by the launcher) workgroups per tile of the K-split form
 };
 hipError_t launch_gemm_i8(const GemmI8Args& a, hipStream_t st);
+// gemm_pipe_i8.hip: A [M, K] with 16-byte-aligned rows and B [N, K] the same, or B [K, N] with 4-byte-aligned rows; K a
+// multiple of 16, operands below 2^31 bytes
+hipError_t launch_gemm_i8_pipe(const GemmI8Args& a, hipStream_t st);
 // Decode-sized batches (M <= 64: one row tile of 32 or 64 rows; K % 256 == 0) -- B given [K, N] (trans_b 0) with long
 // K or wide N on x 128 tiles, B given [N, K] with long K and few x 32 tiles -- split each tile's K over several
 // workgroups (four waves each) so that about 256 workgroups stream B; their accumulators meet in the workspace and a
@@ -139,6 +142,8 @@ struct GemmF8Args {
     int splits;           // (set by the launcher) workgroups per tile of the K-split form
 };
 hipError_t launch_gemm_f8(const GemmF8Args& a, hipStream_t st);
+// gemm_pipe_f8.hip: A [M, K] and B [N, K] fp8 with 16-byte-aligned rows below 2^31 bytes in all, K % 128 == 0
+hipError_t launch_gemm_f8_pipe(const GemmF8Args& a, hipStream_t st);
 
 // group_gemm.hip
 struct GroupGemmArgs {

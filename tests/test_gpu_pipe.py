@@ -1,0 +1,92 @@
+"""GPU parity of the pipelined GEMM tiles (gemm_pipe.h) at sizes the dispatch gives to each tile shape: partial last tiles
+in M and N, K tails of 16-byte chunks, odd stage counts, both B layouts, vector and element-wise stores.  int8: bit-exact
+against the oracle.  fp8: integer-valued codes (-4 .. 4) make every sum exact in fp32, so f32 C equals the fp64 product
+and bf16 C its one rounding."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import oracle_lib as O
+from conftest import seeded
+
+pytestmark = pytest.mark.gpu
+
+# (M, N, K): the tile pick_pipe_tile chooses
+SHAPES = [
+    (77, 377, 64),       # 64 x 128, one partial stage
+    (65, 4100, 336),     # 64 x 128, three stages, the last of 80 bytes
+    (3353, 536, 272),    # 128 x 128
+    (4127, 932, 416),    # 128 x 192
+    (1607, 3736, 528),   # 128 x 256
+    (3457, 1732, 64),    # 192 x 256
+    (3273, 1816, 144),   # 256 x 192
+    (3301, 3804, 80),    # 256 x 256
+]
+
+
+def _dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def _bits(t):
+    return t.cpu().view(torch.int16).numpy().view(np.uint16)
+
+
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("M,N,K", SHAPES + [(130, 1001, 2048), (300, 5003, 1040)])  # odd N: odd pitches of C
+def test_int8_pipe(ascq_gpu, oracle, M, N, K, trans_b):
+    if not trans_b and N % 4:
+        pytest.skip("[K, N] with N % 4 != 0 takes the any-alignment tiles")
+    rng = seeded(M + N + K + trans_b)
+    A = rng.integers(-128, 128, (M, K), dtype=np.int8)
+    B = rng.integers(-128, 128, (N, K) if trans_b else (K, N), dtype=np.int8)
+    bias = rng.integers(-(1 << 20), 1 << 20, N, dtype=np.int32)
+    words = np.exp(rng.uniform(np.log(2.0 ** -20), np.log(2.0 ** -8), N)).astype(np.float32).view(np.uint32).astype(np.uint64)
+    acc = O.matmul_i8(A, B, bias, False, trans_b)
+    a, b, bi, w = _dev(A), _dev(B), _dev(bias), _dev(words.view(np.int64))
+    for c_type, dt, ref in [(ascq_gpu.F16, torch.float16, O.mm_dequant(acc, O.F16, qvec=words)),
+                            (ascq_gpu.BF16, torch.bfloat16, O.mm_dequant(acc, O.BF16, qvec=words)),
+                            (ascq_gpu.INT32, torch.int32, acc),
+                            (ascq_gpu.INT8, torch.int8, O.mm_requant(acc, qvec=words | np.uint64(1 << 46)))]:
+        mm = ascq_gpu.Matmul(ascq_gpu.INT8, ascq_gpu.INT8, c_type, ascq_gpu.INT32)
+        mm.SetOrgShape(M, N, K)
+        if c_type != ascq_gpu.INT32:
+            mm.SetQuantVector(_dev((words | np.uint64(1 << 46)).view(np.int64)) if c_type == ascq_gpu.INT8 else w)
+        mm.SetTensorA(a)
+        mm.SetTensorB(b, trans_b)
+        mm.SetBias(bi)
+        out = torch.zeros(M * N + 16, dtype=dt, device="cuda")  # the 16 past the end must stay zero
+        mm.IterateAll(out)
+        torch.cuda.synchronize()
+        got = out[:M * N].view(M, N)
+        assert not bool(out[M * N:].any()), c_type
+        if dt in (torch.float16, torch.bfloat16):
+            np.testing.assert_array_equal(_bits(got), ref)
+        else:
+            np.testing.assert_array_equal(got.cpu().numpy(), ref.view(np.int8) if dt == torch.int8 else ref)
+
+
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("M,N,K", SHAPES + [(300, 5003, 1040)])
+def test_fp8_pipe(ascq_gpu, M, N, K, trans_b):
+    if not trans_b and N % 4:
+        pytest.skip("[K, N] with N % 4 != 0 takes the generic kernel")
+    g = torch.Generator().manual_seed(M + N + K + trans_b)
+    A = torch.randint(-4, 5, (M, K), generator=g)
+    B = torch.randint(-4, 5, (N, K) if trans_b else (K, N), generator=g)
+    bias = torch.randint(-8, 9, (N,), generator=g).float()
+    ref = A.double() @ (B.double().t() if trans_b else B.double()) + bias.double()
+    a, b = A.float().to(torch.float8_e4m3fn).cuda(), B.float().to(torch.float8_e5m2).cuda()
+    for c_type, dt in [(ascq_gpu.F32, torch.float32), (ascq_gpu.BF16, torch.bfloat16)]:
+        mm = ascq_gpu.Matmul(ascq_gpu.FP8_E4M3, ascq_gpu.FP8_E5M2, c_type, ascq_gpu.F32)
+        mm.SetOrgShape(M, N, K)
+        mm.SetTensorA(a)
+        mm.SetTensorB(b, trans_b)
+        mm.SetBias(bias.cuda())
+        out = torch.zeros(M * N + 16, dtype=dt, device="cuda")
+        mm.IterateAll(out)
+        torch.cuda.synchronize()
+        assert not bool(out[M * N:].any()), c_type
+        assert torch.equal(out[:M * N].view(M, N).cpu(), ref.float().to(dt)), c_type
