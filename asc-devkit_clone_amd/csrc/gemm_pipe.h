@@ -32,6 +32,9 @@
 // 16-lane group g reads 8 K rows x 16 columns and lane j receives the 8 K of column j, so two reads (K rows 16 g ..
 // + 7 and 16 g + 8 .. + 15) give the lane's 16 K bytes.  Chunk c of K row k lies at c ^ swz_tr(k), which spreads the 16
 // pieces that two lane groups read together over 16 distinct 16-byte bank groups.
+// MX-FP4: the E8M0 scales arrive stage-major, the eight of (stage, row) -- k-step s, block g of it -- at byte 2 g + s of
+// its eight, and each stage's go to one of four scale slots, requested three stages ahead, one copy per wave and stage;
+// a lane reads the two bytes of block g of its row and the MFMA's op_sel picks the k-step's.
 // K is a multiple of 16 bytes: a lane's chunks at or past the end of K are not read (zeros), nor are a [K, N] B's rows.
 #pragma once
 
@@ -69,13 +72,19 @@ struct PipeArgs {
     uint32_t lda, ldb;
     uint32_t a0, b0;    // byte offsets of the tile origin
     int32_t kbytes;     // K, a multiple of 16
+    // MX: the stage-major scales ([stage][rows][8]) of both operands through one resource: byte offsets of the tile's
+    // first row in stage 0, and the stage strides
+    rsrc4_t aux;
+    uint32_t sa_off, sa_stride, sb_off, sb_stride;
 };
 
 template <int BM, int BN, int WM, int WN, int ST, int OP, int FMT = 0, bool BTR = false>
 struct GemmPipe {
     static constexpr bool IS_F8 = OP == OP_F8;
-    static_assert(OP == OP_I8 || OP == OP_F8, "int8 or fp8");
-    static constexpr int CBSZ = FMT & 7, BLGP = (FMT >> 3) & 7;  // f8f6f4 formats of A and B
+    static constexpr bool IS_MX = OP == OP_MXFP4;
+    static_assert(OP == OP_I8 || OP == OP_F8 || (IS_MX && !BTR), "int8, fp8, or MX-FP4 with a K-contiguous B");
+    static constexpr int CBSZ = IS_MX ? F8F6F4_E2M1 : FMT & 7;  // f8f6f4 formats of A and B
+    static constexpr int BLGP = IS_MX ? F8F6F4_E2M1 : (FMT >> 3) & 7;
     static constexpr int TBM = BM, TBN = BN, TWN = WN;
     static constexpr int ROWB = 128;
     static constexpr int KPS = IS_F8 ? 1 : 2;        // k-steps per stage
@@ -92,7 +101,9 @@ struct GemmPipe {
     static constexpr int ca(int h) { return hm(h) / 8 / NW; }  // 1 KiB copies per wave of an A / B half
     static constexpr int cb(int h) { return hn(h) / 8 / NW; }
     static constexpr int A_REG = ST * BM * ROWB, B_REG = ST * BN * ROWB;
-    static constexpr size_t LDS_BYTES = (size_t)A_REG + B_REG;
+    static constexpr int SCA = IS_MX ? (BM * 8 + 1023) / 1024 : 0, SCB = IS_MX ? (BN * 8 + 1023) / 1024 : 0;  // scale copies
+    static constexpr int SC_SLOT = (SCA + SCB) * 1024;
+    static constexpr size_t LDS_BYTES = (size_t)A_REG + B_REG + 4 * SC_SLOT;
     typedef typename std::conditional<OP == OP_I8, v4i, v4f>::type acc_t;
     typedef typename std::conditional<IS_F8, v8i, v4i>::type frag_t;
     static_assert(whm(0) % 16 == 0 && whm(1) % 16 == 0 && whn(0) % 32 == 0 && whn(1) % 32 == 0, "wave quadrants");
@@ -102,6 +113,7 @@ struct GemmPipe {
     static_assert(ST == 2 || ST == 4, "the stage loop is unrolled by the ring");
     static_assert(A_REG <= 65536 && B_REG <= 65536, "LDS read offsets are 16 bits");
     static_assert(LDS_BYTES <= 160 * 1024, "LDS");
+    static_assert(SCA + SCB <= NW, "one scale copy per wave");
     static_assert(!BTR || ((hn(0) == 128 || hn(0) == 64) && (hn(1) == 128 || hn(1) == 64)), "[K, N] halves");
 
     // copies of half H(i)
@@ -111,6 +123,8 @@ struct GemmPipe {
     {
         int n = 0;
         for (int i = p + 3; i <= p + 4 * ST; ++i) n += half_copies(i);
+        if (IS_MX)  // ... and the scale copies of the phases 2 among the 4 ST - 2 before
+            for (int t = p + 2; t < p + 4 * ST; ++t) n += t % 4 == 2;
         return n;
     }
     static constexpr int RING = ST * (ca(0) + ca(1) + cb(0) + cb(1));  // copies of the whole ring
@@ -146,6 +160,10 @@ struct GemmPipe {
 
     __device__ __forceinline__ static void run(const PipeArgs& p, uint8_t* smem, acc_t (&acc)[FM][FN])
     {
+        using I0 = std::integral_constant<int, 0>;
+        using I1 = std::integral_constant<int, 1>;
+        using I2 = std::integral_constant<int, 2>;
+        using I3 = std::integral_constant<int, 3>;
         const int t = (int)threadIdx.x, lane = t & 63;
         const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
         const int wm = wave / WN, wn = wave % WN;
@@ -190,6 +208,21 @@ struct GemmPipe {
             }
         };
 
+        // MX: this wave's 1 KiB of a stage's scales (waves past the copies repeat one)
+        const uint8_t* sS = smem + A_REG + B_REG;
+        uint32_t sc_off = 0, sc_stride = 0, sc_dst = 0;
+        if constexpr (IS_MX) {
+            const int c = wave % (SCA + SCB);
+            const bool isb = c >= SCA;
+            sc_off = (isb ? p.sb_off + (uint32_t)(c - SCA) * 1024u : p.sa_off + (uint32_t)c * 1024u) + (uint32_t)lane * 16u;
+            sc_stride = isb ? p.sb_stride : p.sa_stride;
+            sc_dst = lds_addr(sS) + (uint32_t)c * 1024u;
+        }
+        auto request_scales = [&](int kt) {
+            if constexpr (IS_MX)
+                dma16(p.aux, sc_dst + (uint32_t)(kt & 3) * SC_SLOT, sc_off + (kt < nk ? (uint32_t)kt * sc_stride : OOB));
+        };
+
         // lane offsets of the fragment reads: 16-byte chunk 4 c + g of the lane's row (within a half, wave row 0); BTR: the
         // lane's 8-byte piece of fragment column j
         constexpr int FA = fmh(0) > fmh(1) ? fmh(0) : fmh(1), FB = fnh(0) > fnh(1) ? fnh(0) : fnh(1);
@@ -207,21 +240,40 @@ struct GemmPipe {
         const uint32_t wa[2] = {(uint32_t)(wm * whm(0) * ROWB), (uint32_t)((hm(0) + wm * whm(1)) * ROWB)};
         const uint32_t wb[2] = {(uint32_t)(wn * whn(0) * ROWB), (uint32_t)((hn(0) + wn * whn(1)) * ROWB)};
         frag_t fa[2][FA][KPS], fb[2][FB][KPS];
-        auto read_frag = [&](const uint8_t* base, int s) -> frag_t {
+        auto read_frag = [&](const uint8_t* base, const uint32_t (&off)[2], int s) -> frag_t {
             if constexpr (IS_F8) {
-                const v4i x = *(const v4i*)(base + rl[0]);
-                const v4i y = *(const v4i*)(base + rl[1]);
+                const v4i x = *(const v4i*)(base + off[0]);
+                const v4i y = *(const v4i*)(base + off[1]);
                 return (v8i){x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
             } else {
-                return *(const v4i*)(base + rl[s]);
+                return *(const v4i*)(base + off[s]);
             }
         };
-        auto read_a = [&](auto HH, int slot) {
+        // the lane offsets of a read, added up in front of it: kept over the loop for every half they cost more
+        // registers than the 256 x 256 tiles have
+        auto at = [&](uint32_t (&off)[2], uint32_t w) {
+            asm volatile("" : "+s"(w));
+            off[0] = rl[0] + w;
+            off[1] = rl[1] + w;
+        };
+        // MX: the scale bytes of fragment rows i and i + 1 (k-steps 0 and 1 each) in one register
+        us2_t swa[2][(FA + 1) / 2], swb[2][(FB + 1) / 2];
+        const uint32_t rs = (uint32_t)(r16 * 8 + 2 * g);
+        auto read_scale = [&](int kt, int row) -> uint16_t {
+            return *(const uint16_t*)(sS + (kt & 3) * SC_SLOT + row * 8 + rs);
+        };
+        auto read_a = [&](auto HH, int slot, int kt) {
             constexpr int h = decltype(HH)::value;
+            uint32_t off[2];
+            at(off, wa[h]);
+            if constexpr (IS_MX) {
+#pragma unroll
+                for (int i = 0; i < fmh(h); ++i) swa[h][i / 2][i % 2] = read_scale(kt, h * hm(0) + wm * whm(h) + i * 16);
+            }
 #pragma unroll
             for (int i = 0; i < fmh(h); ++i)
 #pragma unroll
-                for (int s = 0; s < KPS; ++s) fa[h][i][s] = read_frag(sA + wa[h] + slot * (BM * ROWB) + i * 16 * ROWB, s);
+                for (int s = 0; s < KPS; ++s) fa[h][i][s] = read_frag(sA + slot * (BM * ROWB) + i * 16 * ROWB, off, s);
         };
         typedef int v2i_t __attribute__((ext_vector_type(2)));
         auto read_tr = [&](const uint8_t* base, int h, int j, int s) -> v4i {  // K rows 64 s + 16 g .. + 15
@@ -230,8 +282,15 @@ struct GemmPipe {
             const v2i_t y = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lp)(base + rt[h][j] + (s * 64 + 8) * hn(h)));
             return (v4i){x[0], x[1], y[0], y[1]};
         };
-        auto read_b = [&](auto HH, int set, int slot) {
+        auto read_b = [&](auto HH, int set, int slot, int kt) {
             constexpr int h = decltype(HH)::value;
+            uint32_t off[2];
+            if constexpr (!BTR) at(off, A_REG + wb[h]);
+            if constexpr (IS_MX) {
+#pragma unroll
+                for (int j = 0; j < fnh(h); ++j)
+                    swb[set][j / 2][j % 2] = read_scale(kt, SCA * 128 + h * hn(0) + wn * whn(h) + j * 16);
+            }
 #pragma unroll
             for (int j = 0; j < fnh(h); ++j)
 #pragma unroll
@@ -245,7 +304,7 @@ struct GemmPipe {
                             fb[set][j][s] = read_tr(base, h, j, s);
                         }
                     } else {
-                        fb[set][j][s] = read_frag(sB + wb[h] + slot * (BN * ROWB) + j * 16 * ROWB, s);
+                        fb[set][j][s] = read_frag(sA + slot * (BN * ROWB) + j * 16 * ROWB, off, s);
                     }
                 }
         };
@@ -260,9 +319,30 @@ struct GemmPipe {
                 acc_t& c = acc[ha * fmh(0) + i][hb * fnh(0) + j];
                 if constexpr (OP == OP_I8)
                     c = __builtin_amdgcn_mfma_i32_16x16x64_i8(fb[set][j][s], fa[ha][i][s], c, 0, 0, 0);
-                else
+                else if constexpr (OP == OP_F8)
                     c = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fb[set][j][s], fa[ha][i][s], c, BLGP, CBSZ, 0, 0, 0,
                                                                          0);
+                else {
+                    const v4i u = fb[set][j][s], v = fa[ha][i][s];
+                    const v8i b8 = (v8i){u[0], u[1], u[2], u[3], 0, 0, 0, 0}, a8 = (v8i){v[0], v[1], v[2], v[3], 0, 0, 0, 0};
+                    const int sb = __builtin_bit_cast(int, swb[set][j / 2]), sa = __builtin_bit_cast(int, swa[ha][i / 2]);
+                    // (the byte of an operand's scale register: 2 (fragment % 2) + s; an immediate of the instruction)
+                    auto f = [&](auto SB, auto SA) {
+                        c = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b8, a8, c, BLGP, CBSZ, decltype(SB)::value, sb,
+                                                                             decltype(SA)::value, sa);
+                    };
+                    if (s == 0) {
+                        if (j % 2 == 0 && i % 2 == 0) f(I0{}, I0{});
+                        if (j % 2 == 0 && i % 2 == 1) f(I0{}, I2{});
+                        if (j % 2 == 1 && i % 2 == 0) f(I2{}, I0{});
+                        if (j % 2 == 1 && i % 2 == 1) f(I2{}, I2{});
+                    } else {
+                        if (j % 2 == 0 && i % 2 == 0) f(I1{}, I1{});
+                        if (j % 2 == 0 && i % 2 == 1) f(I1{}, I3{});
+                        if (j % 2 == 1 && i % 2 == 0) f(I3{}, I1{});
+                        if (j % 2 == 1 && i % 2 == 1) f(I3{}, I3{});
+                    }
+                }
             }
         };
 
@@ -271,23 +351,22 @@ struct GemmPipe {
 #pragma unroll
             for (int j = 0; j < FN; ++j) acc[i][j] = (acc_t){};
 
-        using I0 = std::integral_constant<int, 0>;
-        using I1 = std::integral_constant<int, 1>;
-        using I2 = std::integral_constant<int, 2>;
-        using I3 = std::integral_constant<int, 3>;
         // prologue: the ring's halves in flight, H(0) and H(1) into registers, then H(4 ST) into the slot of H(0)
+        // (scales where the loop's phases 2 would have requested them, so that `outstanding` holds from phase 0 on)
+        request_scales(0);
 #pragma unroll
         for (int k = 0; k < ST; ++k) {
             request(I0{}, k, k);
             request(I1{}, k, k);
             request(I2{}, k, k);
+            if (k >= ST - 2) request_scales(k - ST + 3);
             request(I3{}, k, k);
         }
         __builtin_amdgcn_sched_barrier(0);
         wait_vmcnt<RING - ca(0) - cb(0)>();
         stage_barrier();
-        read_a(I0{}, 0);
-        read_b(I0{}, 0, 0);
+        read_a(I0{}, 0, 0);
+        read_b(I0{}, 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
         wait_half<RING - ca(0) - cb(0)>();
         stage_barrier();
@@ -308,14 +387,17 @@ struct GemmPipe {
             stage_barrier();
             multiply(HA{}, HB{}, set, 0, LEAD);
             __builtin_amdgcn_sched_barrier(0);
-            if constexpr (P == 0) read_b(I1{}, set1, SL);
-            if constexpr (P == 1) read_a(I1{}, SL);
-            if constexpr (P == 2) read_a(I0{}, SN);
-            if constexpr (P == 3) read_b(I0{}, set1, SN);
+            if constexpr (P == 0) read_b(I1{}, set1, SL, kt);
+            if constexpr (P == 1) read_a(I1{}, SL, kt);
+            if constexpr (P == 2) read_a(I0{}, SN, kt + 1);
+            if constexpr (P == 3) read_b(I0{}, set1, SN, kt + 1);
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (P == 0) request(I1{}, kt + ST, SL);
             if constexpr (P == 1) request(I2{}, kt + ST, SL);
-            if constexpr (P == 2) request(I3{}, kt + ST, SL);
+            if constexpr (P == 2) {
+                request_scales(kt + 3);
+                request(I3{}, kt + ST, SL);
+            }
             if constexpr (P == 3) request(I0{}, kt + 1 + ST, SN);
             __builtin_amdgcn_sched_barrier(0);
             multiply(HA{}, HB{}, set, LEAD, NX);

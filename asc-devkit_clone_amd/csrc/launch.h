@@ -199,6 +199,7 @@ struct MxGemmArgs {
     int splits;             // (set by the launcher) workgroups per tile of the K-split form
 };
 hipError_t launch_mx_gemm(const MxGemmArgs& a, hipStream_t st);
+hipError_t launch_mx_fp4_pipe(const MxGemmArgs& a, hipStream_t st);  // gemm_pipe_mx.hip; E2M1 elements, K % 128 == 0
 // MX-FP4 at decode-sized batches (M <= 64) with the scales read in place: with few 64 x 64 tiles (N / 64 well under
 // 256) K is split across workgroups as well, the partials meeting in the workspace; the workgroups per tile (1: not
 // used) and the workspace the partials need

@@ -11,8 +11,8 @@
 // FP4 (cbsz = blgp = 4): per lane 32 E2M1 values (16 bytes, one MX block) of row (lane % 32) at k block
 // (lane / 32), and one E8M0 scale byte for that (row, block) -- the hardware applies 2^(e-127) per 32-element
 // block, which is exactly the MX product.  Two fp4 per byte, even k in the low nibble: the reference packing
-// (gen_data.py:25-34) is also the MFMA's nibble order.  Block tile 256 x 256, 256 fp4 of K per stage (128-byte
-// rows, four k-steps per barrier), two stages, 8 waves (4 x 2), wave tile 64 x 128.  The E8M0 scales, rearranged
+// (gen_data.py:25-34) is also the MFMA's nibble order.  These are the decode-sized 64 x 64 tiles; larger MX-FP4
+// problems run on gemm_pipe_mx.hip.  The E8M0 scales, rearranged
 // stage-major by mx_scale_stage_major_kernel, ride in the same LDS stage.  B stored [K, N]
 // (the reference's non-transposed layout, two fp4 per byte along N) is first transposed to [N, K] in a
 // workspace by fp4_transpose_kernel.
@@ -391,7 +391,6 @@ hipError_t launch_mx_gemm(const MxGemmArgs& a, hipStream_t st)
         return launch_mx_tiled<64, 64, 2, 2, 4, 64, OP_MXFP6, 0>(a, st);
     }
     if (fp4) {
-        if (big) return launch_mx_tiled<256, 256, 4, 2, 2, 128, OP_MXFP4, 0>(a, st);
         // decode-sized batches (M <= 64) with A's scales row-major [M, sK] and B's row-major [N, sK] or in block
         // pairs [sK / 2, N, 2] (N even; 4-byte aligned): the 64 x 64 tiles read the scales as given, so no
         // rearrangement launch precedes the GEMM (measured, K = 4096, N = 11008, row-major B scales: M = 1 / 16 / 64
@@ -410,7 +409,12 @@ hipError_t launch_mx_gemm(const MxGemmArgs& a, hipStream_t st)
             if (a.N % 2 == 0)
                 return split ? launch_mx_split<2>(b, st) : launch_mx_tiled<64, 64, 2, 2, 4, 64, OP_MXFP4, 0, true, 2>(a, st);
         }
-        return launch_mx_tiled<64, 64, 2, 2, 4, 64, OP_MXFP4, 0>(a, st);
+        // above decode size: the pipelined tiles, where they are more than half the CUs; with fewer, twice as many 64 x 64
+        // tiles (K = 4096, N = 4096, M = 128: 12.1 against 12.7 us; K = 8192, N = 1024, M = 100: 17.0 against 19.0; at
+        // K = 384, N = 2048, M = 1024, 256 tiles, 16.5 against 9.2)
+        if (((a.M + 63) / 64) * ((a.N + 127) / 128) <= 128)
+            return launch_mx_tiled<64, 64, 2, 2, 4, 64, OP_MXFP4, 0>(a, st);
+        return launch_mx_fp4_pipe(a, st);
     }
     switch (a.fmt_a | (a.fmt_b << 3)) {
     case F8F6F4_E4M3 | (F8F6F4_E4M3 << 3): return launch_mx_f8<F8F6F4_E4M3 | (F8F6F4_E4M3 << 3)>(a, st);

@@ -90,3 +90,41 @@ def test_fp8_pipe(ascq_gpu, M, N, K, trans_b):
         torch.cuda.synchronize()
         assert not bool(out[M * N:].any()), c_type
         assert torch.equal(out[:M * N].view(M, N).cpu(), ref.float().to(dt)), c_type
+
+
+# (M, N, K): more than 128 tiles of 64 x 128, the tile pick_pipe_tile chooses; odd and even counts of half stages
+MX_SHAPES = [(513, 1900, 640), (1100, 2100, 384), (3353, 536, 640), (4127, 932, 896), (1607, 3736, 1152), (3457, 1732, 128),
+             (3273, 1816, 384), (3301, 3804, 128)]
+E2M1 = torch.tensor([0, 0.5, 1, 1.5, 2, 3, 4, 6, 0, -0.5, -1, -1.5, -2, -3, -4, -6], dtype=torch.float64)
+
+
+@pytest.mark.parametrize("pairs", [False, True])
+@pytest.mark.parametrize("M,N,K", MX_SHAPES)
+def test_mxfp4_pipe(ascq_gpu, M, N, K, pairs):
+    """Elements of at most two significant bits and block scales of 2^-2 .. 2^2: products are multiples of 2^-6 and the
+    sums (at most 2^18 in magnitude here) are exact in fp32, so f32 C equals the fp64 product, bf16 C its rounding"""
+    g = torch.Generator().manual_seed(M + N + K + pairs)
+    A = torch.randint(0, 256, (M, K // 2), generator=g, dtype=torch.uint8)
+    B = torch.randint(0, 256, (N, K // 2), generator=g, dtype=torch.uint8)
+    sA = torch.randint(125, 130, (M, K // 32), generator=g, dtype=torch.uint8)
+    sB = torch.randint(125, 130, (N, K // 32), generator=g, dtype=torch.uint8)
+
+    def decode(x, s):
+        v = torch.stack([E2M1[(x & 15).long()], E2M1[(x >> 4).long()]], -1).reshape(x.shape[0], -1)
+        return v * torch.exp2(s.double() - 127).repeat_interleave(32, 1)
+
+    ref = decode(A, sA) @ decode(B, sB).t()
+    assert float(ref.abs().max()) < 2.0 ** 18
+    to_pairs = lambda s: s.reshape(s.shape[0], -1, 2).permute(1, 0, 2).contiguous()  # noqa: E731
+    for c_type, dt in [(ascq_gpu.F32, torch.float32), (ascq_gpu.BF16, torch.bfloat16)]:
+        mm = ascq_gpu.Matmul(ascq_gpu.FP4_E2M1, ascq_gpu.FP4_E2M1, c_type, 0, ascq_gpu.E8M0)
+        mm.SetOrgShape(M, N, K)
+        mm.SetTensorA(A.cuda())
+        mm.SetTensorB(B.cuda(), True)
+        mm.SetTensorScaleA(to_pairs(sA).cuda() if pairs else sA.cuda(), pairs)
+        mm.SetTensorScaleB(to_pairs(sB).cuda() if pairs else sB.cuda(), not pairs)
+        out = torch.zeros(M * N + 16, dtype=dt, device="cuda")
+        mm.IterateAll(out)
+        torch.cuda.synchronize()
+        assert not bool(out[M * N:].any()), c_type
+        assert torch.equal(out[:M * N].view(M, N).cpu(), ref.float().to(dt)), c_type
