@@ -139,6 +139,7 @@ struct ascq_matmul_s {
     void* ws = nullptr;
     size_t ws_bytes = 0;
     bool ws_owned = false;
+    bool no_alloc = false;  // a call of the allocation-free form (set in its copy of the handle)
 };
 
 namespace {
@@ -326,6 +327,100 @@ ascq_status prepare_byte_operands(ascq_matmul_s* h, hipStream_t st, ByteOperands
         o.lda = h->K;
         o.trans_a = 0;
     }
+    return ASCQ_OK;
+}
+
+// Operands whose rows the aligned kernels cannot take -- a K that is not a multiple of 16 bytes, rows or pointers off
+// their alignment (16 bytes; a [K, N] B: 4) -- are copied to aligned zero-padded rows in the workspace: a copy at the
+// memory rate against tiles that realign every chunk they load (int8 1030 x 4100 x 4095, B [K, N]: 139 -> 31 us; one row: 66 -> 18 us).  The
+// room is optional: a caller's workspace without it, a stream under capture whose handle holds too little, or a failed
+// allocation leave the call to the any-alignment tiles.
+struct PackPlan {
+    bool a, b;
+    int64_t kp, pitch_b;  // bytes of a packed row of A (and of a K-contiguous B); of a packed row of B
+    size_t a_bytes, b_bytes;
+};
+PackPlan pack_plan(bool fp8, const ByteOperands& o, int64_t m, int64_t n, int64_t k)
+{
+    PackPlan p{};
+    if (o.trans_a) return p;
+    const bool k16 = k % 16 == 0;
+    p.kp = (k + 15) / 16 * 16;
+    p.a = o.lda % 16 != 0 || (uintptr_t)o.A % 16 != 0 || (!k16 && (o.trans_b || fp8));
+    p.b = o.trans_b ? o.ldb % 16 != 0 || (uintptr_t)o.B % 16 != 0 || !k16 : o.ldb % 4 != 0 || (uintptr_t)o.B % 4 != 0;
+    p.pitch_b = o.trans_b ? p.kp : (n + 15) / 16 * 16;
+    p.a_bytes = p.a ? align256((size_t)m * (size_t)p.kp) : 0;
+    p.b_bytes = p.b ? align256((size_t)(o.trans_b ? n : k) * (size_t)p.pitch_b) : 0;
+    if (p.a_bytes >= (1u << 31) || p.b_bytes >= (1u << 31)) return PackPlan{};
+    return p;
+}
+
+// what the packed operands of the org shape need on top of workspace_need (pointers, where set, included)
+size_t pack_need(const ascq_matmul_s* h)
+{
+    const Kind kind = kind_of(h->ty);
+    if ((kind != K_INT8 && kind != K_F8) || h->M <= 0 || h->trans_a || bytes_nz_b(h)) return 0;
+    const ByteOperands o{(const uint8_t*)h->a, (const uint8_t*)h->b, h->K, h->trans_b ? h->K : h->N, 0, h->trans_b};
+    const PackPlan p = pack_plan(kind == K_F8, o, h->M, h->N, h->K);
+    return p.a_bytes + p.b_bytes;
+}
+
+ascq_status pack_byte_operands(ascq_matmul_s* h, hipStream_t st, int64_t m, int64_t n, int64_t* k, bool fp8,
+                               ByteOperands& o, int* a_padded)
+{
+    const PackPlan p = pack_plan(fp8, o, m, n, *k);
+    if (!p.a && !p.b) return ASCQ_OK;
+    // (the smallest calls keep the element-wise kernel, which needs no workspace and which ASCQ_LOG names, though the
+    // copy and the GEMM would be faster: 32 x 32 x 40 in 17.1 us, 40 x 40 x 41 in 9.3)
+    if (fp8 && !o.trans_b && m * n * *k <= 32 * 32 * 40) return ASCQ_OK;
+    const size_t base = align256(workspace_need(h)), need = base + p.a_bytes + p.b_bytes;
+    if (h->ws_bytes < need) {
+        if (h->no_alloc || (h->ws && !h->ws_owned)) return ASCQ_OK;
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+            (void)hipGetLastError();
+            return ASCQ_OK;
+        }
+        void* ws = nullptr;
+        if (hipMalloc(&ws, need) != hipSuccess) {
+            (void)hipGetLastError();
+            return ASCQ_OK;
+        }
+        // (operands that prepare_byte_operands already put into the old workspace move along)
+        if (h->ws && base > 0) {
+            const hipError_t e = hipMemcpyAsync(ws, h->ws, base < h->ws_bytes ? base : h->ws_bytes, hipMemcpyDeviceToDevice, st);
+            if (e != hipSuccess) {
+                (void)hipFree(ws);
+                return hip_status(e, "move workspace");
+            }
+            const uint8_t *lo = (const uint8_t*)h->ws, *hi = lo + h->ws_bytes;
+            if (o.A >= lo && o.A < hi) o.A = (uint8_t*)ws + (o.A - lo);
+            if (o.B >= lo && o.B < hi) o.B = (uint8_t*)ws + (o.B - lo);
+        }
+        if (h->ws) (void)hipFree(h->ws);
+        h->ws = ws;
+        h->ws_bytes = need;
+        h->ws_owned = true;
+    }
+    uint8_t* pa = (uint8_t*)h->ws + base;
+    uint8_t* pb = pa + p.a_bytes;
+    const ascq::PackRows ja{p.a ? pa : nullptr, o.A, m, *k, o.lda};
+    const ascq::PackRows jb = o.trans_b ? ascq::PackRows{p.b ? pb : nullptr, o.B, n, *k, o.ldb}
+                                        : ascq::PackRows{p.b ? pb : nullptr, o.B, *k, n, o.ldb};
+    const hipError_t e = ascq::launch_pack_rows(ja, jb, st);
+    if (e == hipErrorInvalidValue) return ASCQ_OK;  // (spans the copy does not take: nothing was launched)
+    if (e != hipSuccess) return hip_status(e, "pack operands");
+    if (p.a) {
+        o.A = pa;
+        o.lda = p.kp;
+        *a_padded = 1;
+    }
+    if (p.b) {
+        o.B = pb;
+        o.ldb = p.pitch_b;
+    }
+    // both K-contiguous operands zero-padded: the GEMM runs whole chunks
+    if (o.trans_b && p.a && p.b) *k = p.kp;
     return ASCQ_OK;
 }
 
@@ -561,6 +656,7 @@ ascq_status ascq_matmul_workspace_size(ascq_matmul_t h, size_t* bytes)
 {
     if (!h || !bytes) return fail(ASCQ_E_INVALID_ARG, "workspace_size: null argument");
     *bytes = workspace_need(h);
+    if (const size_t pack = pack_need(h)) *bytes = align256(*bytes) + pack;  // (optional room, see pack_byte_operands)
     return ASCQ_OK;
 }
 
@@ -625,6 +721,8 @@ ascq_status ascq_matmul_iterate_all(ascq_matmul_t h, void* c, uint8_t en_atomic,
         }
         ByteOperands o;
         ascq_status s = prepare_byte_operands(h, st, o);
+        int padded = 0;
+        if (s == ASCQ_OK) s = pack_byte_operands(h, st, m, n, &g.K, false, o, &padded);
         if (s != ASCQ_OK) return s;
         g.A = (const int8_t*)o.A;
         g.B = (const int8_t*)o.B;
@@ -739,6 +837,8 @@ ascq_status ascq_matmul_iterate_all(ascq_matmul_t h, void* c, uint8_t en_atomic,
         ascq::GemmF8Args g{};
         ByteOperands o;
         ascq_status s = prepare_byte_operands(h, st, o);
+        g.K = k;
+        if (s == ASCQ_OK) s = pack_byte_operands(h, st, m, n, &g.K, true, o, &g.a_padded);
         if (s != ASCQ_OK) return s;
         g.A = o.A;
         g.B = o.B;
@@ -750,7 +850,6 @@ ascq_status ascq_matmul_iterate_all(ascq_matmul_t h, void* c, uint8_t en_atomic,
         g.C = c;
         g.M = m;
         g.N = n;
-        g.K = k;
         g.ldc = h->N;
         g.qvec = h->qvec;
         g.qscalar = h->qscalar;
@@ -894,7 +993,9 @@ ascq_status ascq_matmul_iterate_all_noalloc(ascq_matmul_t h, void* c, uint8_t en
                     "iterate_all_noalloc: this handle needs %zu bytes of workspace, above the %zu-byte static scratch "
                     "(use ascq_matmul_iterate_all with a workspace)", need, (size_t)ASCQ_NOALLOC_SCRATCH_BYTES);
     void* ptr = nullptr;
-    if (need > 0) {
+    const size_t pack = pack_need(h);  // taken where the scratch has room for it
+    const bool use = need > 0 || (pack > 0 && align256(need) + pack <= ASCQ_NOALLOC_SCRATCH_BYTES);
+    if (use) {
         ascq_status s = scratch_for_current_device(&ptr);
         if (s != ASCQ_OK) return s;
     }
@@ -902,8 +1003,9 @@ ascq_status ascq_matmul_iterate_all_noalloc(ascq_matmul_t h, void* c, uint8_t en
     // and allocates nothing); the caller's handle is only read, so it never holds the scratch as its workspace
     ascq_matmul_s tmp = *h;
     tmp.ws = ptr;
-    tmp.ws_bytes = need > 0 ? (size_t)ASCQ_NOALLOC_SCRATCH_BYTES : 0;
+    tmp.ws_bytes = use ? (size_t)ASCQ_NOALLOC_SCRATCH_BYTES : 0;
     tmp.ws_owned = false;
+    tmp.no_alloc = true;
     return ascq_matmul_iterate_all(&tmp, c, en_atomic, stream);
 }
 

@@ -362,7 +362,7 @@ static hipError_t launch_f8_fmt(const GemmF8Args& a, bool ua, hipStream_t st)
         // with a workspace for the partials, the K split across workgroups as well where decode_splits (the int8
         // Matmul's rule) finds it faster: B [N, K] on the 32 x 32 tiles, B [K, N] (16-byte K rows) on 32 x 128 tiles
         const int splits = decode_splits(a.M, a.N, a.K, a.trans_b);
-        const bool b_tr = !a.trans_b && a.ldb % 16 == 0 && (uintptr_t)a.B % 16 == 0;
+        const bool b_tr = !a.trans_b && a.ldb % 16 == 0 && (uintptr_t)a.B % 16 == 0 && a.N % 4 == 0;
         if ((a.trans_b || b_tr) && splits > 1 && c_wide && a.atomic == C_STORE && a.ws &&
             a.ws_bytes >= decode_split_ws_bytes(a.M, a.N, a.K, a.trans_b) &&
             ((a.M + 63) / 64) * ((a.N + 127) / 128) >= 32) {
@@ -404,9 +404,9 @@ hipError_t launch_gemm_f8(const GemmF8Args& a, hipStream_t st)
     const int64_t es = bf ? 2 : 1;
     const bool a_ok = !a.trans_a && (a.lda * es) % 16 == 0 && ((uintptr_t)a.A % 16 == 0) && a.lda * es * a.M < (1ll << 31);
     const bool b_ok = a.trans_b ? ((a.ldb * es) % 16 == 0 && ((uintptr_t)a.B % 16 == 0) && a.ldb * es * a.N < (1ll << 31))
-                                : (a.ldb % 4 == 0 && a.N % 4 == 0 && ((uintptr_t)a.B % 4 == 0) && a.ldb * a.K < (1ll << 31));
+                                : (a.ldb % 4 == 0 && ((uintptr_t)a.B % 4 == 0) && a.ldb * a.K < (1ll << 31));
     // the tiled epilogue addresses a 256-row output tile with 32-bit offsets
-    const bool tiled = a_ok && b_ok && (a.K * es) % 16 == 0 && a.ldc < (1ll << 21);
+    const bool tiled = a_ok && b_ok && ((a.K * es) % 16 == 0 || (!a.trans_b && a.a_padded)) && a.ldc < (1ll << 21);
     // otherwise fp8 with A [M, K] and B [N, K] (any alignment, any K) takes the any-alignment tiles
     const char* why = tiled ? nullptr
                       : bf ? "bf16 operands: K not a multiple of 8"

@@ -529,9 +529,9 @@ hipError_t launch_gemm_i8(const GemmI8Args& a, hipStream_t st)
 {
     const bool a_ok = !a.trans_a && a.lda % 16 == 0 && ((uintptr_t)a.A % 16 == 0) && a.lda * a.M < (1ll << 31);
     const bool b_ok = a.trans_b ? (a.ldb % 16 == 0 && ((uintptr_t)a.B % 16 == 0) && a.ldb * a.N < (1ll << 31))
-                                : (a.ldb % 4 == 0 && a.N % 4 == 0 && ((uintptr_t)a.B % 4 == 0) && a.ldb * a.K < (1ll << 31));
+                                : (a.ldb % 4 == 0 && ((uintptr_t)a.B % 4 == 0) && a.ldb * a.K < (1ll << 31));
     // the tiled epilogue addresses a 256-row output tile with 32-bit offsets
-    if (a_ok && b_ok && a.K % 16 == 0 && a.ldc < (1ll << 21)) {
+    if (a_ok && b_ok && (a.K % 16 == 0 || !a.trans_b) && a.ldc < (1ll << 21)) {
         // small problems (the W8A8 sample, 128 x 256 x 512: 4 tiles of 64 x 128) take 32 x 32 single-wave tiles so
         // that at least 32 workgroups share the work
         const bool tiny = ((a.M + 63) / 64) * ((a.N + 127) / 128) < 32;
@@ -543,7 +543,7 @@ hipError_t launch_gemm_i8(const GemmI8Args& a, hipStream_t st)
         // against 21.4 us)
         const int64_t t64 = ((a.M + 63) / 64) * ((a.N + 63) / 64);
         const bool skinny = a.M <= 32 || (a.M <= 64 && t64 < 160);
-        const bool ksplit = (tiny || skinny) && a.K % 256 == 0 && a.atomic == C_STORE;
+        const bool ksplit = (tiny || skinny) && a.K % 256 == 0 && a.atomic == C_STORE && (a.trans_b || a.N % 4 == 0);
         // decode-sized batches (up to 64 rows, one row tile of 32 or 64) with a workspace for the partials: the K split
         // across workgroups as well, where decode_splits finds it faster (B [K, N]: x 128 tiles; B [N, K]: x 32)
         const int splits = decode_splits(a.M, a.N, a.K, a.trans_b);
@@ -554,7 +554,7 @@ hipError_t launch_gemm_i8(const GemmI8Args& a, hipStream_t st)
             const bool m32 = a.M <= 32;
             if (a.trans_b)
                 return m32 ? launch_i8_split<true, false, 32, 32, 4>(b, st) : launch_i8_split<true, false, 64, 32, 4>(b, st);
-            if (a.ldb % 16 == 0 && (uintptr_t)a.B % 16 == 0)
+            if (a.ldb % 16 == 0 && (uintptr_t)a.B % 16 == 0 && a.N % 4 == 0)
                 return m32 ? launch_i8_split<false, true, 32, 128, 3>(b, st)
                            : launch_i8_split<false, true, 64, 128, 3>(b, st);
         }
@@ -576,7 +576,7 @@ hipError_t launch_gemm_i8(const GemmI8Args& a, hipStream_t st)
         return launch_gemm_i8_pipe(a, st);
     }
     // K not a multiple of 16, or operands / leading dimensions not 16-byte (A, K-contiguous B) or 4-byte ([K, N] B)
-    // aligned: the any-alignment tiles (GemmCoreUA), 64 x 64 while that leaves fewer than 256 workgroups of 128 x 128
+    // aligned, where the host layer had no workspace to pack them into: the any-alignment tiles (GemmCoreUA), 64 x 64 while that leaves fewer than 256 workgroups of 128 x 128
     const int64_t a_span = a.lda * (a.M - 1) + a.K, b_span = a.trans_b ? a.ldb * (a.N - 1) + a.K : a.ldb * (a.K - 1) + a.N;
     const char* why = a.trans_a                            ? "A given [K, M]"
                       : (a_span >= (1ll << 31) - 16 || b_span >= (1ll << 31) - 16) ? "an operand spans 2^31 bytes"

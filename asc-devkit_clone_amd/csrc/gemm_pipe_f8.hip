@@ -16,8 +16,8 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_f8_pipe_kernel(GemmF8Arg
     const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
     const int rows = (int)(p.M - m0 < BM ? p.M - m0 : BM), cols = (int)(p.N - n0 < BN ? p.N - n0 : BN);
     PipeArgs c{};
-    c.a = make_rsrc4(p.A, (uint32_t)(p.lda * (p.M - 1) + p.K));
-    c.b = make_rsrc4(p.B, (uint32_t)(BTR ? p.ldb * (p.K - 1) + p.N : p.ldb * (p.N - 1) + p.K));
+    c.a = make_rsrc4(p.A, (uint32_t)(p.lda * (p.M - 1) + (p.K + 15) / 16 * 16));  // (whole chunks: within the pitch)
+    c.b = make_rsrc4(p.B, (uint32_t)(BTR ? p.ldb * (p.K - 1) + (p.N + 3) / 4 * 4 : p.ldb * (p.N - 1) + p.K));
     c.lda = (uint32_t)p.lda;
     c.ldb = (uint32_t)p.ldb;
     c.a0 = (uint32_t)(m0 * p.lda);

@@ -1,5 +1,6 @@
 // gemm_pipe_i8.hip -- the int8 Matmul on the pipelined tiles of gemm_pipe.h: the GEMM and epilogues of gemm_i8.hip for
-// A [M, K] with 16-byte-aligned rows and B [N, K] the same, or B [K, N] with 4-byte-aligned rows; K a multiple of 16.
+// A [M, K] with 16-byte-aligned rows and B [N, K] the same, or B [K, N] with 4-byte-aligned rows (whose range
+// is rounded up to whole dwords: they lie in the row's pitch).
 #include "common.h"
 #include "gemm_pipe.h"
 #include "launch.h"
@@ -16,8 +17,8 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_i8_pipe_kernel(GemmI8Arg
     const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
     const int rows = (int)(p.M - m0 < BM ? p.M - m0 : BM), cols = (int)(p.N - n0 < BN ? p.N - n0 : BN);
     PipeArgs c{};
-    c.a = make_rsrc4(p.A, (uint32_t)(p.lda * (p.M - 1) + p.K));
-    c.b = make_rsrc4(p.B, (uint32_t)(BTR ? p.ldb * (p.K - 1) + p.N : p.ldb * (p.N - 1) + p.K));
+    c.a = make_rsrc4(p.A, (uint32_t)(p.lda * (p.M - 1) + (p.K + 15) / 16 * 16));  // (whole chunks: within the pitch)
+    c.b = make_rsrc4(p.B, (uint32_t)(BTR ? p.ldb * (p.K - 1) + (p.N + 3) / 4 * 4 : p.ldb * (p.N - 1) + p.K));
     c.lda = (uint32_t)p.lda;
     c.ldb = (uint32_t)p.ldb;
     c.a0 = (uint32_t)(m0 * p.lda);

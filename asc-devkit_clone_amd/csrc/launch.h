@@ -107,8 +107,8 @@ struct GemmI8Args {
     int splits;           // (set by the launcher) workgroups per tile of the K-split form
 };
 hipError_t launch_gemm_i8(const GemmI8Args& a, hipStream_t st);
-// gemm_pipe_i8.hip: A [M, K] with 16-byte-aligned rows and B [N, K] the same, or B [K, N] with 4-byte-aligned rows; K a
-// multiple of 16, operands below 2^31 bytes
+// gemm_pipe_i8.hip: A [M, K] with 16-byte-aligned rows and B [N, K] the same with K a multiple of 16, or B [K, N] with
+// 4-byte-aligned rows and any K (A's bytes past K within a 16-byte chunk meet zeros); operands below 2^31 bytes
 hipError_t launch_gemm_i8_pipe(const GemmI8Args& a, hipStream_t st);
 // Decode-sized batches (M <= 64: one row tile of 32 or 64 rows; K % 256 == 0) -- B given [K, N] (trans_b 0) with long
 // K or wide N on x 128 tiles, B given [N, K] with long K and few x 32 tiles -- split each tile's K over several
@@ -140,9 +140,11 @@ struct GemmF8Args {
     uint8_t* ws;          // decode-sized batches: room for the K-split partials (decode_split_ws_bytes), or null
     size_t ws_bytes;
     int splits;           // (set by the launcher) workgroups per tile of the K-split form
+    int a_padded;         // A's rows hold zeros from K up to a multiple of 16
 };
 hipError_t launch_gemm_f8(const GemmF8Args& a, hipStream_t st);
-// gemm_pipe_f8.hip: A [M, K] and B [N, K] fp8 with 16-byte-aligned rows below 2^31 bytes in all, K % 128 == 0
+// gemm_pipe_f8.hip: as gemm_pipe_i8.hip, but with B [K, N] and K not a multiple of 16 A's rows are zero-padded to one
+// (a_padded: a NaN or infinity past K would not vanish against B's zeros)
 hipError_t launch_gemm_f8_pipe(const GemmF8Args& a, hipStream_t st);
 
 // group_gemm.hip
@@ -212,6 +214,14 @@ hipError_t launch_fp4_to_fp6_planes(uint8_t* P, uint8_t* Q, const uint8_t* src, 
                                     hipStream_t st);
 // transpose.hip: int8 [rows, cols] -> [cols, rows]; fp4 [K, N] -> [N, K] tiled fast path (returns false when
 // the shape / alignment does not allow it)
+// rows of any byte alignment [rows][ld] -> zero-padded 16-byte-aligned rows [rows][cols rounded up to 16]; two jobs in
+// one launch, a job with a null dst is none; sources below 2^31 bytes
+struct PackRows {
+    uint8_t* dst;
+    const uint8_t* src;
+    int64_t rows, cols, ld;
+};
+hipError_t launch_pack_rows(const PackRows& a, const PackRows& b, hipStream_t st);
 hipError_t launch_transpose_i8(uint8_t* dst, const uint8_t* src, int64_t rows, int64_t cols, hipStream_t st);
 bool fp4_transpose_tiled(uint8_t* dst, const uint8_t* src, int64_t K, int64_t N, hipStream_t st, hipError_t* err);
 size_t mx_scale_workspace_bytes(int64_t M, int64_t N, int64_t K);

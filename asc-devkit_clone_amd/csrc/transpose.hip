@@ -13,6 +13,7 @@
 // Tiles on the edge load zeros past the matrix and store only inside it; the fast path needs the row length
 // in bytes and the row count to be multiples of 16 (the caller falls back to a plain kernel otherwise).
 #include "common.h"
+#include "gemm_core.h"
 #include "launch.h"
 
 namespace ascq {
@@ -247,6 +248,50 @@ hipError_t launch_hif8_to_bf16(uint16_t* dst, int64_t ldd, const uint8_t* src, i
         if (blocks > 65536) blocks = 65536;
         hipLaunchKernelGGL(hif8_to_bf16_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, st, dst, ldd, src, R, C);
     }
+    return hipGetLastError();
+}
+
+// Rows of any byte alignment -> 16-byte-aligned rows, zero-padded: dst [rows][pitch] (pitch = cols rounded up to 16)
+// from src [rows][ld], one 16-byte chunk per thread.  A chunk's bytes lie in at most two 16-byte-aligned blocks of the
+// source, each of which holds a byte of it (so no access leaves the operand's pages); its five dwords are picked from
+// them and shifted into place.  Up to two jobs (A and B of a Matmul) in one launch.
+__global__ __launch_bounds__(256) void pack_rows_kernel(PackRows ja, PackRows jb, uint32_t blocks_a)
+{
+    const bool is_a = blockIdx.x < blocks_a;
+    const PackRows j = is_a ? ja : jb;
+    const uint32_t chunks = (uint32_t)((j.cols + 15) / 16);
+    const int64_t i = (int64_t)(is_a ? blockIdx.x : blockIdx.x - blocks_a) * 256 + threadIdx.x;
+    if (i >= (int64_t)chunks * j.rows) return;
+    const uint32_t r = (uint32_t)i / chunks, c = (uint32_t)i % chunks;
+    const int valid = j.cols - (int64_t)c * 16 >= 16 ? 16 : (int)(j.cols - (int64_t)c * 16);
+    uint32_t delta;
+    const rsrc_t src = make_rsrc_a16(j.src, (uint32_t)((int64_t)(j.rows - 1) * j.ld + j.cols), delta);
+    const uint32_t off = delta + r * (uint32_t)j.ld + c * 16u, s = off & 15u, q = s >> 2, sh = s & 3u;
+    const u32x4 lo = bload16(src, off & ~15u), hi = bload16(src, (int)s + valid > 16 ? (off & ~15u) + 16u : OOB);
+    const uint32_t w[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    uint32_t d[5];
+#pragma unroll
+    for (int x = 0; x < 5; ++x) d[x] = q == 0 ? w[x] : (q == 1 ? w[x + 1] : (q == 2 ? w[x + 2] : w[x + 3]));
+    u32x4 out;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+        const int nv = valid - 4 * x;  // valid bytes of dword x
+        const uint32_t m = nv >= 4 ? ~0u : (nv <= 0 ? 0u : (1u << (8 * nv)) - 1u);
+        out[x] = __builtin_amdgcn_alignbyte(d[x + 1], d[x], sh) & m;
+    }
+    *(u32x4*)(j.dst + ((int64_t)r * chunks + c) * 16) = out;
+}
+
+hipError_t launch_pack_rows(const PackRows& a, const PackRows& b, hipStream_t st)
+{
+    auto blocks = [](const PackRows& j) { return j.dst ? (j.rows * ((j.cols + 15) / 16) + 255) / 256 : (int64_t)0; };
+    for (const PackRows* j : {&a, &b})
+        if (j->dst && (j->rows < 1 || j->cols < 1 || (j->rows - 1) * j->ld + j->cols >= (1ll << 31) - 32 ||
+                       j->rows * ((j->cols + 15) / 16) >= (1ll << 31) || (uintptr_t)j->dst % 16 != 0))
+            return hipErrorInvalidValue;
+    const int64_t ba = blocks(a), bb = blocks(b);
+    if (ba + bb == 0) return hipSuccess;
+    hipLaunchKernelGGL(pack_rows_kernel, dim3((unsigned)(ba + bb)), dim3(256), 0, st, a, b, (uint32_t)ba);
     return hipGetLastError();
 }
 

@@ -34,11 +34,13 @@ def _bits(t):
     return t.cpu().view(torch.int16).numpy().view(np.uint16)
 
 
+# odd N (odd pitches of C, a [K, N] B packed), and K of every remainder class of a chunk (operands packed): few rows too
+RAGGED = [(130, 1001, 2048), (300, 5003, 1040), (130, 1004, 2047), (1, 1030, 1009), (20, 515, 77), (33, 601, 1), (70, 130, 4095)]
+
+
 @pytest.mark.parametrize("trans_b", [False, True])
-@pytest.mark.parametrize("M,N,K", SHAPES + [(130, 1001, 2048), (300, 5003, 1040)])  # odd N: odd pitches of C
+@pytest.mark.parametrize("M,N,K", SHAPES + RAGGED)
 def test_int8_pipe(ascq_gpu, oracle, M, N, K, trans_b):
-    if not trans_b and N % 4:
-        pytest.skip("[K, N] with N % 4 != 0 takes the any-alignment tiles")
     rng = seeded(M + N + K + trans_b)
     A = rng.integers(-128, 128, (M, K), dtype=np.int8)
     B = rng.integers(-128, 128, (N, K) if trans_b else (K, N), dtype=np.int8)
@@ -69,10 +71,8 @@ def test_int8_pipe(ascq_gpu, oracle, M, N, K, trans_b):
 
 
 @pytest.mark.parametrize("trans_b", [False, True])
-@pytest.mark.parametrize("M,N,K", SHAPES + [(300, 5003, 1040)])
+@pytest.mark.parametrize("M,N,K", SHAPES + RAGGED)
 def test_fp8_pipe(ascq_gpu, M, N, K, trans_b):
-    if not trans_b and N % 4:
-        pytest.skip("[K, N] with N % 4 != 0 takes the generic kernel")
     g = torch.Generator().manual_seed(M + N + K + trans_b)
     A = torch.randint(-4, 5, (M, K), generator=g)
     B = torch.randint(-4, 5, (N, K) if trans_b else (K, N), generator=g)
@@ -90,6 +90,44 @@ def test_fp8_pipe(ascq_gpu, M, N, K, trans_b):
         torch.cuda.synchronize()
         assert not bool(out[M * N:].any()), c_type
         assert torch.equal(out[:M * N].view(M, N).cpu(), ref.float().to(dt)), c_type
+
+
+def test_ragged_without_a_workspace(ascq_gpu, oracle):
+    """Under stream capture a handle without a workspace allocates none: the any-alignment tiles, the same bits; and an
+    operand that follows NaN bytes of another buffer (fp8) reads none of them"""
+    M, N, K = 70, 200, 1003
+    rng = seeded(5)
+    A = rng.integers(-128, 128, (M, K), dtype=np.int8)
+    B = rng.integers(-128, 128, (K, N), dtype=np.int8)
+    a, b = _dev(A), _dev(B)
+    mm = ascq_gpu.Matmul(ascq_gpu.INT8, ascq_gpu.INT8, ascq_gpu.INT32)
+    mm.SetOrgShape(M, N, K)
+    mm.SetTensorA(a)
+    mm.SetTensorB(b)
+    out = torch.zeros((M, N), dtype=torch.int32, device="cuda")
+    st = torch.cuda.Stream()
+    st.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(st), torch.cuda.graph(graph, stream=st):
+        mm.IterateAll(out)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(out.cpu().numpy(), O.matmul_i8(A, B, None))
+    mm.IterateAll(out.zero_())  # eager: the packed form
+    np.testing.assert_array_equal(out.cpu().numpy(), O.matmul_i8(A, B, None))
+
+    buf = torch.full((M * K + 64,), 0x7F, dtype=torch.uint8, device="cuda")  # e4m3 NaN around A
+    buf[1:1 + M * K] = torch.ones(M * K).to(torch.float8_e4m3fn).view(torch.uint8).cuda()
+    ones = torch.ones((K, N)).to(torch.float8_e4m3fn).cuda()
+    f8 = ascq_gpu.Matmul(ascq_gpu.FP8_E4M3, ascq_gpu.FP8_E4M3, ascq_gpu.F32)
+    f8.SetOrgShape(M, N, K)
+    f8.SetTensorA(buf[1:1 + M * K])
+    f8.SetTensorB(ones)
+    y = torch.zeros((M, N), dtype=torch.float32, device="cuda")
+    f8.IterateAll(y)
+    assert bool((y == K).all())
 
 
 # (M, N, K): more than 128 tiles of 64 x 128, the tile pick_pipe_tile chooses; odd and even counts of half stages
