@@ -21,7 +21,7 @@ CSRC = PKG / "csrc"
 BUILD = PKG / "_build"
 LIB = PKG / "libascq.so"
 SOURCES = ["api.cpp", "quant.hip", "gemm_i8.hip", "gemm_f8.hip", "gemm_pipe_f8.hip", "gemm_pipe_i8.hip",
-           "gemm_pipe_mx.hip", "gemv_antiquant.hip", "aq_gemm.hip", "mx_gemm.hip", "transpose.hip", "layout.hip"]
+           "gemm_pipe_mx.hip", "gemm_pipe_group.hip", "gemv_antiquant.hip", "aq_gemm.hip", "mx_gemm.hip", "transpose.hip", "layout.hip"]
 ARCH = os.environ.get("ASCQ_OFFLOAD_ARCH", "gfx950")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 

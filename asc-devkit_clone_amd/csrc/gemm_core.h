@@ -28,11 +28,6 @@
 //    chunk l % (ROWB / 16)); the swizzle is applied on the global side.
 //  * Global reads are raw buffer loads: an out-of-range offset returns zeros, so tile edges and the K tail
 //    need no branches.
-//  * B given row-major [K, N] (int8 only) goes through registers instead: each lane loads an 8(k) x 4(n) byte
-//    block as 8 dwords, v_perm_b32 turns it into 4 K-contiguous 8-byte pieces, and they are written one
-//    iteration after they were loaded (two iterations of latency cover; the registers are double-buffered).
-//    The row written by store j of a lane is rotated by (n-block / 4) so the 64 lanes of a store spread over
-//    the LDS banks.
 //  * MX: the E8M0 scales arrive stage-major ([sK/SCB][rows][SCB], SCB = scale bytes per row per stage: ROWB / 16
 //    for fp4, ROWB / 32 for fp8), so a stage's scales for 1024 / SCB tile rows are one contiguous 1 KiB copy
 //    into the stage.
@@ -131,22 +126,6 @@ __device__ __forceinline__ void stage_barrier()
     __builtin_amdgcn_s_barrier();
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __builtin_amdgcn_sched_barrier(0);
-}
-
-__device__ __forceinline__ uint32_t perm_b32(uint32_t hi, uint32_t lo, uint32_t sel) { return __builtin_amdgcn_perm(hi, lo, sel); }
-
-// 4x4 byte transpose: in r[i] byte j = M[i][j]; out t[j] byte i = M[i][j]
-__device__ __forceinline__ void transpose4x4(uint32_t r0, uint32_t r1, uint32_t r2, uint32_t r3, uint32_t& t0,
-                                             uint32_t& t1, uint32_t& t2, uint32_t& t3)
-{
-    const uint32_t lo01 = perm_b32(r1, r0, 0x05010400u);  // r0.b0 r1.b0 r0.b1 r1.b1
-    const uint32_t hi01 = perm_b32(r1, r0, 0x07030602u);  // r0.b2 r1.b2 r0.b3 r1.b3
-    const uint32_t lo23 = perm_b32(r3, r2, 0x05010400u);
-    const uint32_t hi23 = perm_b32(r3, r2, 0x07030602u);
-    t0 = perm_b32(lo23, lo01, 0x05040100u);  // r0.b0 r1.b0 r2.b0 r3.b0
-    t1 = perm_b32(lo23, lo01, 0x07060302u);
-    t2 = perm_b32(hi23, hi01, 0x05040100u);
-    t3 = perm_b32(hi23, hi01, 0x07060302u);
 }
 
 // XCD-aware tile order: consecutive workgroup ids go to different XCDs; XCD x gets the ids [x*per, (x+1)*per)
@@ -264,20 +243,18 @@ struct GemmCore {
     static constexpr int SC_COPIES = (AUX_INSTR + NW - 1) / NW;
     static constexpr int SC_BYTES = SA_REG + SB_REG;
     static constexpr int COPIES = A_COPIES + B_COPIES + SC_COPIES;
-    static constexpr int B_BLK = (B_KCONTIG || B_TR) ? 0 : (ROWB / 8) * (BN / 4) / NT;  // 8x4-byte blocks per lane
-    static constexpr int B_LOADS = 8 * B_BLK;         // dword loads per lane per stage for a [K, N] B
     static constexpr int STAGE = (BM + BN) * ROWB + Q_REG + SC_BYTES;
     static constexpr int SC_OFF = (BM + BN) * ROWB + Q_REG;  // the scale regions within a stage
     static constexpr size_t LDS_BYTES = (size_t)STAGES * STAGE;
     // vmem operations of this wave issued after stage kt's copies, at the top of iteration kt
-    static constexpr int IN_FLIGHT = (STAGES - 2) * (COPIES + B_LOADS);
+    static constexpr int IN_FLIGHT = (STAGES - 2) * COPIES;
     // copies issued before each k-step of a stage (ILV false: all before the first)
     static constexpr int CPS = ILV ? (COPIES + KPS - 1) / KPS : COPIES;
     typedef typename std::conditional<OP == OP_I8, v16i, v16f>::type acc_t;
     static_assert(FM >= 1 && FN >= 1 && WTM % 32 == 0 && WTN % 32 == 0, "wave tile must be a multiple of 32");
     static_assert(BM % (ROWS_PER_COPY * NW) == 0 && A_COPIES >= 1, "A copies must split evenly over the waves");
     static_assert(!B_KCONTIG || (BN % (ROWS_PER_COPY * NW) == 0 && B_COPIES >= 1), "B copies");
-    static_assert(B_KCONTIG || B_TR || (((ROWB / 8) * (BN / 4)) % NT == 0 && B_BLK >= 1), "B blocks");
+    static_assert(B_KCONTIG || B_TR, "B rows of K, or K rows read by LDS transpose reads");
     static_assert(!B_TR || (!B_KCONTIG && (OP == OP_I8 || OP == OP_F8) && 1024 % BN == 0 && BN >= 32 && BN <= 256 &&
                             (ROWB * BN) % (1024 * NW) == 0 && B_COPIES >= 1), "B_TR copies");
     static_assert(!IS_MX || B_KCONTIG, "MX B must be K-contiguous");
@@ -289,7 +266,7 @@ struct GemmCore {
     static_assert(SC_DIRECT != 2 || 2 * PLANE_B <= SB_INSTR * 1024, "pair planes fit the B scale region");
     static_assert(!IS_FP6 || (ROWB == 64 && BM % 32 == 0 && BN % 32 == 0), "fp6 Q blocks: 4 MX blocks per stage");
     static_assert(KPS >= 1, "a stage holds at least one k-step");
-    static_assert((STAGES >= 3 || ((B_KCONTIG || B_TR) && STAGES == 2)) && IN_FLIGHT < 64, "stages");
+    static_assert(STAGES >= 2 && IN_FLIGHT < 64, "stages");
     static_assert(ROWB == 64 || ROWB == 128, "stage row");
     static_assert(LDS_BYTES <= 160 * 1024, "LDS");
 
@@ -406,49 +383,6 @@ struct GemmCore {
         const int lane = t & 63;
         const int wave = __builtin_amdgcn_readfirstlane(t >> 6);  // wave-uniform: copy bases stay scalar
         const int wm = wave / WN, wn = wave % WN;
-        typedef uint32_t breg_t[B_BLK > 0 ? B_BLK : 1][8];
-        breg_t rb0, rb1;  // two register sets, alternated by the 2x-unrolled main loop (no copies between them)
-
-        // [K, N] B: the 8x4-byte blocks of stage kt into rbt
-        auto load_b_regs = [&](breg_t& rbt, int64_t kt) {
-            if constexpr (!B_KCONTIG && !B_TR) {
-                const int64_t kb0 = kt * ROWB;
-#pragma unroll
-                for (int i = 0; i < B_BLK; ++i) {
-                    const int id = t + i * NT, nb = id % (BN / 4), kb = id / (BN / 4);
-#pragma unroll
-                    for (int r = 0; r < 8; ++r) {
-                        const int64_t k = kb0 + kb * 8 + r;
-                        const uint32_t off =
-                            (nb * 4 < p.cols && k < p.kbytes) ? p.b0 + (uint32_t)k * p.ldb + (uint32_t)(nb * 4) : OOB;
-                        rbt[i][r] = bload4(p.b, off);
-                    }
-                }
-            }
-        };
-        // transpose the blocks held in rb and write them K-contiguous into the B part of a slot
-        auto store_b_regs = [&](breg_t& rb, int slot) {
-            if constexpr (!B_KCONTIG && !B_TR) {
-                uint8_t* sB = smem + slot * STAGE + BM * ROWB;
-#pragma unroll
-                for (int i = 0; i < B_BLK; ++i) {
-                    const int id = t + i * NT, nb = id % (BN / 4), kb = id / (BN / 4);
-                    uint32_t lo[4], hi[4];
-                    transpose4x4(rb[i][0], rb[i][1], rb[i][2], rb[i][3], lo[0], lo[1], lo[2], lo[3]);
-                    transpose4x4(rb[i][4], rb[i][5], rb[i][6], rb[i][7], hi[0], hi[1], hi[2], hi[3]);
-                    const int rot = (nb >> 2) & 3;
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const int jj = (j + rot) & 3;
-                        const uint32_t l = jj == 0 ? lo[0] : jj == 1 ? lo[1] : jj == 2 ? lo[2] : lo[3];
-                        const uint32_t h = jj == 0 ? hi[0] : jj == 1 ? hi[1] : jj == 2 ? hi[2] : hi[3];
-                        const int n = nb * 4 + jj;
-                        *(u32x2*)(sB + n * ROWB + swz(n, kb >> 1) * 16 + (kb & 1) * 8) = (u32x2){l, h};
-                    }
-                }
-            }
-        };
-
         // MX auxiliary copies of this wave (A scales, B scales, then the fp6 Q blocks of A and of B): their source
         // (offset in p.aux at stage 0, stride per stage) and LDS offset within a stage depend on the wave only, so
         // they are worked out here, once.  The main loop then issues them with no branches: a branch there splits
@@ -567,29 +501,20 @@ struct GemmCore {
 #pragma unroll
         for (int j = 0; j < FN; ++j) troff[j] = B_TR ? tr_lane_off(wn * WTN + j * 32, lane) : 0u;
 
-        // prologue: stages 0 .. STAGES - 2 in flight; a [K, N] B is written for stages 0 .. STAGES - 3 and
-        // held in rb1 for stage STAGES - 2 (written at the end of iteration 0)
+        // prologue: stages 0 .. STAGES - 2 in flight
 #pragma unroll
         for (int s = 0; s < STAGES - 1; ++s) {
-            if (s < STAGES - 2) load_b_regs(rb0, s);
-            else load_b_regs(rb1, s);
-            __builtin_amdgcn_sched_barrier(0);
             issue_copies(s, s);
             __builtin_amdgcn_sched_barrier(0);
-            if (s < STAGES - 2) store_b_regs(rb0, s);
         }
 
-        // one iteration: stage kt is multiplied; the registers of stage kt + STAGES - 1 are loaded into rb_new and
-        // those of stage kt + STAGES - 2 (loaded one iteration ago into rb_old) are written to their slot
-        auto iteration = [&](int64_t kt, breg_t& rb_new, breg_t& rb_old) {
+        // one iteration: stage kt is multiplied, stage kt + STAGES - 1 requested
+        auto iteration = [&](int64_t kt) {
             const int slot = (int)(kt % STAGES);
             const int nslot = (int)((kt + STAGES - 1) % STAGES);
-            const int pslot = (int)((kt + STAGES - 2) % STAGES);
             __builtin_amdgcn_sched_barrier(0);  // the wait stays below the previous iteration's MFMAs
             wait_vmcnt<IN_FLIGHT>();            // this wave's copies of stage kt have landed
             stage_barrier();                    // ... and every wave's; the slot multiplied last iteration is free
-            load_b_regs(rb_new, kt + STAGES - 1);
-            __builtin_amdgcn_sched_barrier(0);
             const uint8_t* sA = smem + slot * STAGE;
             const uint8_t* sB = sA + BM * ROWB;
             // k-steps in pairs; a scheduling barrier between pairs keeps the fragment reads of a stage from
@@ -691,18 +616,13 @@ struct GemmCore {
                     }
                 }
             }
-            if constexpr (!B_KCONTIG && !B_TR) {
-                // rb_old's slot was freed two iterations ago and is next read after at least one more barrier
-                __builtin_amdgcn_sched_barrier(0);
-                store_b_regs(rb_old, pslot);
-            }
         };
         int64_t kt = 0;
         for (; kt + 1 < nk; kt += 2) {
-            iteration(kt, rb0, rb1);
-            iteration(kt + 1, rb1, rb0);
+            iteration(kt);
+            iteration(kt + 1);
         }
-        if (kt < nk) iteration(kt, rb0, rb1);
+        if (kt < nk) iteration(kt);
         // drain: no copy may still target LDS when the caller reuses it or the wave ends
         wait_vmcnt<0>();
     }

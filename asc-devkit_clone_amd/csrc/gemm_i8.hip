@@ -13,17 +13,10 @@
 //   (accompanying_quantization.md:79-103).
 #include "common.h"
 #include "gemm_core.h"
+#include "group_tile.h"
 #include "launch.h"
 
 namespace ascq {
-
-// a value every lane of the wave holds alike, moved to scalar registers
-__device__ __forceinline__ int64_t uniform64(int64_t v)
-{
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)((uint64_t)v >> 32));
-    return (int64_t)(((uint64_t)hi << 32) | lo);
-}
 
 // The int8 main loop of a tile: GemmCore (16-byte-aligned K-contiguous rows, K % 16 == 0), or GemmCoreUA (UA: any
 // alignment, any K; two stages of 64 bytes, a [K, N] B staged by K rows)
@@ -216,38 +209,6 @@ __global__ __launch_bounds__(PH == 2 ? (BM / 32) * (BN / 32) * 64 : WM * WN * 64
               [&](uint8_t x, uint32_t o) { __builtin_amdgcn_raw_buffer_store_b8(x, out.r, o, 0, 0); });
 }
 
-// QuantGroupMatmul: the m axis is split into G ragged groups (group_list), group g multiplies its rows by
-// W[g].  The real tiles are ordered group-major, then n-tile, then m-tile within the group, and the order is cut
-// into 8 contiguous ranges, one per XCD (workgroup ids go round-robin over the XCDs): an XCD then works on one
-// or two experts' column ranges, so its L2 holds the weight columns it streams instead of every XCD fetching
-// every expert's weights.  m-tiles never straddle a group.  The grid is sized for ceil(M / BM) + G m-tiles per
-// n-tile; ids past the real tile count exit at once.
-constexpr int GROUP_MAX = 1024;  // groups the tiled kernel takes (the host refuses more)
-
-// exclusive prefix sum over the workgroup of one value per thread (NT threads); *total gets the full sum
-template <int NT>
-__device__ __forceinline__ int64_t block_exclusive_scan(int64_t v, int64_t* wtot, int64_t* total)
-{
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    int64_t x = v;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int64_t y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
-    }
-    if (lane == 63) wtot[w] = x;
-    __syncthreads();
-    int64_t base = 0, tot = 0;
-#pragma unroll
-    for (int i = 0; i < NT / 64; ++i) {
-        if (i < w) base += wtot[i];
-        tot += wtot[i];
-    }
-    __syncthreads();  // wtot may be reused
-    *total = tot;
-    return base + x - v;
-}
-
 // WPE: waves per SIMD the register allocation must allow (2 for two 4-wave workgroups per CU)
 // UA: X and W of any alignment and any K (GemmCoreUA)
 // KW > 1 (one-wave tiles, few rows per group: decode-sized MoE batches): the workgroup's KW waves each run the tile's
@@ -263,74 +224,18 @@ __global__ __launch_bounds__(WM * WN * 64 * KW, WPE) void group_gemm_i8_kernel(G
     static_assert(KW == 1 || (WM == 1 && WN == 1 && !UA), "k-split waves run one-wave tiles");
     constexpr int NTT = T::NT * KW;  // threads of the workgroup
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    __shared__ int64_t wtot[NTT / 64];
-    __shared__ int64_t tile_info[4];  // group, first row, end row, first m-tile of this workgroup's tile
     // the tile's per-token (BM) and per-channel (BN) scales, copied global -> LDS by one wave-wide copy each
     // (1 KiB: lanes past the scales read zeros)
     static_assert(BM <= 256 && BN <= 256, "one 1 KiB copy per scale vector");
     __shared__ __attribute__((aligned(16))) float s_pt[256], s_sc[256];
-    const int G = (int)p.G;
-    const int64_t M = p.M;
-    // Group g's rows are [start_g, end_g) clamped to [0, M) (rows outside [0, M) exist in no group) and its
-    // m-tiles follow those of groups 0 .. g-1.  Thread t owns groups [t * per, (t + 1) * per): two block-wide
-    // prefix sums (rows, then m-tiles) give every thread its groups' starts, and the thread owning this
-    // workgroup's tile publishes it -- no G-sized table, so the LDS stays with the stage ring.
-    const int per = (G + NTT - 1) / NTT, ga = (int)threadIdx.x * per;
-    auto count = [&](int g) {
-        const int64_t c = p.list_type == 0 ? p.group_list[g + 1] - p.group_list[g] : p.group_list[g];
-        return c < 0 ? (int64_t)0 : c;
-    };
-    auto clampM = [&](int64_t v) { return v < 0 ? (int64_t)0 : (v > M ? M : v); };
-    const int64_t base = p.list_type == 0 ? p.group_list[0] : 0;
-    int64_t rows_total, tiles_total, mine = 0;
-    for (int k = 0; k < per; ++k)
-        if (ga + k < G) mine += count(ga + k);
-    const int64_t s0 = base + block_exclusive_scan<NTT>(mine, wtot, &rows_total);
-    mine = 0;
-    {
-        int64_t st = s0;
-        for (int k = 0; k < per; ++k)
-            if (ga + k < G) {
-                const int64_t c = count(ga + k);
-                mine += (clampM(st + c) - clampM(st) + BM - 1) / BM;
-                st += c;
-            }
-    }
-    const int64_t tiles_n = (p.N + BN - 1) / BN;
-    const int64_t t0 = block_exclusive_scan<NTT>(mine, wtot, &tiles_total);
-    const int64_t total = tiles_total * tiles_n;  // real (m-tile, n-tile) pairs
-    const int64_t per_xcd = (total + 7) / 8;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wm = KW > 1 ? 0 : wave / WN, wn = KW > 1 ? 0 : wave % WN;
     const int kw = KW > 1 ? __builtin_amdgcn_readfirstlane(wave) : 0;
+    GroupTile tile;
+    if (!find_group_tile<NTT, BM, BN>(p, tile)) return;
     {
-        const int64_t lin = (int64_t)(blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-        if ((int64_t)(blockIdx.x / 8) >= per_xcd || lin >= total) return;
-        int64_t st = s0, tf = t0;
-        for (int k = 0; k < per; ++k)
-            if (ga + k < G) {
-                const int64_t c = count(ga + k), a0 = clampM(st), a1 = clampM(st + c);
-                const int64_t nt = (a1 - a0 + BM - 1) / BM;
-                if (nt > 0 && tf * tiles_n <= lin && lin < (tf + nt) * tiles_n) {
-                    tile_info[0] = ga + k;
-                    tile_info[1] = a0;
-                    tile_info[2] = a1;
-                    tile_info[3] = tf;
-                }
-                st += c;
-                tf += nt;
-            }
-        __syncthreads();
-        // every lane reads the same values; readfirstlane keeps them (and the buffer resources built from them)
-        // in scalar registers -- a resource in VGPRs costs a waterfall loop around every access
-        const int g = __builtin_amdgcn_readfirstlane((int)tile_info[0]);
-        const int64_t g_first = uniform64(tile_info[1]), m_end = uniform64(tile_info[2]);
-        const int64_t g_tile0 = uniform64(tile_info[3]);
-        const int64_t mt_g = (m_end - g_first + BM - 1) / BM;  // m-tiles of group g (>= 1 here)
-        const int64_t rem = lin - g_tile0 * tiles_n;
-        const int tn = __builtin_amdgcn_readfirstlane((int)(rem / mt_g));
-        const int64_t m0 = uniform64(g_first + (rem % mt_g) * BM);
-        const int64_t n0 = (int64_t)tn * BN;
+        const int g = tile.g;
+        const int64_t m0 = tile.m0, n0 = tile.n0, m_end = tile.m_end;
         CoreArgs c{};
         uint32_t da = 0, db = 0;  // UA: the operands' offsets from their resources' 16-byte-aligned bases
         if constexpr (UA) {
@@ -672,23 +577,7 @@ hipError_t launch_group_gemm(const GroupGemmArgs& a, hipStream_t st)
             return a.M >= 8 * a.G ? launch_group_tiled<32, 64, 1, 1, 4, false, 64, 1, true, false, 4>(a, st)
                                   : launch_group_tiled<32, 32, 1, 1, 4, false, 64, 1, true, false, 4>(a, st);
     }
-    {
-        // 128 x 256 tiles.  Short K (the reference sample's K = 1024): 4 waves with 64 x 128 wave tiles and
-        // 64-byte stages, two workgroups per CU, so one's epilogue and its store / load latencies overlap the
-        // other's MFMAs (measured 110-120 us against 145-150 us for one 8-wave workgroup per CU).  Long K (the
-        // MoE shape, 4096 tokens, 16 experts, K = 4096, N = 1408: ~250 tiles, one per CU): 8 waves, 128-byte
-        // stages (16 MFMAs per wave per barrier), three stages keep two in flight.
-        if (a.w_trans && a.K <= 2048) return launch_group_tiled<128, 256, 2, 2, 3, true, 64, 2>(a, st);
-        if (a.w_trans && a.K % 128 == 0) return launch_group_tiled<128, 256, 2, 4, 3, true, 128>(a, st);
-        if (a.w_trans) return launch_group_tiled<128, 256, 2, 4, 6, true>(a, st);
-        // W [G, K, N] with 16-byte K rows: the same tiles, K rows copied like A's and read by LDS transpose reads
-        // (the 4-wave, two-workgroups-per-CU form of the short-K case spills here: 8 waves for every K)
-        if (a.N % 16 == 0 && (uintptr_t)a.W % 16 == 0) {
-            if (a.K % 128 == 0) return launch_group_tiled<128, 256, 2, 4, 3, false, 128, 1, true>(a, st);
-            return launch_group_tiled<128, 256, 2, 4, 6, false, 64, 1, true>(a, st);
-        }
-        return launch_group_tiled<128, 128, 2, 2, 4, false>(a, st);
-    }
+    return launch_group_pipe(a, st);
 }
 
 }  // namespace ascq

@@ -226,16 +226,14 @@ struct GemmPipe {
         // lane offsets of the fragment reads: 16-byte chunk 4 c + g of the lane's row (within a half, wave row 0); BTR: the
         // lane's 8-byte piece of fragment column j
         constexpr int FA = fmh(0) > fmh(1) ? fmh(0) : fmh(1), FB = fnh(0) > fnh(1) ? fnh(0) : fnh(1);
-        uint32_t rl[2], rt[2][FB];
+        uint32_t rl[2], rt[2];
 #pragma unroll
         for (int c = 0; c < 2; ++c) rl[c] = (uint32_t)(r16 * ROWB + (((4 * c + g) ^ ((r16 >> 1) & 7)) * 16));
         if constexpr (BTR) {
             const int k = 16 * g + (r16 >> 1);
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int j = 0; j < fnh(h); ++j)
-                    rt[h][j] = (uint32_t)(k * hn(h) + ((wn * fnh(h) + j) ^ swz_tr(h, k)) * 16 + (r16 & 1) * 8);
+            for (int h = 0; h < 2; ++h)  // of fragment column 0; column j's chunk differs by an XOR (fnh is a power of two)
+                rt[h] = (uint32_t)(k * hn(h) + ((wn * fnh(h)) ^ swz_tr(h, k)) * 16 + (r16 & 1) * 8);
         }
         const uint32_t wa[2] = {(uint32_t)(wm * whm(0) * ROWB), (uint32_t)((hm(0) + wm * whm(1)) * ROWB)};
         const uint32_t wb[2] = {(uint32_t)(wn * whn(0) * ROWB), (uint32_t)((hn(0) + wn * whn(1)) * ROWB)};
@@ -276,10 +274,10 @@ struct GemmPipe {
                 for (int s = 0; s < KPS; ++s) fa[h][i][s] = read_frag(sA + slot * (BM * ROWB) + i * 16 * ROWB, off, s);
         };
         typedef int v2i_t __attribute__((ext_vector_type(2)));
-        auto read_tr = [&](const uint8_t* base, int h, int j, int s) -> v4i {  // K rows 64 s + 16 g .. + 15
+        auto read_tr = [&](const uint8_t* base, int h, uint32_t off, int s) -> v4i {  // K rows 64 s + 16 g .. + 15
             typedef __attribute__((address_space(3))) v2i_t* lp;
-            const v2i_t x = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lp)(base + rt[h][j] + s * 64 * hn(h)));
-            const v2i_t y = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lp)(base + rt[h][j] + (s * 64 + 8) * hn(h)));
+            const v2i_t x = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lp)(base + off + s * 64 * hn(h)));
+            const v2i_t y = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lp)(base + off + (s * 64 + 8) * hn(h)));
             return (v4i){x[0], x[1], y[0], y[1]};
         };
         auto read_b = [&](auto HH, int set, int slot, int kt) {
@@ -292,21 +290,28 @@ struct GemmPipe {
                     swb[set][j / 2][j % 2] = read_scale(kt, SCA * 128 + h * hn(0) + wn * whn(h) + j * 16);
             }
 #pragma unroll
-            for (int j = 0; j < fnh(h); ++j)
+            for (int j = 0; j < fnh(h); ++j) {
+                uint32_t tr = 0;
+                if constexpr (BTR) {
+                    uint32_t x = (uint32_t)j * 16u;
+                    asm volatile("" : "+s"(x));  // (as in `at`)
+                    tr = (rt[h] ^ x) + A_REG;
+                }
 #pragma unroll
                 for (int s = 0; s < KPS; ++s) {
                     if constexpr (BTR) {
-                        const uint8_t* base = sB + slot * (BN * ROWB) + h * hn(0) * ROWB;
+                        const uint8_t* base = sA + slot * (BN * ROWB) + h * hn(0) * ROWB;
                         if constexpr (IS_F8) {
-                            const v4i x = read_tr(base, h, j, 0), y = read_tr(base, h, j, 1);
+                            const v4i x = read_tr(base, h, tr, 0), y = read_tr(base, h, tr, 1);
                             fb[set][j][s] = (v8i){x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
                         } else {
-                            fb[set][j][s] = read_tr(base, h, j, s);
+                            fb[set][j][s] = read_tr(base, h, tr, s);
                         }
                     } else {
                         fb[set][j][s] = read_frag(sA + slot * (BN * ROWB) + j * 16 * ROWB, off, s);
                     }
                 }
+            }
         };
         // MFMAs x0 .. x1 - 1 (k-step, then B fragment, then A fragment) of the quadrant (A half HA, B half HB held in
         // register set `set`)
@@ -437,7 +442,8 @@ struct GemmPipe {
 // 25.6 (128 x 256), 27.8 (128 x 128), 30.2 (64 x 128); M = 256 128 x 128 in 16.6 against 20.3 (128 x 192), 20.6
 // (64 x 128); M = 128 64 x 128 in 12.5 against 16.0 (128 x 128).
 enum PipeTile { PIPE_256x256, PIPE_192x256, PIPE_256x192, PIPE_128x256, PIPE_128x192, PIPE_128x128, PIPE_64x128, PIPE_TILES };
-inline PipeTile pick_pipe_tile(int64_t M, int64_t N, int64_t kbytes)
+// groups: of a group matmul, whose M rows fall into groups of sizes the host does not know: half a row tile more each.
+inline PipeTile pick_pipe_tile(int64_t M, int64_t N, int64_t kbytes, int64_t groups = 0)
 {
     static const struct {
         int bm, bn;
@@ -449,7 +455,7 @@ inline PipeTile pick_pipe_tile(int64_t M, int64_t N, int64_t kbytes)
     PipeTile best = PIPE_256x256;
     float least = 0.0f;
     for (int t = 0; t < PIPE_TILES; ++t) {
-        const int64_t tiles = ((M + T[t].bm - 1) / T[t].bm) * ((N + T[t].bn - 1) / T[t].bn);
+        const int64_t tiles = ((M + T[t].bm - 1) / T[t].bm + groups / 2) * ((N + T[t].bn - 1) / T[t].bn);
         const float c = (float)((tiles + 255) / 256), fill = (float)tiles / (256.0f * c);
         const float cost = c * ((T[t].solo + (T[t].full - T[t].solo) * fill) * stages + T[t].tail * fill);
         if (t == 0 || cost < least) {
@@ -481,8 +487,8 @@ __device__ __forceinline__ void pipe_tile(int pid, int tiles_m, int tiles_n, int
 // j + 1's, after which a lane owns eight consecutive columns -- 8 (g / 2) .. of fragment j + g % 2: one 16-byte
 // (2-byte elements), 8-byte (1-byte) or 4-byte (int4 codes, ES 0) store where there were eight of one element.  4-byte
 // elements leave as they are, one 16-byte store per fragment.
-// cols4(tile column) gives the parameters of four columns; conv(accumulator, parameters, e) the element's bits, or, for
-// the 2-byte types (OUT_F16, OUT_BF16), its fp32 value, which is converted here two at a time.
+// cols4(tile column) gives the parameters of four columns; conv(accumulator, parameters, e[, tile row]) the element's
+// bits, or, for the 2-byte types (OUT_F16, OUT_BF16), its fp32 value, which is converted here two at a time.
 // vec: the output's base and row pitch are multiples of four bytes; otherwise, and in runs that cross the tile's last
 // column, elements are stored one by one.
 enum { OUT_I4 = 0, OUT_1 = 1, OUT_F16 = 2, OUT_BF16 = 3, OUT_4 = 4 };
@@ -491,6 +497,10 @@ __device__ __forceinline__ void ct_store(const TileOut& out, bool vec, int cols,
                                          int wm, int wn, int lane, Cols cols4, Conv conv)
 {
     constexpr bool HALF = OUT == OUT_F16 || OUT == OUT_BF16;
+    auto call = [&](auto a, const auto& par, int e, int row) {
+        if constexpr (std::is_invocable_v<Conv, decltype(a), decltype(par), int, int>) return conv(a, par, e, row);
+        else return conv(a, par, e);
+    };
     const int g = lane >> 4;
 #pragma unroll
     for (int j = 0; j < T::FN; j += 2) {
@@ -498,14 +508,15 @@ __device__ __forceinline__ void ct_store(const TileOut& out, bool vec, int cols,
         const auto p0 = cols4(c0), p1 = cols4(c1);
 #pragma unroll
         for (int i = 0; i < T::FM; ++i) {
-            const uint32_t roff = (uint32_t)T::ct_row(wm, i, lane) * out.pitch;
+            const int row = T::ct_row(wm, i, lane);
+            const uint32_t roff = (uint32_t)row * out.pitch;
             const int c = T::block_col(wn, j + (g & 1)) + 8 * (g >> 1);  // this lane's eight columns after the swap
             if constexpr (OUT == OUT_4) {
 #pragma unroll
                 for (int q = 0; q < 2; ++q) {
                     uint32_t x[4];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) x[e] = conv(acc[i][j + q][e], q ? p1 : p0, e);
+                    for (int e = 0; e < 4; ++e) x[e] = call(acc[i][j + q][e], q ? p1 : p0, e, row);
                     const int cq = q ? c1 : c0;
                     if (cq + 4 <= cols) {
                         __builtin_amdgcn_raw_buffer_store_b128((u32x4){x[0], x[1], x[2], x[3]}, out.r,
@@ -525,8 +536,8 @@ __device__ __forceinline__ void ct_store(const TileOut& out, bool vec, int cols,
                     float v[8];
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        v[e] = conv(acc[i][j][e], p0, e);
-                        v[4 + e] = conv(acc[i][j + 1][e], p1, e);
+                        v[e] = call(acc[i][j][e], p0, e, row);
+                        v[4 + e] = call(acc[i][j + 1][e], p1, e, row);
                     }
                     us2_t top = {0, 0};
                     lo[0] = cvt_pair<OUT == OUT_BF16>(v[0], v[1], top);
@@ -552,8 +563,8 @@ __device__ __forceinline__ void ct_store(const TileOut& out, bool vec, int cols,
                     lo[0] = hi[0] = 0u;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        lo[0] |= (conv(acc[i][j][e], p0, e) & MASK) << (SH * e);
-                        hi[0] |= (conv(acc[i][j + 1][e], p1, e) & MASK) << (SH * e);
+                        lo[0] |= (call(acc[i][j][e], p0, e, row) & MASK) << (SH * e);
+                        hi[0] |= (call(acc[i][j + 1][e], p1, e, row) & MASK) << (SH * e);
                     }
                     const auto sw = __builtin_amdgcn_permlane16_swap(lo[0], hi[0], false, false);
                     if constexpr (OUT == OUT_I4) {

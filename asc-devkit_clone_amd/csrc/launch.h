@@ -162,6 +162,9 @@ struct GroupGemmArgs {
     int act;                  // 0 none, 1 FasterGelu
 };
 hipError_t launch_group_gemm(const GroupGemmArgs& a, hipStream_t st);
+// gemm_pipe_group.hip: X with 16-byte-aligned rows, W [G, N, K] the same or [G, K, N] with 4-byte-aligned rows, K % 16
+// == 0, at most 1024 groups, operands below 2^31 bytes
+hipError_t launch_group_pipe(const GroupGemmArgs& a, hipStream_t st);
 
 // gemv_antiquant.hip
 size_t weight_pack_bytes(int w_type, int64_t K, int64_t N);
