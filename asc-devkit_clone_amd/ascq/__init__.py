@@ -39,6 +39,10 @@ FORMAT_ND, FORMAT_PACKED, FORMAT_NZ = 0, 1, 2
 
 OK, E_INVALID_ARG, E_UNSUPPORTED, E_HIP, E_STATE = 0, -1, -2, -3, -4
 
+# torch dtype -> ascq_dtype of floating sources, scales and outputs
+_FLOAT_CODE = {torch.float16: F16, torch.bfloat16: BF16, torch.float32: F32}
+_SRC_CODE = {torch.int32: INT32, torch.float32: F32, torch.int8: INT8}
+
 _TORCH_OF = {INT8: torch.int8, INT32: torch.int32, F16: torch.float16, BF16: torch.bfloat16, F32: torch.float32}
 
 
@@ -186,17 +190,28 @@ def check(status: int, what: str) -> None:
 
 
 def _ptr(t) -> int | None:
-    if t is None:
-        return None
-    if isinstance(t, int):
+    if t is None or isinstance(t, int):
         return t
     return t.data_ptr()
 
 
+# The current stream's handle.  torch.cuda.current_stream() builds a Stream object around it, 2.5 us of the 6.7 us that a
+# small call took; the binding it is built from returns the handle itself in 0.14 us.  The first call goes the public
+# way (which also initialises the device).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", None)
+_stream_ready = False
+
+
 def _stream(stream) -> int | None:
-    if stream is not None:
-        return stream if isinstance(stream, int) else stream.cuda_stream
-    return torch.cuda.current_stream().cuda_stream
+    global _stream_ready
+    if stream is None:
+        if _stream_ready:
+            return _raw_stream(_current_device())
+        handle = torch.cuda.current_stream().cuda_stream
+        _stream_ready = _raw_stream is not None and _current_device is not None
+        return handle
+    return stream if isinstance(stream, int) else stream.cuda_stream
 
 
 def _half_bits(v: float) -> int:
@@ -213,7 +228,7 @@ def pack_quant_pre(m1: float, offset9: int = 0, sign: int = 0) -> int:
 def quant_dynamic_per_token(x: torch.Tensor, round_mode: int = ROUND_RINT, out=None, scale_out=None, stream=None):
     """Per-row absmax -> int8 q and fp32 scale (= absmax/127).  x: [m, n] f16 / bf16 / f32."""
     m, n = x.shape
-    src_type = {torch.float16: F16, torch.bfloat16: BF16, torch.float32: F32}[x.dtype]
+    src_type = _FLOAT_CODE[x.dtype]
     q = out if out is not None else torch.empty((m, n), dtype=torch.int8, device=x.device)
     s = scale_out if scale_out is not None else torch.empty((m,), dtype=torch.float32, device=x.device)
     check(lib().ascq_ascend_quant_dynamic_per_token(_ptr(q), _ptr(s), _ptr(x), src_type, m, n, round_mode,
@@ -225,7 +240,7 @@ def quant_per_token(x: torch.Tensor, scale: torch.Tensor, offset=None, round_mod
                     stream=None):
     """AscendQuant PER_TOKEN: q = sat_s8(round(f32(x) * scale[row] (+ offset[row])))."""
     m, n = x.shape
-    src_type = {torch.float16: F16, torch.bfloat16: BF16, torch.float32: F32}[x.dtype]
+    src_type = _FLOAT_CODE[x.dtype]
     q = out if out is not None else torch.empty((m, n), dtype=torch.int8, device=x.device)
     p = _QuantParam(m, n, m * n, 0, 1 if offset is not None else 0, 1, round_mode)
     check(lib().ascq_ascend_quant_per_token(_ptr(q), _ptr(x), src_type, _ptr(scale), _ptr(offset), ctypes.byref(p),
@@ -240,9 +255,9 @@ def ascend_quant_policy(x: torch.Tensor, scale: torch.Tensor, policy: int, dst_t
     returned as uint8 codes) or fp4 E2M1 / E1M2 (two codes a byte, [m, n/2] uint8).  scale / offset f16 / bf16 / f32; a
     scalar offset_scalar applies when no offset tensor is given."""
     m, n = x.shape
-    src_type = {torch.float16: F16, torch.bfloat16: BF16, torch.float32: F32}[x.dtype]
+    src_type = _FLOAT_CODE[x.dtype]
     if scale_type is None:
-        scale_type = {torch.float16: F16, torch.bfloat16: BF16, torch.float32: F32}[scale.dtype]
+        scale_type = _FLOAT_CODE[scale.dtype]
     if out is not None:
         q = out
     elif dst_type in (FP4_E2M1, FP4_E1M2):
@@ -262,7 +277,7 @@ def ascend_quant(x: torch.Tensor, dst_type: int = INT8, scale=None, offset=None,
     """Legacy AscendQuant (arch-3510 form): per tensor (float scalars) or per channel (scale / offset tensors of the
     source's type; offset None takes offset_scalar as a source-typed value).  dst INT8 / HIF8 (half arithmetic) or
     FP8_E4M3 / FP8_E5M2 (fp32 arithmetic); returns int8 (INT8) or uint8 codes of x's shape."""
-    src_type = {torch.float16: F16, torch.bfloat16: BF16, torch.float32: F32}[x.dtype]
+    src_type = _FLOAT_CODE[x.dtype]
     q = out if out is not None else torch.empty(x.shape, dtype=torch.int8 if dst_type == INT8 else torch.uint8,
                                                 device=x.device)
     if scale is not None:
@@ -273,7 +288,7 @@ def ascend_quant(x: torch.Tensor, dst_type: int = INT8, scale=None, offset=None,
 
 
 def _dtype_code(t) -> int:
-    return {torch.float16: F16, torch.bfloat16: BF16, torch.float32: F32}[t]
+    return _FLOAT_CODE[t]
 
 
 def dequant_dst_shape(dst_dtype, m: int, n: int, cal_count: int, mode: int = DEQUANT_SINGLE_ROW):
@@ -313,8 +328,8 @@ def ascend_dequant_policy(src: torch.Tensor, scale: torch.Tensor, policy: int, d
     groupSize}): PER_TOKEN (scale[row]) or PER_GROUP (kdim 1: scale[row][col / g]; kdim 0: scale[row / g][col])
     on src [rows, n] int32 / f32 (or int8); scale f32 / f16 / bf16."""
     m, n = src.shape
-    src_type = {torch.int32: INT32, torch.float32: F32, torch.int8: INT8}[src.dtype]
-    scale_type = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}[scale.dtype]
+    src_type = _SRC_CODE[src.dtype]
+    scale_type = _FLOAT_CODE[scale.dtype]
     y = out if out is not None else torch.empty((m, n), dtype=dst_dtype, device=src.device)
     p = _DequantPolicyParam(m, n, m * n if cal_count is None else cal_count, group_size, int(offset is not None), kdim)
     check(lib().ascq_ascend_dequant_policy(_ptr(y), _dtype_code(dst_dtype), _ptr(src), src_type, _ptr(scale),
@@ -352,7 +367,7 @@ def ascend_antiquant_policy(src: torch.Tensor, src_type: int, scale: torch.Tenso
                             is_transpose: bool = False, dst_dtype=torch.float16, out=None, stream=None):
     """AscendAntiQuant policy form (PER_TOKEN / PER_GROUP) over [m, n]: int8 / fp8 sources with f16 / bf16 / f32
     scales, fp4 E2M1 / E1M2 sources with E8M0 group scales.  Returns [m, n] of dst_dtype."""
-    dst_type = {torch.float16: F16, torch.bfloat16: BF16, torch.float32: F32}[dst_dtype]
+    dst_type = _FLOAT_CODE[dst_dtype]
     y = out if out is not None else torch.empty((m, n), dtype=dst_dtype, device=src.device)
     check(lib().ascq_ascend_antiquant_policy(_ptr(y), dst_type, _ptr(src), src_type, _ptr(scale), _ptr(offset),
                                              scale_type, policy, m, n, group_size, k_dim, int(is_transpose),
@@ -363,9 +378,6 @@ def ascend_antiquant_policy(src: torch.Tensor, src_type: int, scale: torch.Tenso
 # ------------------------------------------------------------------------------------------
 # Quantize / Dequantize / AntiQuantize (quantize.h / dequantize.h / antiquantize.h)
 # ------------------------------------------------------------------------------------------
-_FLOAT_CODE = {torch.float16: F16, torch.bfloat16: BF16, torch.float32: F32}
-
-
 def quantize(x: torch.Tensor, policy: int, dst_type: int = INT8, scale=None, offset=None, scale_scalar: float = 1.0,
              offset_scalar=None, scale_type: int | None = None, group_size: int = 0, kdim: int = 1,
              round_mode: int = ROUND_RINT, out=None, stream=None):

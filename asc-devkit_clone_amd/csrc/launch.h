@@ -53,8 +53,12 @@ inline void launch_k(F kernel, dim3 grid, dim3 block, uint32_t shm, hipStream_t 
 {
     LaunchEvents& e = launch_events();
     const hipEvent_t a = e.start, b = e.stop;
+    if (!a && !b) {
+        hipLaunchKernelGGL(kernel, grid, block, shm, st, args...);  // callers check hipGetLastError()
+        return;
+    }
     e = LaunchEvents{};
-    hipExtLaunchKernelGGL(kernel, grid, block, shm, st, a, b, 0u, args...);  // callers check hipGetLastError()
+    hipExtLaunchKernelGGL(kernel, grid, block, shm, st, a, b, 0u, args...);
 }
 
 // quant.hip
