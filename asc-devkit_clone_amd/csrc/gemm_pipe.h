@@ -36,8 +36,17 @@
 // its eight, and each stage's go to one of four scale slots, requested three stages ahead, one copy per wave and stage;
 // a lane reads the two bytes of block g of its row and the MFMA's op_sel picks the k-step's.
 // K is a multiple of 16 bytes: a lane's chunks at or past the end of K are not read (zeros), nor are a [K, N] B's rows.
+//
+// Weight-only antiquant (OP_AQ): A is f16 (a stage is 64 k), B the packed int4 / int8 weight.  A wave loads one 16-column
+// strip of a half per stage into registers (packed codes, the columns' scale and offset), six phases ahead, dequantises
+// one fragment per phase under its MFMAs and writes it to the half's rows in LDS at the top of the next phase, so each
+// weight is dequantised once per tile.  B0(k + 1) is written in phases 0 and 1 of stage k, B1(k + 1) in phases 2 and 3:
+// after the reads of B0(k) and B1(k), so B's ring is one stage.  (Two stages' codes per load, eight phases ahead, measured
+// the same to 5 % slower; copies of the kernel without the weight loads took 15 - 20 % less, without the dequantisation
+// the same time.)
 #pragma once
 
+#include "aq_frag.h"
 #include "gemm_core.h"
 
 namespace ascq {
@@ -76,13 +85,24 @@ struct PipeArgs {
     // first row in stage 0, and the stage strides
     rsrc4_t aux;
     uint32_t sa_off, sa_stride, sb_off, sb_stride;
+    // OP_AQ: the packed weight (kbytes / 256 tiles per 16-column strip), the group rows of scale and offset [K / g][n],
+    // g = 64 << gshift, and the tile's first column
+    const uint8_t* wp;
+    const uint16_t *scale, *offset;
+    uint32_t w_bytes, s_bytes, n, n0, gshift;
 };
+
+// B operand of the weight-only antiquant pipeline; FMT bit 0: int4 codes (else int8), bit 1: with offsets
+constexpr int OP_AQ = 16;
 
 template <int BM, int BN, int WM, int WN, int ST, int OP, int FMT = 0, bool BTR = false>
 struct GemmPipe {
     static constexpr bool IS_F8 = OP == OP_F8;
     static constexpr bool IS_MX = OP == OP_MXFP4;
-    static_assert(OP == OP_I8 || OP == OP_F8 || (IS_MX && !BTR), "int8, fp8, or MX-FP4 with a K-contiguous B");
+    static constexpr bool IS_AQ = OP == OP_AQ;
+    static_assert(OP == OP_I8 || OP == OP_F8 || ((IS_MX || IS_AQ) && !BTR),
+                  "int8, fp8, MX-FP4 with a K-contiguous B, or f16 with a packed weight");
+    static_assert(!IS_AQ || ST == 2, "weight registers by stage parity");
     static constexpr int CBSZ = IS_MX ? F8F6F4_E2M1 : FMT & 7;  // f8f6f4 formats of A and B
     static constexpr int BLGP = IS_MX ? F8F6F4_E2M1 : (FMT >> 3) & 7;
     static constexpr int TBM = BM, TBN = BN, TWN = WN;
@@ -100,7 +120,8 @@ struct GemmPipe {
     static constexpr int FM = fmh(0) + fmh(1), FN = fnh(0) + fnh(1);
     static constexpr int ca(int h) { return hm(h) / 8 / NW; }  // 1 KiB copies per wave of an A / B half
     static constexpr int cb(int h) { return hn(h) / 8 / NW; }
-    static constexpr int A_REG = ST * BM * ROWB, B_REG = ST * BN * ROWB;
+    static constexpr int A_REG = ST * BM * ROWB, B_REG = (IS_AQ ? 1 : ST) * BN * ROWB;
+    static_assert(!IS_AQ || (cb(0) <= 2 && cb(1) <= 2), "a wave dequantises columns of one strip per half");
     static constexpr int SCA = IS_MX ? (BM * 8 + 1023) / 1024 : 0, SCB = IS_MX ? (BN * 8 + 1023) / 1024 : 0;  // scale copies
     static constexpr int SC_SLOT = (SCA + SCB) * 1024;
     static constexpr size_t LDS_BYTES = (size_t)A_REG + B_REG + 4 * SC_SLOT;
@@ -118,9 +139,15 @@ struct GemmPipe {
 
     // copies of half H(i)
     static constexpr int half_copies(int i) { return i % 4 == 0 ? ca(0) : i % 4 == 1 ? cb(0) : i % 4 == 2 ? cb(1) : ca(1); }
-    // copies a wave may have outstanding at the barrier in front of phase p: H(t + 3) .. H(t + 4 ST)
+    // OP_AQ: loads of a weight half into registers
+    static constexpr int WLOADS = FMT & 2 ? 3 : 2;
+    // copies a wave may have outstanding at the barrier in front of phase p: H(t + 3) .. H(t + 4 ST).  OP_AQ: phase 1 loads
+    // B0 three stages ahead, phase 2 requests A1 two ahead, phase 3 loads B1 and requests A0 three ahead; phase 1 reads
+    // A1 (after its copies came B1, A0, B0, A1, B1, A0), phase 2 A0 (B0, A1, B1, A0, B0), phases 0 and 3 what ds_writes
+    // put there
     static constexpr int outstanding(int p)
     {
+        if (IS_AQ) return p == 1 ? 2 * ca(0) + ca(1) + 3 * WLOADS : p == 2 ? ca(0) + ca(1) + 3 * WLOADS : 63;
         int n = 0;
         for (int i = p + 3; i <= p + 4 * ST; ++i) n += half_copies(i);
         if (IS_MX)  // ... and the scale copies of the phases 2 among the 4 ST - 2 before
@@ -196,6 +223,7 @@ struct GemmPipe {
             const uint32_t dst = isa ? lA + slot * (BM * ROWB) + h * hm(0) * ROWB : lB + slot * (BN * ROWB) + h * hn(0) * ROWB;
             uint32_t v = isa ? va : vb[h], s = (uint32_t)kt * ROWB;
             if constexpr (BTR && !isa) s = kt < nk ? s * p.ldb : OOB;
+            else if constexpr (IS_AQ) s = kt < nk ? s : OOB;  // (whole stages)
             else v += kt * ROWB + kchunk < p.kbytes ? 0u : OOB;
 #pragma unroll
             for (int u = 0; u < (isa ? ca(h) : cb(h)); ++u) {
@@ -223,6 +251,50 @@ struct GemmPipe {
                 dma16(p.aux, sc_dst + (uint32_t)(kt & 3) * SC_SLOT, sc_off + (kt < nk ? (uint32_t)kt * sc_stride : OOB));
         };
 
+        // OP_AQ: this wave's strip of half h and the lane's offsets into the packed weight and the group rows
+        struct WeightRegs {
+            uint32_t w[2][2];  // [fragment][code words]
+            uint32_t sc, of;
+        };
+        constexpr bool I4 = FMT & 1, HAS_OFF = (FMT & 2) != 0;
+        constexpr int CW = I4 ? 1 : 2;  // code words per fragment
+        [[maybe_unused]] WeightRegs wr[2][2];  // [stage parity][half]
+        uint32_t w_at[2] = {}, s_at[2] = {}, magic = 0;
+        const rsrc_t r_w = make_rsrc(p.wp, p.w_bytes), r_s = make_rsrc(p.scale, p.s_bytes),
+                     r_o = make_rsrc(HAS_OFF ? p.offset : p.scale, p.s_bytes);
+        if constexpr (IS_AQ) {
+            magic = half_magic_vgpr();
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {  // two fragments of a stage (32 k each) per wave, or one
+                const uint32_t col = p.n0 + (uint32_t)(h * hn(0)) + (cb(h) == 2 ? wave : wave >> 1) * 16u;
+                const bool ok = col < p.n;
+                w_at[h] = ok ? col / 16u * (uint32_t)(p.kbytes / 256) * (CW * 1024u) + lane * (CW * 16u) +
+                                   (cb(h) == 2 ? 0 : wave & 1) * (CW * 4u)
+                             : OOB;
+                s_at[h] = ok ? (col + r16) * 2u : OOB;
+            }
+        }
+        auto load_w = [&](auto HH, auto PAR, int kt) {
+            constexpr int h = decltype(HH)::value, par = decltype(PAR)::value & 1;
+            WeightRegs& r = wr[par][h];
+            const uint32_t k = (uint32_t)(kt < nk ? kt : nk - 1);  // (stages past the last: read, never multiplied)
+            const uint32_t off = w_at[h] + par * (CW * 8u);
+            const int soff = (int)((k >> 1) * (CW * 1024u));
+            if constexpr (cb(h) * CW == 4) {
+                const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r_w, off, soff, 0);
+                r.w[0][0] = v[0], r.w[0][1] = v[1], r.w[1][0] = v[2], r.w[1][1] = v[3];
+            } else if constexpr (cb(h) * CW == 2) {
+                const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r_w, off, soff, 0);
+                r.w[0][0] = v[0];
+                r.w[I4 ? 1 : 0][I4 ? 0 : 1] = v[1];
+            } else {
+                r.w[0][0] = __builtin_amdgcn_raw_buffer_load_b32(r_w, off, soff, 0);
+            }
+            const int grow = (int)((k >> p.gshift) * p.n * 2u);
+            r.sc = __builtin_amdgcn_raw_buffer_load_b16(r_s, s_at[h], grow, 0);
+            if constexpr (HAS_OFF) r.of = __builtin_amdgcn_raw_buffer_load_b16(r_o, s_at[h], grow, 0);
+        };
+
         // lane offsets of the fragment reads: 16-byte chunk 4 c + g of the lane's row (within a half, wave row 0); BTR: the
         // lane's 8-byte piece of fragment column j
         constexpr int FA = fmh(0) > fmh(1) ? fmh(0) : fmh(1), FB = fnh(0) > fnh(1) ? fnh(0) : fnh(1);
@@ -235,6 +307,24 @@ struct GemmPipe {
             for (int h = 0; h < 2; ++h)  // of fragment column 0; column j's chunk differs by an XOR (fnh is a power of two)
                 rt[h] = (uint32_t)(k * hn(h) + ((wn * fnh(h)) ^ swz_tr(h, k)) * 16 + (r16 & 1) * 8);
         }
+        // fragment u of the weights held for half h, dequantised; its place: column l % 16 of the strip, chunk 4 jj + l / 16
+        // (the layout of the reads)
+        [[maybe_unused]] h8 wfrag;
+        auto dequant_w = [&](auto HH, auto PAR, int u) {
+            constexpr int h = decltype(HH)::value, par = decltype(PAR)::value & 1;
+            if (u >= cb(h)) return;
+            const WeightRegs& r = wr[par][h];
+            const _Float16 sv = __builtin_bit_cast(_Float16, (uint16_t)r.sc);
+            const _Float16 ov = HAS_OFF ? __builtin_bit_cast(_Float16, (uint16_t)r.of) : (_Float16)0.0f;
+            wfrag = dequant8<I4, HAS_OFF>(r.w[u][0], I4 ? 0u : r.w[u][1], (h2){ov, ov}, (h2){sv, sv}, magic);
+        };
+        auto store_w = [&](auto HH, int u) {
+            constexpr int h = decltype(HH)::value;
+            if (u >= cb(h)) return;
+            const int strip = cb(h) == 2 ? wave : wave >> 1;
+            const uint32_t o = cb(h) == 2 ? rl[u] : rl[0] ^ ((wave & 1) * 64u);
+            *(h8*)(sB + (h * hn(0) + strip * 16) * ROWB + o) = wfrag;
+        };
         const uint32_t wa[2] = {(uint32_t)(wm * whm(0) * ROWB), (uint32_t)((hm(0) + wm * whm(1)) * ROWB)};
         const uint32_t wb[2] = {(uint32_t)(wn * whn(0) * ROWB), (uint32_t)((hn(0) + wn * whn(1)) * ROWB)};
         frag_t fa[2][FA][KPS], fb[2][FB][KPS];
@@ -322,7 +412,10 @@ struct GemmPipe {
                 if (x < x0 || x >= x1) continue;
                 const int s = x / (fn * fm), j = x / fm % fn, i = x % fm;
                 acc_t& c = acc[ha * fmh(0) + i][hb * fnh(0) + j];
-                if constexpr (OP == OP_I8)
+                if constexpr (IS_AQ)
+                    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, fb[set][j][s]),
+                                                               __builtin_bit_cast(h8, fa[ha][i][s]), c, 0, 0, 0);
+                else if constexpr (OP == OP_I8)
                     c = __builtin_amdgcn_mfma_i32_16x16x64_i8(fb[set][j][s], fa[ha][i][s], c, 0, 0, 0);
                 else if constexpr (OP == OP_F8)
                     c = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fb[set][j][s], fa[ha][i][s], c, BLGP, CBSZ, 0, 0, 0,
@@ -358,6 +451,41 @@ struct GemmPipe {
 
         // prologue: the ring's halves in flight, H(0) and H(1) into registers, then H(4 ST) into the slot of H(0)
         // (scales where the loop's phases 2 would have requested them, so that `outstanding` holds from phase 0 on)
+        if constexpr (IS_AQ) {  // in the loop's order, so that `outstanding` holds from phase 1 on
+            load_w(I0{}, I0{}, 0);
+            load_w(I1{}, I0{}, 0);
+            load_w(I0{}, I1{}, 1);
+            __builtin_amdgcn_sched_barrier(0);
+            request(I0{}, 0, 0);
+            request(I3{}, 0, 0);
+            load_w(I1{}, I1{}, 1);
+            __builtin_amdgcn_sched_barrier(0);
+            request(I0{}, 1, 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                dequant_w(I0{}, I0{}, u);
+                store_w(I0{}, u);
+                dequant_w(I1{}, I0{}, u);
+                store_w(I1{}, u);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            load_w(I0{}, I0{}, 2);
+            __builtin_amdgcn_sched_barrier(0);
+            request(I3{}, 1, 1);
+            load_w(I1{}, I0{}, 2);
+            dequant_w(I0{}, I1{}, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            wait_half<ca(0) + 2 * ca(1)>();
+            stage_barrier();
+            read_a(I0{}, 0, 0);
+            read_b(I0{}, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            wait_half<63>();
+            stage_barrier();
+            request(I0{}, ST, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        } else {
         request_scales(0);
 #pragma unroll
         for (int k = 0; k < ST; ++k) {
@@ -377,6 +505,7 @@ struct GemmPipe {
         stage_barrier();
         request(I0{}, ST, 0);
         __builtin_amdgcn_sched_barrier(0);
+        }
 
         // phase P of stage kt, which lies in slot SL of the ring (kt = SL modulo ST)
         auto phase = [&](auto PP, auto SS, int kt) {
@@ -390,21 +519,35 @@ struct GemmPipe {
             __builtin_amdgcn_sched_barrier(0);
             wait_half<outstanding(P)>();
             stage_barrier();
+            if constexpr (IS_AQ) {
+                store_w(std::integral_constant<int, (P >= 2)>{}, P & 1);
+                __builtin_amdgcn_sched_barrier(0);
+            }
             multiply(HA{}, HB{}, set, 0, LEAD);
             __builtin_amdgcn_sched_barrier(0);
-            if constexpr (P == 0) read_b(I1{}, set1, SL, kt);
+            constexpr int SB = IS_AQ ? 0 : SL, SBN = IS_AQ ? 0 : SN;  // B's slots
+            if constexpr (P == 0) read_b(I1{}, set1, SB, kt);
             if constexpr (P == 1) read_a(I1{}, SL, kt);
             if constexpr (P == 2) read_a(I0{}, SN, kt + 1);
-            if constexpr (P == 3) read_b(I0{}, set1, SN, kt + 1);
+            if constexpr (P == 3) read_b(I0{}, set1, SBN, kt + 1);
             __builtin_amdgcn_sched_barrier(0);
-            if constexpr (P == 0) request(I1{}, kt + ST, SL);
-            if constexpr (P == 1) request(I2{}, kt + ST, SL);
+            if constexpr (IS_AQ) {
+                if constexpr (P == 1) load_w(I0{}, std::integral_constant<int, SN>{}, kt + 3);
+                if constexpr (P == 3) load_w(I1{}, std::integral_constant<int, SN>{}, kt + 3);
+                __builtin_amdgcn_sched_barrier(0);
+            } else {
+                if constexpr (P == 0) request(I1{}, kt + ST, SL);
+                if constexpr (P == 1) request(I2{}, kt + ST, SL);
+            }
             if constexpr (P == 2) {
                 request_scales(kt + 3);
                 request(I3{}, kt + ST, SL);
             }
             if constexpr (P == 3) request(I0{}, kt + 1 + ST, SN);
             __builtin_amdgcn_sched_barrier(0);
+            if constexpr (IS_AQ)  // (phase 3: of the stage after)
+                dequant_w(std::integral_constant<int, (P == 1 || P == 2)>{}, std::integral_constant<int, P == 3 ? SL : SN>{},
+                          P == 0 || P == 2);
             multiply(HA{}, HB{}, set, LEAD, NX);
         };
         auto stage = [&](auto SS, int kt) {

@@ -1372,28 +1372,48 @@ hipError_t launch_antiquant_matmul(uint16_t* y, const uint16_t* x, const void* w
     // column-block kernels: groups of 128 << s, or one group over all of K (per channel)
     const bool cols_ok = K % KT == 0 && ((g % KT == 0 && ((g / KT) & (g / KT - 1)) == 0) || g >= K);
     // Above 64 rows: aq_ring_kernel over row blocks (grid.y) -- x shared through the LDS ring by the strip groups of a
-    // block, each weight fragment dequantised once per block of rows and multiplied against all of them.  64-row
-    // blocks of 6 strips (2 strip groups x 4 k-split waves) while they make about one block per CU, else 128-row blocks
-    // of 12 strips (4 strip groups x 2 k-split waves).  Measured at K = 4096, N = 11008 (int4 / int8, M = 128 / 512 /
-    // 2048): 27 / 63 / 239 us against 71 / 78 / 250 us for the LDS-staged MFMA GEMM of aq_gemm.hip, which takes the
-    // shapes the ring does not (LDS too small for the scale rows), then 64-row passes of the kernels below.  When KW does
-    // not divide the k tiles (K = 11008: 86 tiles) the ring's last round is partial.
-    if (M > 64 && cols_ok) {
+    // block, each weight fragment dequantised once per block of rows and multiplied against all of them -- or the
+    // pipelined tiles of aq_gemm.hip, which dequantise a weight once per 64 - 256 rows.  Ring blocks of 64 rows and up to
+    // 6 strips (2 strip groups x 4 k-split waves) while they make about one block per CU, else of 128 rows and up to 12
+    // strips (4 strip groups x 2 k-split waves); a long K with a scale row per k tile (K = 11008, g = 128: 86 rows)
+    // leaves both without LDS for the scale rows, and 64-row blocks of two k-split waves halve the activation stages.  No
+    // more blocks than CUs where the strips per block allow it: 258 blocks run twice as long as 256 (768 x 4096 x 4096:
+    // 78 us).  About what a form takes per 64 k, in microseconds, measured at the sizes of aq_gemm_us: 64-row blocks 0.36
+    // in one round, 0.54 in up to 320 blocks, 0.35 a round with two k-split waves; 128-row blocks 0.65 a round to 6
+    // strips, 0.87 at 12.  Ring against tiles: 512 x 11008 x 4096 57 / 61 us, 256 x 4096 x 4096 21 / 39, 1024 x 11008 x
+    // 4096 109 / 86, 2048 x 11008 x 4096 222 / 177, 1024 x 8192 x 8192 int8 303 / 147, 512 x 4096 x 11008 122 / 100.
+    // Groups of 64 (256 x 14336 x 4096, int8): 48 us, in 64-row passes of the kernels below 99.
+    if (M > 64 && K % KT == 0) {
         const int64_t rb64 = (M + 63) / 64, rb128 = (M + 127) / 128;
-        const int c64 = aq_blocks(NBT, 6, (int)((256 + rb64 - 1) / rb64));
+        auto blocks = [&](int smax, int64_t rb) { return aq_blocks(NBT, smax, (int)(rb < 256 ? 256 / rb : 1)); };
+        const int c64 = blocks(6, rb64), c128 = blocks(12, rb128);
+        enum { NONE, R64, R128, R64_LONG } form = NONE;
+        const float st64 = (float)(K / 64), rounds64 = (float)((c64 * rb64 + 255) / 256);
+        float us = 0.0f;
+        if (!cols_ok) {
+        } else if (c64 * rb64 <= 320 && aq_ring_lds<4, 3, 2, 4, 2, 2>(K, offset != nullptr)) {
+            form = R64;
+            us = (rounds64 > 1.0f ? 0.54f : 0.36f) * st64;
+        } else if (aq_ring_lds<8, 3, 4, 2, 2, 2>(K, offset != nullptr)) {
+            form = R128;
+            const int64_t strips = (NBT + c128 - 1) / c128;
+            us = (float)((c128 * rb128 + 255) / 256) * (0.65f + 0.0375f * (float)(strips > 6 ? strips - 6 : 0)) * st64;
+        } else if (aq_ring_lds<4, 3, 2, 2, 2, 2>(K, offset != nullptr)) {
+            form = R64_LONG;
+            us = rounds64 * 0.35f * st64;
+        }
         hipError_t e = hipErrorInvalidValue;
-        if (c64 * rb64 <= 320 && aq_ring_lds<4, 3, 2, 4, 2, 2>(K, offset != nullptr))
-            e = launch_aq_ring<4, 3, 2, 4, 2, 2>(y, x, wp, int4, scale, offset, g, M, N, K, c64, atomic, st);
-        else if (aq_ring_lds<8, 3, 4, 2, 2, 2>(K, offset != nullptr))
-            e = launch_aq_ring<8, 3, 4, 2, 2, 2>(y, x, wp, int4, scale, offset, g, M, N, K,
-                                                 aq_blocks(NBT, 12, (int)((256 + rb128 - 1) / rb128)), atomic, st);
-        // long K with a scale row per k tile (K = 11008, g = 128: 86 rows) leaves both forms above without LDS for
-        // the scale rows; 64-row blocks of two k-split waves halve the activation stages
-        else if (aq_ring_lds<4, 3, 2, 2, 2, 2>(K, offset != nullptr))
-            e = launch_aq_ring<4, 3, 2, 2, 2, 2>(y, x, wp, int4, scale, offset, g, M, N, K, c64, atomic, st);
+        auto tiles = [&]() { return launch_aq_gemm(y, x, wp, w_type, scale, offset, group, M, N, K, atomic, st); };
+        const bool tiles_first = form == NONE || aq_gemm_us(M, N, K) < us;
+        if (tiles_first) e = tiles();
         if (e == hipErrorInvalidValue) {
+            if (form == R64) e = launch_aq_ring<4, 3, 2, 4, 2, 2>(y, x, wp, int4, scale, offset, g, M, N, K, c64, atomic, st);
+            if (form == R128) e = launch_aq_ring<8, 3, 4, 2, 2, 2>(y, x, wp, int4, scale, offset, g, M, N, K, c128, atomic, st);
+            if (form == R64_LONG) e = launch_aq_ring<4, 3, 2, 2, 2, 2>(y, x, wp, int4, scale, offset, g, M, N, K, c64, atomic, st);
+        }
+        if (e == hipErrorInvalidValue && !tiles_first) {
             (void)hipGetLastError();
-            e = launch_aq_gemm(y, x, wp, w_type, scale, offset, group, M, N, K, atomic, st);
+            e = tiles();
         }
         if (e != hipErrorInvalidValue) return e;
         (void)hipGetLastError();

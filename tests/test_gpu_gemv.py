@@ -190,11 +190,11 @@ def test_partial_rounds_and_per_channel(ascq_gpu, oracle, w_type, M, K, N, group
     (200, 1024, 4112, 256),   # partial row block; 257 strips: the last column block holds one strip
     (128, 2048, 272, 2048),   # one group over all of K
     (1000, 768, 1008, 128),   # eight row blocks, the last one partial
-    (300, 640, 272, 128),     # K = 5 tiles of 128: the LDS-staged MFMA GEMM (the ring kernels split K in 2 or 4)
+    (300, 640, 272, 128),     # K = 5 tiles of 128 (the ring kernels split K in 2 or 4)
 ])
 def test_prefill_gemm(ascq_gpu, oracle, w_type, with_offset, M, K, N, group):
     """M > 64: the ring kernel over row blocks (64-row blocks while they make about one block per CU, else 128-row
-    blocks) or, for K not a multiple of 256, the LDS-staged MFMA GEMM of aq_gemm.hip; the weights bit-exact as
+    blocks) or the pipelined MFMA tiles of aq_gemm.hip, whichever is estimated faster; the weights bit-exact as
     AscendAntiQuant, fp32 accumulation within the bound of check_close"""
     rng = seeded(M + K + N + group + with_offset)
     code = O.INT8 if w_type == "int8" else O.INT4
@@ -206,6 +206,33 @@ def test_prefill_gemm(ascq_gpu, oracle, w_type, with_offset, M, K, N, group):
     _, y_exact, y_abs = O.antiquant_matmul(x.view(np.uint16), w, code, scale.view(np.uint16),
                                            None if offset is None else offset.view(np.uint16), group, M, N, K)
     check_close(y.cpu().numpy(), y_exact, y_abs, K)
+
+
+@pytest.mark.parametrize("w_type,with_offset", [("int4", True), ("int8", False), ("int4", False), ("int8", True)])
+@pytest.mark.parametrize("M,K,N,group", [
+    (65, 128, 16, 64),        # 64 x 128 tiles: two stages, one strip, one row in the second tile
+    (129, 640, 4112, 64),     # 64 x 128: one row and one strip in the last tiles
+    (577, 2560, 4112, 64),    # 128 x 128
+    (383, 4096, 11008, 64),   # 128 x 192: 64 columns in the last tile
+    (1000, 1024, 11008, 64),  # 256 x 192: 232 rows and 64 columns in the last tiles
+    (1000, 1280, 11024, 256), # groups over two packed tiles, against the ring kernel's time
+    (600, 2944, 4096, 2944),  # one group over all of K, 23 packed tiles
+])
+def test_prefill_tiles(ascq_gpu, oracle, w_type, with_offset, M, K, N, group):
+    """M > 64 on the pipelined tiles of aq_gemm.hip (groups of 64 always; the others where they beat the ring kernel):
+    every output of sampled rows, both sides of each 64-row boundary among them, within the bound of check_close"""
+    rng = seeded(M + K + N + group + with_offset)
+    code = O.INT8 if w_type == "int8" else O.INT4
+    at = ascq_gpu.INT8 if w_type == "int8" else ascq_gpu.INT4
+    w, scale, offset = make_weights(rng, K, N, code, group, with_offset)
+    x = rng.standard_normal((M, K)).astype(np.float16)
+    wp = ascq_gpu.weight_pack(_dev(w), at, K, N)
+    y = ascq_gpu.antiquant_matmul(_dev(x), wp, at, _dev(scale), None if offset is None else _dev(offset), group, N)
+    edges = np.arange(0, M, 64)
+    rows = np.unique(np.concatenate([edges, edges[1:] - 1, [M - 1], rng.choice(M, 8)]))
+    _, y_exact, y_abs = O.antiquant_matmul(np.ascontiguousarray(x[rows]).view(np.uint16), w, code, scale.view(np.uint16),
+                                           None if offset is None else offset.view(np.uint16), group, len(rows), N, K)
+    check_close(y.cpu().numpy()[rows], y_exact, y_abs, K)
 
 
 @pytest.mark.parametrize("w_type", ["int4", "int8"])
