@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdarg>
+#include <cstdint>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -266,26 +267,31 @@ ascq_status ensure_workspace(ascq_matmul_s* h)
     return ASCQ_OK;
 }
 
-// the K-split partials' region of the workspace for this call (null when the call cannot use it: no split form for
-// these sizes, enAtomic, or a caller's workspace too small for it -- then the call runs without the split)
-ascq_status split_region(ascq_matmul_s* h, int64_t m, int64_t n, int64_t k, uint8_t en_atomic, uint8_t** ws,
+// the end of the K-split partials' region of a call of m x n x k (bytes_workspace is that of the org shape, which can have
+// no split form where a smaller single shape has one)
+size_t split_end(const ascq_matmul_s* h, int64_t m, int64_t n, int64_t k)
+{
+    return bytes_operands(h) + ascq::decode_split_ws_bytes(m, n, k, h->trans_b || bytes_nz_b(h));
+}
+
+// the K-split partials' region of the workspace for this call, `end` bytes of which are the call's own (packed operands
+// lie behind them); null when the call cannot use it: no split form for these sizes, enAtomic, or a workspace too small
+// for it -- then the call runs without the split
+ascq_status split_region(ascq_matmul_s* h, int64_t m, int64_t n, int64_t k, uint8_t en_atomic, size_t end, uint8_t** ws,
                          size_t* bytes)
 {
     *ws = nullptr;
     *bytes = 0;
-    const int tb = h->trans_b || bytes_nz_b(h);  // B as the GEMM sees it
-    const size_t need = ascq::decode_split_ws_bytes(m, n, k, tb);
-    if (need == 0 || en_atomic != 0) return ASCQ_OK;
-    const size_t off = bytes_operands(h);
-    if (h->ws && !h->ws_owned) {  // the caller's workspace: used when it has room, never replaced
-        if (h->ws_bytes < off + need) return ASCQ_OK;
-    } else {
+    const size_t off = bytes_operands(h), need = split_end(h, m, n, k);
+    if (need == off || en_atomic != 0) return ASCQ_OK;
+    if (!h->ws || h->ws_owned) {  // (a caller's workspace is used when it has room, never replaced)
         ascq_status s = ensure_workspace(h);
         if (s != ASCQ_OK) return s;
-        if (h->ws_bytes < off + need) return ASCQ_OK;
     }
+    if (end > h->ws_bytes) end = h->ws_bytes;
+    if (end < need) return ASCQ_OK;
     *ws = (uint8_t*)h->ws + off;
-    *bytes = h->ws_bytes - off;
+    *bytes = end - off;
     return ASCQ_OK;
 }
 
@@ -296,6 +302,7 @@ struct ByteOperands {
     const uint8_t* B;
     int64_t lda, ldb;
     int trans_a, trans_b;
+    size_t ws_end = SIZE_MAX;  // the workspace up to the packed operands, if it holds any
 };
 
 ascq_status prepare_byte_operands(ascq_matmul_s* h, hipStream_t st, ByteOperands& o)
@@ -355,14 +362,22 @@ PackPlan pack_plan(bool fp8, const ByteOperands& o, int64_t m, int64_t n, int64_
     return p;
 }
 
-// what the packed operands of the org shape need on top of workspace_need (pointers, where set, included)
+// where the packed operands of a call of m x n x k begin: behind everything else that the call can take of the workspace
+size_t pack_base(const ascq_matmul_s* h, int64_t m, int64_t n, int64_t k)
+{
+    const size_t need = workspace_need(h), split = split_end(h, m, n, k);
+    return align256(need > split ? need : split);
+}
+
+// workspace_size with the room for the packed operands of the present shape and pointers; 0 when nothing is packed
 size_t pack_need(const ascq_matmul_s* h)
 {
     const Kind kind = kind_of(h->ty);
     if ((kind != K_INT8 && kind != K_F8) || h->M <= 0 || h->trans_a || bytes_nz_b(h)) return 0;
+    const int64_t m = h->sm > 0 ? h->sm : h->M, n = h->sn > 0 ? h->sn : h->N, k = h->sk > 0 ? h->sk : h->K;
     const ByteOperands o{(const uint8_t*)h->a, (const uint8_t*)h->b, h->K, h->trans_b ? h->K : h->N, 0, h->trans_b};
-    const PackPlan p = pack_plan(kind == K_F8, o, h->M, h->N, h->K);
-    return p.a_bytes + p.b_bytes;
+    const PackPlan p = pack_plan(kind == K_F8, o, m, n, k);
+    return p.a || p.b ? pack_base(h, m, n, k) + p.a_bytes + p.b_bytes : 0;
 }
 
 ascq_status pack_byte_operands(ascq_matmul_s* h, hipStream_t st, int64_t m, int64_t n, int64_t* k, bool fp8,
@@ -373,7 +388,7 @@ ascq_status pack_byte_operands(ascq_matmul_s* h, hipStream_t st, int64_t m, int6
     // (the smallest calls keep the element-wise kernel, which needs no workspace and which ASCQ_LOG names, though the
     // copy and the GEMM would be faster: 32 x 32 x 40 in 17.1 us, 40 x 40 x 41 in 9.3)
     if (fp8 && !o.trans_b && m * n * *k <= 32 * 32 * 40) return ASCQ_OK;
-    const size_t base = align256(workspace_need(h)), need = base + p.a_bytes + p.b_bytes;
+    const size_t base = pack_base(h, m, n, *k), need = base + p.a_bytes + p.b_bytes;
     if (h->ws_bytes < need) {
         if (h->no_alloc || (h->ws && !h->ws_owned)) return ASCQ_OK;
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
@@ -419,6 +434,7 @@ ascq_status pack_byte_operands(ascq_matmul_s* h, hipStream_t st, int64_t m, int6
         o.B = pb;
         o.ldb = p.pitch_b;
     }
+    o.ws_end = base;
     // both K-contiguous operands zero-padded: the GEMM runs whole chunks
     if (o.trans_b && p.a && p.b) *k = p.kp;
     return ASCQ_OK;
@@ -656,7 +672,7 @@ ascq_status ascq_matmul_workspace_size(ascq_matmul_t h, size_t* bytes)
 {
     if (!h || !bytes) return fail(ASCQ_E_INVALID_ARG, "workspace_size: null argument");
     *bytes = workspace_need(h);
-    if (const size_t pack = pack_need(h)) *bytes = align256(*bytes) + pack;  // (optional room, see pack_byte_operands)
+    if (const size_t pack = pack_need(h)) *bytes = pack;  // (optional room, see pack_byte_operands)
     return ASCQ_OK;
 }
 
@@ -731,7 +747,7 @@ ascq_status ascq_matmul_iterate_all(ascq_matmul_t h, void* c, uint8_t en_atomic,
         g.trans_a = o.trans_a;
         g.trans_b = o.trans_b;
         g.atomic = atomic;
-        s = split_region(h, m, n, k, atomic, &g.ws, &g.ws_bytes);
+        s = split_region(h, m, n, k, atomic, o.ws_end, &g.ws, &g.ws_bytes);
         if (s != ASCQ_OK) return s;
         return hip_status(ascq::launch_gemm_i8(g, st), "gemm_i8");
     }
@@ -858,7 +874,7 @@ ascq_status ascq_matmul_iterate_all(ascq_matmul_t h, void* c, uint8_t en_atomic,
         g.fmt_a = f8f6f4_code(h->ty.a_type);
         g.fmt_b = f8f6f4_code(h->ty.b_type);
         g.atomic = atomic;
-        s = split_region(h, m, n, k, atomic, &g.ws, &g.ws_bytes);
+        s = split_region(h, m, n, k, atomic, o.ws_end, &g.ws, &g.ws_bytes);
         if (s != ASCQ_OK) return s;
         return hip_status(ascq::launch_gemm_f8(g, st), "gemm_f8");
     }
@@ -994,7 +1010,7 @@ ascq_status ascq_matmul_iterate_all_noalloc(ascq_matmul_t h, void* c, uint8_t en
                     "(use ascq_matmul_iterate_all with a workspace)", need, (size_t)ASCQ_NOALLOC_SCRATCH_BYTES);
     void* ptr = nullptr;
     const size_t pack = pack_need(h);  // taken where the scratch has room for it
-    const bool use = need > 0 || (pack > 0 && align256(need) + pack <= ASCQ_NOALLOC_SCRATCH_BYTES);
+    const bool use = need > 0 || (pack > 0 && pack <= ASCQ_NOALLOC_SCRATCH_BYTES);
     if (use) {
         ascq_status s = scratch_for_current_device(&ptr);
         if (s != ASCQ_OK) return s;

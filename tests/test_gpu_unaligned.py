@@ -185,3 +185,33 @@ def test_fallback_logged_under_ascq_log():
     lines = [ln for ln in r.stderr.splitlines() if ln.startswith("ascq:")]
     assert lines == ["ascq: fallback: gemm_f8_generic_kernel (B given [K, N] with K not a multiple of 16 or operands "
                      "not aligned)"], r.stderr[-2000:]
+
+
+@pytest.mark.parametrize("where", ["owned", "reported", "scratch"])
+@pytest.mark.parametrize("org,single,b_off", [((1000, 4096, 8200), (16, 4096, 8192), 0), ((16, 8192, 8192), (16, 4096, 8192), 4),
+                                              ((128, 4096, 8192), (40, 4096, 8192), 1)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_packed_operands_beside_split_partials(ascq_gpu, oracle, fp8, org, single, b_off, where):
+    """B [N, K] rows off their alignment (packed), an org shape without the K split across workgroups and a single shape
+    with it: the split's partials and the packed operands are both in use.  Integer-valued operands, exact sums"""
+    ascq = ascq_gpu
+    (M, N, K), (m, n, k) = org, single
+    rng = seeded(M + K + b_off)
+    A = rng.integers(-4, 5, (M, K), dtype=np.int8)
+    B = rng.integers(-4, 5, (N, K), dtype=np.int8)
+    ref = torch.from_numpy(A[:m, :k]).float() @ torch.from_numpy(B[:n, :k]).float().t()  # (below 2^18: exact)
+    code = (lambda v: torch.from_numpy(v).float().to(torch.float8_e4m3fn).view(torch.uint8).numpy()) if fp8 else (lambda v: v)
+    mm = ascq.Matmul(ascq.FP8_E4M3, ascq.FP8_E4M3, ascq.F32) if fp8 else ascq.Matmul(ascq.INT8, ascq.INT8, ascq.INT32)
+    mm.SetOrgShape(M, N, K)
+    mm.SetSingleShape(m, n, k)
+    mm.SetTensorA(_dev(code(A)))
+    mm.SetTensorB(_dev_at(code(B), b_off), True)
+    if where == "reported":
+        nbytes = mm.WorkspaceSize()
+        mm.SetWorkspace(torch.empty(nbytes, dtype=torch.uint8, device="cuda"), nbytes)
+    c = torch.zeros((M, N), dtype=torch.float32 if fp8 else torch.int32, device="cuda")
+    for _ in range(3):
+        c.zero_()
+        (mm.IterateAllNoAlloc if where == "scratch" else mm.IterateAll)(c)
+        assert torch.equal(c[:m, :n].cpu().float(), ref)
+    assert not bool(c[m:].any()) and not bool(c[:, n:].any())

@@ -1,0 +1,29 @@
+"""The host layer's use of workspaces (CPU only): the built library driven by tests/cpp/workspace_regions.cpp, which
+stands in for its kernel launchers and HIP calls."""
+from __future__ import annotations
+
+import os
+import subprocess
+from pathlib import Path
+
+import ascq
+
+ROOT = Path(__file__).resolve().parent.parent
+HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+
+
+def _run(tmp_path, name):
+    exe = tmp_path / name
+    libdir = Path(ascq.LIB_PATH).parent
+    subprocess.run([HIPCC, "--offload-arch=gfx950", "--offload-host-only", "-x", "hip", "-std=c++17", "-O1", "-I", str(ROOT / "include"),
+                    str(ROOT / "tests" / "cpp" / f"{name}.cpp"), "-rdynamic", "-L", str(libdir), "-lascq",
+                    f"-Wl,-rpath,{libdir}", "-Wl,-rpath,/opt/rocm/lib", "-o", str(exe)],
+                   check=True)
+    return subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
+
+
+def test_regions_of_a_call_are_disjoint(tmp_path):
+    """int8 and fp8, org x single shape x layout x alignment, in a handle's own workspace, a caller's of the reported
+    size, a larger one and the static scratch: packed operands, operand copies and split partials share no byte"""
+    r = _run(tmp_path, "workspace_regions")
+    assert r.returncode == 0, r.stdout[-3000:] + r.stderr[-2000:]
