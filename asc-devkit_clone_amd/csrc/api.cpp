@@ -140,6 +140,8 @@ struct ascq_matmul_s {
     void* ws = nullptr;
     size_t ws_bytes = 0;
     bool ws_owned = false;
+    void* pack = nullptr;   // room for packed operands (pack_byte_operands)
+    size_t pack_bytes = 0;
     bool no_alloc = false;  // a call of the allocation-free form (set in its copy of the handle)
 };
 
@@ -338,10 +340,12 @@ ascq_status prepare_byte_operands(ascq_matmul_s* h, hipStream_t st, ByteOperands
 }
 
 // Operands whose rows the aligned kernels cannot take -- a K that is not a multiple of 16 bytes, rows or pointers off
-// their alignment (16 bytes; a [K, N] B: 4) -- are copied to aligned zero-padded rows in the workspace: a copy at the
-// memory rate against tiles that realign every chunk they load (int8 1030 x 4100 x 4095, B [K, N]: 139 -> 31 us; one row: 66 -> 18 us).  The
-// room is optional: a caller's workspace without it, a stream under capture whose handle holds too little, or a failed
-// allocation leave the call to the any-alignment tiles.
+// their alignment (16 bytes; a [K, N] B: 4) -- are copied to aligned zero-padded rows: a copy at the memory rate against
+// tiles that realign every chunk they load (int8 1030 x 4100 x 4095, B [K, N]: 139 -> 31 us; one row: 66 -> 18 us).  They
+// go behind the rest of a caller's workspace, or into an allocation of the handle's own beside its workspace, which a
+// graph may hold and a mere pointer must not replace.  The room is optional: a caller's workspace without it, a stream
+// under capture (the graph would share the room with later eager calls) or a failed allocation leave the call to the
+// any-alignment tiles.
 struct PackPlan {
     bool a, b;
     int64_t kp, pitch_b;  // bytes of a packed row of A (and of a K-contiguous B); of a packed row of B
@@ -380,6 +384,27 @@ size_t pack_need(const ascq_matmul_s* h)
     return p.a || p.b ? pack_base(h, m, n, k) + p.a_bytes + p.b_bytes : 0;
 }
 
+// `bytes` of the handle's own room for packed operands, or null
+uint8_t* pack_room(ascq_matmul_s* h, hipStream_t st, size_t bytes)
+{
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (h->no_alloc || hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (h->pack_bytes < bytes) {
+        if (h->pack) (void)hipFree(h->pack);
+        h->pack_bytes = 0;
+        if (hipMalloc(&h->pack, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            h->pack = nullptr;
+            return nullptr;
+        }
+        h->pack_bytes = bytes;
+    }
+    return (uint8_t*)h->pack;
+}
+
 ascq_status pack_byte_operands(ascq_matmul_s* h, hipStream_t st, int64_t m, int64_t n, int64_t* k, bool fp8,
                                ByteOperands& o, int* a_padded)
 {
@@ -388,36 +413,17 @@ ascq_status pack_byte_operands(ascq_matmul_s* h, hipStream_t st, int64_t m, int6
     // (the smallest calls keep the element-wise kernel, which needs no workspace and which ASCQ_LOG names, though the
     // copy and the GEMM would be faster: 32 x 32 x 40 in 17.1 us, 40 x 40 x 41 in 9.3)
     if (fp8 && !o.trans_b && m * n * *k <= 32 * 32 * 40) return ASCQ_OK;
-    const size_t base = pack_base(h, m, n, *k), need = base + p.a_bytes + p.b_bytes;
-    if (h->ws_bytes < need) {
-        if (h->no_alloc || (h->ws && !h->ws_owned)) return ASCQ_OK;
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
-            (void)hipGetLastError();
-            return ASCQ_OK;
-        }
-        void* ws = nullptr;
-        if (hipMalloc(&ws, need) != hipSuccess) {
-            (void)hipGetLastError();
-            return ASCQ_OK;
-        }
-        // (operands that prepare_byte_operands already put into the old workspace move along)
-        if (h->ws && base > 0) {
-            const hipError_t e = hipMemcpyAsync(ws, h->ws, base < h->ws_bytes ? base : h->ws_bytes, hipMemcpyDeviceToDevice, st);
-            if (e != hipSuccess) {
-                (void)hipFree(ws);
-                return hip_status(e, "move workspace");
-            }
-            const uint8_t *lo = (const uint8_t*)h->ws, *hi = lo + h->ws_bytes;
-            if (o.A >= lo && o.A < hi) o.A = (uint8_t*)ws + (o.A - lo);
-            if (o.B >= lo && o.B < hi) o.B = (uint8_t*)ws + (o.B - lo);
-        }
-        if (h->ws) (void)hipFree(h->ws);
-        h->ws = ws;
-        h->ws_bytes = need;
-        h->ws_owned = true;
+    const size_t need = p.a_bytes + p.b_bytes;
+    uint8_t* pa = nullptr;
+    if (h->ws && !h->ws_owned) {
+        const size_t base = pack_base(h, m, n, *k);
+        if (h->ws_bytes < base + need) return ASCQ_OK;
+        pa = (uint8_t*)h->ws + base;
+        o.ws_end = base;
+    } else {
+        pa = pack_room(h, st, need);
+        if (!pa) return ASCQ_OK;
     }
-    uint8_t* pa = (uint8_t*)h->ws + base;
     uint8_t* pb = pa + p.a_bytes;
     const ascq::PackRows ja{p.a ? pa : nullptr, o.A, m, *k, o.lda};
     const ascq::PackRows jb = o.trans_b ? ascq::PackRows{p.b ? pb : nullptr, o.B, n, *k, o.ldb}
@@ -434,7 +440,6 @@ ascq_status pack_byte_operands(ascq_matmul_s* h, hipStream_t st, int64_t m, int6
         o.B = pb;
         o.ldb = p.pitch_b;
     }
-    o.ws_end = base;
     // both K-contiguous operands zero-padded: the GEMM runs whole chunks
     if (o.trans_b && p.a && p.b) *k = p.kp;
     return ASCQ_OK;
@@ -680,6 +685,11 @@ ascq_status ascq_matmul_set_workspace(ascq_matmul_t h, void* workspace, size_t b
 {
     if (!h) return fail(ASCQ_E_INVALID_ARG, "null handle");
     if (h->ws_owned && h->ws) (void)hipFree(h->ws);
+    if (workspace && h->pack) {  // (the caller's workspace takes its place)
+        (void)hipFree(h->pack);
+        h->pack = nullptr;
+        h->pack_bytes = 0;
+    }
     h->ws = workspace;
     h->ws_bytes = workspace ? bytes : 0;
     h->ws_owned = false;
@@ -1040,6 +1050,7 @@ ascq_status ascq_matmul_destroy(ascq_matmul_t h)
 {
     if (!h) return ASCQ_OK;
     if (h->ws_owned && h->ws) (void)hipFree(h->ws);
+    if (h->pack) (void)hipFree(h->pack);
     delete h;
     return ASCQ_OK;
 }

@@ -1,98 +1,10 @@
 // Where an int8 / fp8 IterateAll puts what it keeps in a workspace: packed operands, transposed or converted operands and
-// the K-split partials of one call must not share a byte, and must lie inside the memory the call may use.  Links the
-// built library and stands in for its kernel launchers and for the HIP calls it makes (no GPU, nothing is computed).
+// the K-split partials of one call must not share a byte, and must lie inside the memory the call may use.
 // Exit status 0 = every call kept its regions apart.
-#include <cstdint>
 #include <cstdio>
-#include <cstdlib>
-#include <map>
 #include <string>
-#include <vector>
 
-#include "../../asc-devkit_clone_amd/csrc/launch.h"
-#include "ascq.h"
-
-struct Region {
-    uintptr_t at;
-    size_t bytes;
-    const char* what;
-};
-static std::vector<Region> used;         // by the present call
-static std::map<uintptr_t, size_t> heap;  // allocations (addresses only, never dereferenced)
-static uintptr_t next_at = 0x100000000ull;
-static bool capturing = false;
-
-static void use(const void* p, size_t bytes, const char* what)
-{
-    if (bytes) used.push_back({(uintptr_t)p, bytes, what});
-}
-
-extern "C" {
-hipError_t hipMalloc(void** p, size_t n)
-{
-    heap[next_at] = n;
-    *p = (void*)next_at;
-    next_at += (n + 0xFFFFF) / 0x100000 * 0x100000 + 0x100000;
-    return hipSuccess;
-}
-hipError_t hipFree(void* p)
-{
-    if (p && !heap.erase((uintptr_t)p)) std::abort();
-    return hipSuccess;
-}
-hipError_t hipMemcpyAsync(void* dst, const void* src, size_t n, hipMemcpyKind, hipStream_t)
-{
-    for (Region& r : used)
-        if (r.at >= (uintptr_t)src && r.at < (uintptr_t)src + n) r.at += (uintptr_t)dst - (uintptr_t)src;
-    return hipSuccess;
-}
-hipError_t hipGetLastError() { return hipSuccess; }
-hipError_t hipGetDevice(int* d)
-{
-    *d = 0;
-    return hipSuccess;
-}
-hipError_t hipGetSymbolAddress(void** p, const void*)
-{
-    *p = (void*)0x80000000ull;
-    return hipSuccess;
-}
-hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* s)
-{
-    *s = capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
-    return hipSuccess;
-}
-}
-
-namespace ascq {
-hipError_t launch_pack_rows(const PackRows& a, const PackRows& b, hipStream_t)
-{
-    if (a.dst) use(a.dst, (size_t)a.rows * ((a.cols + 15) / 16 * 16), "packed A");
-    if (b.dst) use(b.dst, (size_t)b.rows * ((b.cols + 15) / 16 * 16), "packed B");
-    return hipSuccess;
-}
-hipError_t launch_transpose_i8(uint8_t* dst, const uint8_t*, int64_t rows, int64_t cols, hipStream_t)
-{
-    use(dst, (size_t)(rows * cols), "transposed A");
-    return hipSuccess;
-}
-hipError_t launch_nz_to_nd(void* dst, const void*, int, int, int64_t rows, int64_t cols, int, hipStream_t)
-{
-    use(dst, (size_t)(rows * cols), "B from NZ");
-    return hipSuccess;
-}
-template <class G>
-static hipError_t gemm(const G& g)
-{
-    if (g.ws) {
-        use(g.ws, decode_split_ws_bytes(g.M, g.N, g.K, g.trans_b), "split partials");
-        if (decode_split_ws_bytes(g.M, g.N, g.K, g.trans_b) > g.ws_bytes) use(g.ws, SIZE_MAX / 2, "split partials (room)");
-    }
-    return hipSuccess;
-}
-hipError_t launch_gemm_i8(const GemmI8Args& g, hipStream_t) { return gemm(g); }
-hipError_t launch_gemm_f8(const GemmF8Args& g, hipStream_t) { return gemm(g); }
-}  // namespace ascq
+#include "host_stubs.h"
 
 static int failures = 0, calls = 0, packed_and_split = 0;
 static void check(const std::string& name, uintptr_t ws, size_t ws_bytes)

@@ -47,3 +47,43 @@ def test_antiquant_matmul_graph_replays(ascq_gpu, w_type, M):
         ascq_gpu.antiquant_matmul(xs[1], wp, at, scale, offset, g, N, out=ys[0])
         torch.cuda.synchronize()
     del graph
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+def test_eager_packed_call_leaves_a_captured_graph_alone(ascq_gpu, fp8):
+    """A decode call whose K-split partials lie in the handle's workspace, captured; then eager calls of the same handle
+    with a misaligned A, which is packed: every replay between them equals the eager result (integer-valued operands,
+    exact sums)"""
+    ascq = ascq_gpu
+    M, N, K = 16, 4096, 8192
+    g = torch.Generator().manual_seed(11)
+    A, B = torch.randint(-4, 5, (M, K), generator=g), torch.randint(-4, 5, (N, K), generator=g)
+    A2 = torch.randint(-4, 5, (M, K), generator=g)
+    dt = torch.float8_e4m3fn if fp8 else torch.int8
+    code = lambda t: t.float().to(dt).cuda()  # noqa: E731
+    ref, ref2 = A.float() @ B.float().t(), A2.float() @ B.float().t()
+    mm = ascq.Matmul(ascq.FP8_E4M3, ascq.FP8_E4M3, ascq.F32) if fp8 else ascq.Matmul(ascq.INT8, ascq.INT8, ascq.INT32)
+    mm.SetOrgShape(M, N, K)
+    a, b = code(A), code(B)
+    buf = torch.zeros(M * K + 16, dtype=torch.uint8, device="cuda")
+    buf[3:3 + M * K] = code(A2).view(torch.uint8).reshape(-1)
+    mm.SetTensorA(a)
+    mm.SetTensorB(b, True)
+    out = torch.zeros((M, N), dtype=torch.float32 if fp8 else torch.int32, device="cuda")
+    out2 = torch.zeros_like(out)
+    mm.IterateAll(out)
+    st = torch.cuda.Stream()
+    st.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(st), torch.cuda.graph(graph, stream=st):
+        mm.IterateAll(out)
+    torch.cuda.current_stream().wait_stream(st)
+    mm.SetTensorA(buf[3:3 + M * K])
+    for _ in range(3):
+        out2.zero_()
+        mm.IterateAll(out2)
+        assert torch.equal(out2.cpu().float(), ref2)
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.cpu().float(), ref)

@@ -27,3 +27,10 @@ def test_regions_of_a_call_are_disjoint(tmp_path):
     size, a larger one and the static scratch: packed operands, operand copies and split partials share no byte"""
     r = _run(tmp_path, "workspace_regions")
     assert r.returncode == 0, r.stdout[-3000:] + r.stderr[-2000:]
+
+
+def test_captured_memory_outlives_eager_calls(tmp_path):
+    """A graph captured over a handle that uses its own workspace, then eager calls whose operands are packed: the memory
+    that the graph uses stays allocated, and captured calls pack into a caller's workspace only"""
+    r = _run(tmp_path, "workspace_lifetime")
+    assert r.returncode == 0, r.stdout[-3000:] + r.stderr[-2000:]
