@@ -115,6 +115,15 @@ ascq_status scratch_for_current_device(void** out)
 }
 }  // namespace
 
+// Room for the packed operands of a handle's calls on one stream of one device: calls on different streams may overlap.
+struct PackRoom {
+    int device;
+    hipStream_t st;
+    void* p;
+    size_t bytes;
+};
+constexpr int kPackRooms = 4;
+
 struct ascq_matmul_s {
     ascq_matmul_types ty{};
     int64_t M = 0, N = 0, K = 0;        // org shape
@@ -140,8 +149,8 @@ struct ascq_matmul_s {
     void* ws = nullptr;
     size_t ws_bytes = 0;
     bool ws_owned = false;
-    void* pack = nullptr;   // room for packed operands (pack_byte_operands)
-    size_t pack_bytes = 0;
+    PackRoom rooms[kPackRooms] = {};  // for packed operands (pack_byte_operands)
+    int n_rooms = 0;
     bool no_alloc = false;  // a call of the allocation-free form (set in its copy of the handle)
 };
 
@@ -344,8 +353,8 @@ ascq_status prepare_byte_operands(ascq_matmul_s* h, hipStream_t st, ByteOperands
 // tiles that realign every chunk they load (int8 1030 x 4100 x 4095, B [K, N]: 139 -> 31 us; one row: 66 -> 18 us).  They
 // go behind the rest of a caller's workspace, or into an allocation of the handle's own beside its workspace, which a
 // graph may hold and a mere pointer must not replace.  The room is optional: a caller's workspace without it, a stream
-// under capture (the graph would share the room with later eager calls) or a failed allocation leave the call to the
-// any-alignment tiles.
+// under capture (the graph would share the room with later eager calls), a fifth stream or a failed allocation leave the
+// call to the any-alignment tiles.
 struct PackPlan {
     bool a, b;
     int64_t kp, pitch_b;  // bytes of a packed row of A (and of a K-contiguous B); of a packed row of B
@@ -384,25 +393,53 @@ size_t pack_need(const ascq_matmul_s* h)
     return p.a || p.b ? pack_base(h, m, n, k) + p.a_bytes + p.b_bytes : 0;
 }
 
-// `bytes` of the handle's own room for packed operands, or null
+// hipMalloc / hipFree of a room must not invalidate the capture of some other stream, as a call without a workspace never
+// did: in this scope the thread's calls are allowed beside captures.
+struct BesideCaptures {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    BesideCaptures() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~BesideCaptures() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    BesideCaptures(const BesideCaptures&) = delete;
+    BesideCaptures& operator=(const BesideCaptures&) = delete;
+};
+
+void free_rooms(ascq_matmul_s* h)
+{
+    if (h->n_rooms == 0) return;
+    BesideCaptures scope;
+    for (int i = 0; i < h->n_rooms; ++i)
+        if (h->rooms[i].p) (void)hipFree(h->rooms[i].p);
+    h->n_rooms = 0;
+}
+
+// `bytes` of the handle's own room for packed operands of a call on `st`, or null
 uint8_t* pack_room(ascq_matmul_s* h, hipStream_t st, size_t bytes)
 {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (h->no_alloc || hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+    int device = 0;
+    if (h->no_alloc || hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone ||
+        hipGetDevice(&device) != hipSuccess) {
         (void)hipGetLastError();
         return nullptr;
     }
-    if (h->pack_bytes < bytes) {
-        if (h->pack) (void)hipFree(h->pack);
-        h->pack_bytes = 0;
-        if (hipMalloc(&h->pack, bytes) != hipSuccess) {
+    int i = 0;
+    while (i < h->n_rooms && (h->rooms[i].st != st || h->rooms[i].device != device)) ++i;
+    if (i == kPackRooms) return nullptr;
+    if (i == h->n_rooms) h->rooms[h->n_rooms++] = PackRoom{device, st, nullptr, 0};
+    PackRoom& r = h->rooms[i];
+    if (r.bytes < bytes) {
+        BesideCaptures scope;
+        if (r.p) (void)hipFree(r.p);
+        r.p = nullptr;
+        r.bytes = 0;
+        if (hipMalloc(&r.p, bytes) != hipSuccess) {
             (void)hipGetLastError();
-            h->pack = nullptr;
+            r.p = nullptr;
             return nullptr;
         }
-        h->pack_bytes = bytes;
+        r.bytes = bytes;
     }
-    return (uint8_t*)h->pack;
+    return (uint8_t*)r.p;
 }
 
 ascq_status pack_byte_operands(ascq_matmul_s* h, hipStream_t st, int64_t m, int64_t n, int64_t* k, bool fp8,
@@ -685,11 +722,7 @@ ascq_status ascq_matmul_set_workspace(ascq_matmul_t h, void* workspace, size_t b
 {
     if (!h) return fail(ASCQ_E_INVALID_ARG, "null handle");
     if (h->ws_owned && h->ws) (void)hipFree(h->ws);
-    if (workspace && h->pack) {  // (the caller's workspace takes its place)
-        (void)hipFree(h->pack);
-        h->pack = nullptr;
-        h->pack_bytes = 0;
-    }
+    if (workspace) free_rooms(h);  // (the caller's workspace takes their place)
     h->ws = workspace;
     h->ws_bytes = workspace ? bytes : 0;
     h->ws_owned = false;
@@ -1050,7 +1083,7 @@ ascq_status ascq_matmul_destroy(ascq_matmul_t h)
 {
     if (!h) return ASCQ_OK;
     if (h->ws_owned && h->ws) (void)hipFree(h->ws);
-    if (h->pack) (void)hipFree(h->pack);
+    free_rooms(h);
     delete h;
     return ASCQ_OK;
 }

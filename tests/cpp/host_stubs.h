@@ -18,7 +18,10 @@ struct Region {
 static std::vector<Region> used;         // by the present call
 static std::map<uintptr_t, size_t> heap;  // allocations (addresses only, never dereferenced)
 static uintptr_t next_at = 0x100000000ull;
-static bool capturing = false;
+static bool capturing = false;  // the stream of the present call
+static int device = 0;
+static hipStreamCaptureMode capture_mode = hipStreamCaptureModeGlobal;
+static int alloc_not_relaxed = 0;  // hipMalloc / hipFree that would invalidate another stream's capture
 
 static void use(const void* p, size_t bytes, const char* what)
 {
@@ -28,6 +31,7 @@ static void use(const void* p, size_t bytes, const char* what)
 extern "C" {
 hipError_t hipMalloc(void** p, size_t n)
 {
+    alloc_not_relaxed += capture_mode != hipStreamCaptureModeRelaxed;
     heap[next_at] = n;
     *p = (void*)next_at;
     next_at += (n + 0xFFFFF) / 0x100000 * 0x100000 + 0x100000;
@@ -35,13 +39,21 @@ hipError_t hipMalloc(void** p, size_t n)
 }
 hipError_t hipFree(void* p)
 {
+    alloc_not_relaxed += capture_mode != hipStreamCaptureModeRelaxed;
     if (p && !heap.erase((uintptr_t)p)) std::abort();
     return hipSuccess;
 }
 hipError_t hipGetLastError() { return hipSuccess; }
 hipError_t hipGetDevice(int* d)
 {
-    *d = 0;
+    *d = device;
+    return hipSuccess;
+}
+hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode* m)
+{
+    const hipStreamCaptureMode old = capture_mode;
+    capture_mode = *m;
+    *m = old;
     return hipSuccess;
 }
 hipError_t hipGetSymbolAddress(void** p, const void*)

@@ -1,0 +1,52 @@
+// Calls of one handle on different streams and devices may overlap: operands packed by them share no byte; a stream beyond
+// the rooms a handle keeps packs nothing.  No room is allocated or freed in a way that would invalidate a capture of
+// another stream.  Exit status 0 = all of it holds.
+#include <cstdio>
+
+#include "host_stubs.h"
+
+static int failures = 0;
+#define EXPECT(cond)                                   \
+    do {                                               \
+        if (!(cond)) {                                 \
+            std::printf("line %d: %s\n", __LINE__, #cond); \
+            ++failures;                                \
+        }                                              \
+    } while (0)
+
+int main()
+{
+    for (int fp8 = 0; fp8 < 2; ++fp8) {
+        ascq_matmul_t h = nullptr;
+        ascq_matmul_types t{ASCQ_DT_INT8, ASCQ_DT_INT8, ASCQ_DT_INT32, 0, 0, 0};
+        if (fp8) t.a_type = t.b_type = ASCQ_DT_FP8_E4M3, t.c_type = ASCQ_DT_F32;
+        if (ascq_matmul_create(&t, &h) != ASCQ_OK) return 1;
+        ascq_matmul_set_tensor_a(h, (void*)0x10000000, 0);
+        ascq_matmul_set_tensor_b(h, (void*)0x20000000, 1);
+        std::map<std::pair<int, uintptr_t>, std::vector<Region>> last;
+        const std::pair<int, uintptr_t> where[] = {{0, 0}, {0, 0x100}, {1, 0}, {0, 0x200}, {0, 0x300}};
+        for (int call = 0; call < 20; ++call) {
+            const auto key = where[call * 3 % 5];
+            ascq_matmul_set_org_shape(h, 100, 1000, call < 10 ? 1001 : 5001);  // (the rooms grow on the way)
+            used.clear();
+            device = key.first;
+            EXPECT(ascq_matmul_iterate_all(h, (void*)0x30000000, 0, (void*)key.second) == ASCQ_OK);
+            last[key] = used;
+            for (const auto& a : last)
+                for (const auto& b : last)
+                    if (a.first != b.first)
+                        for (const Region& x : a.second)
+                            for (const Region& y : b.second) EXPECT(x.at >= y.at + y.bytes || y.at >= x.at + x.bytes);
+        }
+        int packing = 0;
+        for (const auto& a : last) packing += !a.second.empty();
+        EXPECT(packing == 4);
+        device = 0;
+        ascq_matmul_destroy(h);
+        EXPECT(heap.empty());
+        EXPECT(alloc_not_relaxed == 0);
+        EXPECT(capture_mode == hipStreamCaptureModeGlobal);
+    }
+    std::printf("%d failure(s)\n", failures);
+    return failures != 0;
+}

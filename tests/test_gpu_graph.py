@@ -87,3 +87,49 @@ def test_eager_packed_call_leaves_a_captured_graph_alone(ascq_gpu, fp8):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out.cpu().float(), ref)
+
+
+def test_packed_calls_beside_a_capture_and_on_two_streams(ascq_gpu):
+    """Calls whose operands are packed: the first call of a new handle on another stream while a capture is running leaves
+    the capture valid, and one handle used on two streams without waits between them computes both products"""
+    ascq = ascq_gpu
+    M, N, K = 300, 2000, 3001
+    g = torch.Generator().manual_seed(12)
+    A = [torch.randint(-4, 5, (M, K), generator=g) for _ in range(2)]
+    B = torch.randint(-4, 5, (K, N), generator=g)
+    ref = [x.float() @ B.float() for x in A]
+    a, b = [x.to(torch.int8).cuda() for x in A], B.to(torch.int8).cuda()
+
+    def handle():
+        mm = ascq.Matmul(ascq.INT8, ascq.INT8, ascq.INT32)
+        mm.SetOrgShape(M, N, K)
+        mm.SetTensorA(a[0])
+        mm.SetTensorB(b)
+        return mm
+
+    out = [torch.zeros((M, N), dtype=torch.int32, device="cuda") for _ in range(2)]
+    warm = handle()
+    warm.IterateAll(out[0])
+    x = torch.ones(64, device="cuda")
+    st, other = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    fresh = handle()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(st), torch.cuda.graph(graph, stream=st):
+        x.add_(1.0)
+        fresh.IterateAll(out[1], stream=other)
+    other.synchronize()
+    assert torch.equal(out[1].cpu().float(), ref[0])
+    for rep in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert bool((x == 2.0 + rep).all())
+    for o in out:
+        o.zero_()
+    torch.cuda.synchronize()
+    for i, s in enumerate((st, other)):
+        warm.SetTensorA(a[i])
+        warm.IterateAll(out[i], stream=s)
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert torch.equal(out[i].cpu().float(), ref[i])

@@ -34,3 +34,10 @@ def test_captured_memory_outlives_eager_calls(tmp_path):
     that the graph uses stays allocated, and captured calls pack into a caller's workspace only"""
     r = _run(tmp_path, "workspace_lifetime")
     assert r.returncode == 0, r.stdout[-3000:] + r.stderr[-2000:]
+
+
+def test_overlapping_streams_share_no_room(tmp_path):
+    """Calls of one handle on several streams and devices pack into rooms of their own (four at most), allocated and freed
+    without harm to captures of other streams"""
+    r = _run(tmp_path, "workspace_streams")
+    assert r.returncode == 0, r.stdout[-3000:] + r.stderr[-2000:]
