@@ -353,8 +353,8 @@ ascq_status prepare_byte_operands(ascq_matmul_s* h, hipStream_t st, ByteOperands
 // tiles that realign every chunk they load (int8 1030 x 4100 x 4095, B [K, N]: 139 -> 31 us; one row: 66 -> 18 us).  They
 // go behind the rest of a caller's workspace, or into an allocation of the handle's own beside its workspace, which a
 // graph may hold and a mere pointer must not replace.  The room is optional: a caller's workspace without it, a stream
-// under capture (the graph would share the room with later eager calls), a fifth stream or a failed allocation leave the
-// call to the any-alignment tiles.
+// under capture (the graph would share the room with later eager calls), a fifth stream, a failed allocation or the
+// allocation-free form (whose scratch all handles share) leave the call to the any-alignment tiles.
 struct PackPlan {
     bool a, b;
     int64_t kp, pitch_b;  // bytes of a packed row of A (and of a K-contiguous B); of a packed row of B
@@ -417,7 +417,7 @@ uint8_t* pack_room(ascq_matmul_s* h, hipStream_t st, size_t bytes)
 {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     int device = 0;
-    if (h->no_alloc || hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone ||
+    if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone ||
         hipGetDevice(&device) != hipSuccess) {
         (void)hipGetLastError();
         return nullptr;
@@ -450,6 +450,7 @@ ascq_status pack_byte_operands(ascq_matmul_s* h, hipStream_t st, int64_t m, int6
     // (the smallest calls keep the element-wise kernel, which needs no workspace and which ASCQ_LOG names, though the
     // copy and the GEMM would be faster: 32 x 32 x 40 in 17.1 us, 40 x 40 x 41 in 9.3)
     if (fp8 && !o.trans_b && m * n * *k <= 32 * 32 * 40) return ASCQ_OK;
+    if (h->no_alloc) return ASCQ_OK;
     const size_t need = p.a_bytes + p.b_bytes;
     uint8_t* pa = nullptr;
     if (h->ws && !h->ws_owned) {
@@ -1052,9 +1053,7 @@ ascq_status ascq_matmul_iterate_all_noalloc(ascq_matmul_t h, void* c, uint8_t en
                     "iterate_all_noalloc: this handle needs %zu bytes of workspace, above the %zu-byte static scratch "
                     "(use ascq_matmul_iterate_all with a workspace)", need, (size_t)ASCQ_NOALLOC_SCRATCH_BYTES);
     void* ptr = nullptr;
-    const size_t pack = pack_need(h);  // taken where the scratch has room for it
-    const bool use = need > 0 || (pack > 0 && pack <= ASCQ_NOALLOC_SCRATCH_BYTES);
-    if (use) {
+    if (need > 0) {
         ascq_status s = scratch_for_current_device(&ptr);
         if (s != ASCQ_OK) return s;
     }
@@ -1062,7 +1061,7 @@ ascq_status ascq_matmul_iterate_all_noalloc(ascq_matmul_t h, void* c, uint8_t en
     // and allocates nothing); the caller's handle is only read, so it never holds the scratch as its workspace
     ascq_matmul_s tmp = *h;
     tmp.ws = ptr;
-    tmp.ws_bytes = use ? (size_t)ASCQ_NOALLOC_SCRATCH_BYTES : 0;
+    tmp.ws_bytes = need > 0 ? (size_t)ASCQ_NOALLOC_SCRATCH_BYTES : 0;
     tmp.ws_owned = false;
     tmp.no_alloc = true;
     return ascq_matmul_iterate_all(&tmp, c, en_atomic, stream);

@@ -41,3 +41,9 @@ def test_overlapping_streams_share_no_room(tmp_path):
     without harm to captures of other streams"""
     r = _run(tmp_path, "workspace_streams")
     assert r.returncode == 0, r.stdout[-3000:] + r.stderr[-2000:]
+
+
+def test_allocation_free_calls_pack_nothing(tmp_path):
+    """IterateAllNoAlloc with operands off their alignment does not pack them into the scratch that all handles share"""
+    r = _run(tmp_path, "workspace_noalloc")
+    assert r.returncode == 0, r.stdout[-3000:] + r.stderr[-2000:]
