@@ -151,6 +151,7 @@ struct ascq_matmul_s {
     bool ws_owned = false;
     PackRoom rooms[kPackRooms] = {};  // for packed operands (pack_byte_operands)
     int n_rooms = 0;
+    bool room_later = false;  // a call has left a large room to the handle's next one
     bool no_alloc = false;  // a call of the allocation-free form (set in its copy of the handle)
 };
 
@@ -412,8 +413,11 @@ void free_rooms(ascq_matmul_s* h)
     h->n_rooms = 0;
 }
 
-// `bytes` of the handle's own room for packed operands of a call on `st`, or null
-uint8_t* pack_room(ascq_matmul_s* h, hipStream_t st, size_t bytes)
+// `bytes` of the handle's own room for packed operands of a call on `st`, or null.  gain_us: about what packing saves the
+// call.  hipMalloc, first touch and hipFree of more than 2 MiB take 36 us together (up to 2 MiB: 1 us), so where that is
+// more than one call saves, the handle's first such call goes without and a second one allocates (a handle used once,
+// int8 16 x 4096 x 1001, B [N, K]: 36 us without a room, 59 with; from its second call on 18.6 -> 10.5 us).
+uint8_t* pack_room(ascq_matmul_s* h, hipStream_t st, size_t bytes, float gain_us)
 {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     int device = 0;
@@ -428,6 +432,10 @@ uint8_t* pack_room(ascq_matmul_s* h, hipStream_t st, size_t bytes)
     if (i == h->n_rooms) h->rooms[h->n_rooms++] = PackRoom{device, st, nullptr, 0};
     PackRoom& r = h->rooms[i];
     if (r.bytes < bytes) {
+        if (bytes > (2u << 20) && gain_us < 36.0f && !h->room_later) {
+            h->room_later = true;
+            return nullptr;
+        }
         BesideCaptures scope;
         if (r.p) (void)hipFree(r.p);
         r.p = nullptr;
@@ -459,7 +467,10 @@ ascq_status pack_byte_operands(ascq_matmul_s* h, hipStream_t st, int64_t m, int6
         pa = (uint8_t*)h->ws + base;
         o.ws_end = base;
     } else {
-        pa = pack_room(h, st, need);
+        // the any-alignment tiles take 18 us per 1000 K and round of 128 tiles of 128 x 128, the packed form about 7; fp8
+        // with B [K, N] would run element by element
+        const int64_t rounds = (((m + 127) / 128) * ((n + 127) / 128) + 127) / 128;
+        pa = pack_room(h, st, need, fp8 && !o.trans_b ? 1e9f : 0.011f * (float)*k * (float)rounds);
         if (!pa) return ASCQ_OK;
     }
     uint8_t* pb = pa + p.a_bytes;

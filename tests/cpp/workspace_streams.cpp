@@ -47,6 +47,27 @@ int main()
         EXPECT(alloc_not_relaxed == 0);
         EXPECT(capture_mode == hipStreamCaptureModeGlobal);
     }
+    // a room that costs more than one call gains is left to the second call of a handle
+    const struct {
+        int64_t m, n, k;
+        int fp8, trans_b, first;
+    } once[] = {{16, 4096, 1001, 0, 1, 0}, {16, 4096, 1001, 1, 1, 0}, {16, 4096, 1003, 0, 0, 1}, {16, 4096, 1003, 1, 0, 1},
+                {1, 4100, 4095, 0, 1, 1},  {70, 200, 1003, 0, 1, 1},  {2000, 2000, 2001, 0, 1, 1}, {1000, 3000, 1001, 0, 1, 0}};
+    for (const auto& c : once) {
+        ascq_matmul_t h = nullptr;
+        ascq_matmul_types t{ASCQ_DT_INT8, ASCQ_DT_INT8, ASCQ_DT_INT32, 0, 0, 0};
+        if (c.fp8) t.a_type = t.b_type = ASCQ_DT_FP8_E4M3, t.c_type = ASCQ_DT_F32;
+        if (ascq_matmul_create(&t, &h) != ASCQ_OK) return 1;
+        ascq_matmul_set_org_shape(h, c.m, c.n, c.k);
+        ascq_matmul_set_tensor_a(h, (void*)0x10000000, 0);
+        ascq_matmul_set_tensor_b(h, (void*)0x20000000, c.trans_b);
+        for (int call = 0; call < 3; ++call) {
+            used.clear();
+            EXPECT(ascq_matmul_iterate_all(h, (void*)0x30000000, 0, nullptr) == ASCQ_OK);
+            EXPECT(!used.empty() == (call > 0 || c.first));
+        }
+        ascq_matmul_destroy(h);
+    }
     std::printf("%d failure(s)\n", failures);
     return failures != 0;
 }
