@@ -817,20 +817,16 @@ struct GemmCoreUA : GemmCore<BM, BN, WM, WN, 2, B_KCONTIG, OP, 64, FMT, true, CT
 __device__ __forceinline__ uint32_t acc_bits(float x) { return __float_as_uint(x); }
 __device__ __forceinline__ uint32_t acc_bits(int x) { return (uint32_t)x; }
 
-// Rolled epilogue of a GemmCore tile (T): the raw accumulators are parked in LDS -- free once every wave has left
-// the main loop -- and a rolled loop then takes one element per thread per step and hands put(tile row, tile
-// column, accumulator bits) the element.  Rolling the loop keeps the per-element code (a compare-and-swap, a software
-// encoder) and its registers out of an unrolled store path.  A tile that does not fit the LDS at once goes in NCH
-// chunks of rows: in chunk ch every wave writes the 32-row fragments that lie in it.  Column c of row r is parked at
-// c ^ (r % 32), so neither a layout with one column per lane nor one with one row per lane meets on one bank.
+// The raw accumulators of a tile (T) parked in LDS, which is free once every wave has left the main loop.  A tile that does
+// not fit the LDS at once goes in NCH chunks of rows: in chunk ch every wave writes the fragments that lie in it, then
+// body(first tile row, rows of the chunk) runs.  Column c of row r is parked at c ^ (r % 32), so neither a layout with one
+// column per lane nor one with one row per lane meets on one bank.
 template <class T, class F>
-__device__ __forceinline__ void rolled_epilogue(uint8_t* smem, const typename T::acc_t (&acc)[T::FM][T::FN], int rows,
-                                                int cols, F put)
+__device__ __forceinline__ void parked_chunks(uint8_t* smem, const typename T::acc_t (&acc)[T::FM][T::FN], F body)
 {
     constexpr int NCH = (size_t)T::TBM * T::TBN * 4 <= T::LDS_BYTES ? 1 : (size_t)T::TBM * T::TBN * 2 <= T::LDS_BYTES ? 2 : 4;
     constexpr int CHR = T::TBM / NCH;  // rows per chunk
-    static_assert((size_t)CHR * T::TBN * 4 <= T::LDS_BYTES && CHR % 16 == 0 && T::TBN % 32 == 0,
-                  "rolled epilogue chunks");
+    static_assert((size_t)CHR * T::TBN * 4 <= T::LDS_BYTES && CHR % 16 == 0 && T::TBN % 32 == 0, "chunks of a parked tile");
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wm = wave / T::TWN, wn = wave % T::TWN;
 #pragma unroll
@@ -848,25 +844,107 @@ __device__ __forceinline__ void rolled_epilogue(uint8_t* smem, const typename T:
                 }
         }
         __syncthreads();
-#pragma unroll 1
-        for (int e = threadIdx.x; e < CHR * T::TBN; e += T::NT) {
-            const int rr = ch * CHR + e / T::TBN, cc = e % T::TBN;
-            if (rr >= rows || cc >= cols) continue;
-            put(rr, cc, *(const uint32_t*)(smem + (e ^ (rr & 31)) * 4));
-        }
+        body(ch * CHR, CHR);
     }
 }
 
-// enAtomic epilogue of a GemmCore tile (T): the rolled epilogue with the output conversion conv(tile column,
-// accumulator bits) -> C bits combined into C by c_atomic.
+// Rolled epilogue of a tile (T): a rolled loop over the parked accumulators takes one element per thread per step and
+// hands put(tile row, tile column, accumulator bits) the element.  Rolling the loop keeps the per-element code (a software
+// encoder) and its registers out of an unrolled store path.
+template <class T, class F>
+__device__ __forceinline__ void rolled_epilogue(uint8_t* smem, const typename T::acc_t (&acc)[T::FM][T::FN], int rows,
+                                                int cols, F put)
+{
+    parked_chunks<T>(smem, acc, [&](int r0, int n) {
+#pragma unroll 1
+        for (int e = threadIdx.x; e < n * T::TBN; e += T::NT) {
+            const int rr = r0 + e / T::TBN, cc = e % T::TBN;
+            if (rr >= rows || cc >= cols) continue;
+            put(rr, cc, *(const uint32_t*)(smem + (e ^ (rr & 31)) * 4));
+        }
+    });
+}
+
+// enAtomic epilogue of a tile (T): the parked accumulators, converted by conv(tile column, accumulator bits) -> C bits, are
+// combined into C as c_atomic does: int32 by the native atomics, the other types by compare-and-swap loops on aligned
+// 32-bit words.  What bounds those is the round trip of each compare-and-swap, so a thread keeps four words in flight, and
+// two 16-bit elements of a word are combined by one thread in one exchange (by two threads, one of them always retried).
+// One element per thread and step took (fp8, bf16 C, K = 512, us)
+// 61 at M = 64, N = 256 and 736 at 2048 x 8192, this 21 and 98; f32 C 28 -> 24 on 64 x 128 tiles, 14 on 64 x 64.
 template <class T, int DT, class F>
 __device__ __forceinline__ void atomic_epilogue(uint8_t* smem, const typename T::acc_t (&acc)[T::FM][T::FN],
                                                 const TileOut& out, int rows, int cols, int op, F conv)
 {
-    constexpr int ES = (DT == DT_INT32 || DT == DT_F32) ? 4 : 2;  // bytes per C element
-    rolled_epilogue<T>(smem, acc, rows, cols, [&](int rr, int cc, uint32_t a) {
-        c_atomic<DT>(out.base + (uint32_t)rr * out.pitch + (uint32_t)(cc * ES), conv(cc, a), op);
-    });
+    if constexpr (DT == DT_INT32) {
+        rolled_epilogue<T>(smem, acc, rows, cols, [&](int rr, int cc, uint32_t a) {
+            c_atomic<DT>(out.base + (uint32_t)rr * out.pitch + (uint32_t)(cc * 4), conv(cc, a), op);
+        });
+    } else {
+        constexpr bool W16 = DT != DT_F32;
+        constexpr int WPR = W16 ? T::TBN / 2 + 1 : T::TBN;  // words of a tile row (16 bits: of any alignment)
+        constexpr int U = 4;                                // words in flight per thread
+        parked_chunks<T>(smem, acc, [&](int r0, int n) {
+            const int total = (rows - r0 < n ? rows - r0 : n) * WPR;
+            auto value = [&](int rr, int cc) -> uint32_t {
+                return conv(cc, *(const uint32_t*)(smem + (((rr - r0) * T::TBN + cc) ^ (rr & 31)) * 4));
+            };
+#pragma unroll 1
+            for (int e0 = threadIdx.x; e0 < total; e0 += U * T::NT) {
+                unsigned* w[U];
+                uint32_t v[U], old[U], todo[U];  // todo: which halves of the word (a whole f32 word: 1)
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int e = e0 + u * T::NT, rr = r0 + e / WPR, q = e % WPR;
+                    uint8_t* row = out.base + (uint32_t)rr * out.pitch;
+                    todo[u] = 0u;
+                    if (e >= total) continue;
+                    if constexpr (W16) {
+                        const int c = 2 * q - (int)((uintptr_t)row >> 1 & 1);  // the column of the word's lower half
+                        w[u] = (unsigned*)(row + c * 2);
+                        v[u] = 0u;
+                        if (c >= 0 && c < cols) v[u] = value(rr, c), todo[u] = 1u;
+                        if (c + 1 < T::TBN && c + 1 < cols) v[u] |= value(rr, c + 1) << 16, todo[u] |= 2u;
+                    } else if (q < cols) {
+                        w[u] = (unsigned*)(row + q * 4);
+                        v[u] = value(rr, q);
+                        todo[u] = 1u;
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (todo[u]) old[u] = __hip_atomic_load(w[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                uint32_t left;
+                do {  // (a word ends once no other writer changed it in between)
+                    uint32_t nw[U];
+                    left = 0u;
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        if (!todo[u]) continue;
+                        if constexpr (W16) {
+                            uint32_t lo = old[u] & 0xFFFFu, hi = old[u] >> 16;
+                            if (todo[u] & 1u) lo = c_combine<DT>(lo, v[u] & 0xFFFFu, op);
+                            if (todo[u] & 2u) hi = c_combine<DT>(hi, v[u] >> 16, op);
+                            nw[u] = lo | (hi << 16);
+                        } else {
+                            nw[u] = c_combine<DT>(old[u], v[u], op);
+                        }
+                        if (nw[u] == old[u]) todo[u] = 0u;
+                    }
+                    uint32_t prev[U];
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+                        if (todo[u]) prev[u] = atomicCAS(w[u], old[u], nw[u]);
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        if (!todo[u]) continue;
+                        if (prev[u] == old[u]) todo[u] = 0u;
+                        else old[u] = prev[u];
+                        left |= todo[u];
+                    }
+                } while (left);
+            }
+        });
+    }
 }
 
 }  // namespace ascq

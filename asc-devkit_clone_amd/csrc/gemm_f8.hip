@@ -358,11 +358,12 @@ static hipError_t launch_f8_fmt(const GemmF8Args& a, bool ua, hipStream_t st)
     const bool skinny = a.M <= 32 || (a.M <= 64 && t64 < 160);
     const bool c_wide = a.c_type == DT_F32 || a.c_type == DT_F16 || a.c_type == DT_BF16;
     const bool m64x32 = a.M > 32 && a.N > 7168 && a.N <= 8192;
+    const bool b_tr_rows = !a.trans_b && a.ldb % 16 == 0 && (uintptr_t)a.B % 16 == 0 && a.N % 4 == 0;
     if constexpr (ES == 1) {
         // with a workspace for the partials, the K split across workgroups as well where decode_splits (the int8
         // Matmul's rule) finds it faster: B [N, K] on the 32 x 32 tiles, B [K, N] (16-byte K rows) on 32 x 128 tiles
         const int splits = decode_splits(a.M, a.N, a.K, a.trans_b);
-        const bool b_tr = !a.trans_b && a.ldb % 16 == 0 && (uintptr_t)a.B % 16 == 0 && a.N % 4 == 0;
+        const bool b_tr = b_tr_rows;
         if ((a.trans_b || b_tr) && splits > 1 && c_wide && a.atomic == C_STORE && a.ws &&
             a.ws_bytes >= decode_split_ws_bytes(a.M, a.N, a.K, a.trans_b) &&
             ((a.M + 63) / 64) * ((a.N + 127) / 128) >= 32) {
@@ -385,6 +386,12 @@ static hipError_t launch_f8_fmt(const GemmF8Args& a, bool ua, hipStream_t st)
                                 : launch_f8_tiled<32, 32, 1, 1, 4, false, 64, FMT, false, 4, true>(a, st);
     }
     if constexpr (ES == 1) {
+        // f32 C combined by enAtomic: what a CU exchanges per microsecond bounds it, so more, smaller tiles (M = 64, N = 256,
+        // K = 512: 14 us, 64 x 128 tiles 24)
+        if (a.atomic != C_STORE && a.c_type == DT_F32 && !(a.M >= 1024 && a.N >= 1024)) {
+            if (a.trans_b) return launch_f8_tiled<64, 64, 2, 2, 4, true, 64, FMT>(a, st);
+            if (b_tr_rows && a.K % 16 == 0) return launch_f8_tiled<64, 64, 2, 2, 4, false, 64, FMT, false, 1, true>(a, st);
+        }
         return launch_gemm_f8_pipe(a, st);
     } else {  // (the bf16 operands of a hifloat8 Matmul are always K-contiguous)
         const bool big = a.M >= 1024 && a.N >= 1024;

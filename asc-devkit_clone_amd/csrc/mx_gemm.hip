@@ -412,7 +412,8 @@ hipError_t launch_mx_gemm(const MxGemmArgs& a, hipStream_t st)
         // above decode size: the pipelined tiles, where they are more than half the CUs; with fewer, twice as many 64 x 64
         // tiles (K = 4096, N = 4096, M = 128: 12.1 against 12.7 us; K = 8192, N = 1024, M = 100: 17.0 against 19.0; at
         // K = 384, N = 2048, M = 1024, 256 tiles, 16.5 against 9.2)
-        if (((a.M + 63) / 64) * ((a.N + 127) / 128) <= 128)
+        // (f32 C combined by enAtomic is bound by the exchanges of a CU: more, smaller tiles there too)
+        if (((a.M + 63) / 64) * ((a.N + 127) / 128) <= 128 || (a.atomic != C_STORE && a.c_type == DT_F32 && !big))
             return launch_mx_tiled<64, 64, 2, 2, 4, 64, OP_MXFP4, 0>(a, st);
         return launch_mx_fp4_pipe(a, st);
     }

@@ -193,3 +193,92 @@ def test_atomic_ignored_for_uint8_and_refused_for_int8(ascq_gpu, oracle):
         mm8.IterateAll(c8, ascq_gpu.ATOMIC_ADD)
     with pytest.raises(ascq_gpu.AscqError, match="enAtomic"):
         mm8.IterateAll(c8, 4)
+
+
+# (M, N, K) of each pipelined tile shape, odd N (rows of 16-bit C start on either half of a word) and partial last tiles
+TILE_SHAPES = [(3353, 537, 1040), (4127, 933, 416), (1607, 3737, 528), (3457, 1733, 64), (3273, 1817, 144), (3301, 3805, 80)]
+
+
+@pytest.mark.parametrize("fp8,c_type", [(False, O.INT32), (False, O.F16), (False, O.BF16), (True, O.F32), (True, O.BF16)])
+@pytest.mark.parametrize("shape", TILE_SHAPES)
+def test_atomic_pipelined_tiles(ascq_gpu, oracle, fp8, c_type, shape):
+    """Every tile shape of the int8 and fp8 Matmul (128 x 128 .. 256 x 256: the accumulators go through LDS in one, two or
+    four chunks); neighbouring tiles and rows share 32-bit words of a 16-bit C"""
+    M, N, K = shape
+    g = torch.Generator().manual_seed(M + N + c_type)
+    A, B = torch.randint(-8, 9, (M, K), generator=g), torch.randint(-8, 9, (N, K), generator=g)
+    if fp8:
+        mm = ascq_gpu.Matmul(ascq_gpu.FP8_E4M3, ascq_gpu.FP8_E4M3, c_type, ascq_gpu.F32)
+        a, b = A.float().to(torch.float8_e4m3fn).cuda(), B.float().to(torch.float8_e4m3fn).cuda()
+        mm.SetBias(torch.randn(N, generator=g).cuda())
+    else:
+        mm = ascq_gpu.Matmul(ascq_gpu.INT8, ascq_gpu.INT8, c_type, ascq_gpu.INT32)
+        a, b = A.to(torch.int8).cuda(), B.to(torch.int8).cuda()
+        mm.SetBias(torch.randint(-1000, 1000, (N,), generator=g, dtype=torch.int32).cuda())
+    mm.SetOrgShape(M, N, K)
+    mm.SetTensorA(a)
+    mm.SetTensorB(b, True)
+    if c_type not in (O.INT32, O.F32):
+        mm.SetQuantVector(_dev(_quant_words(seeded(N), N).view(np.int64)))
+    _check(ascq_gpu, mm, c_type, M, N, seed=M + c_type, ops=(1, 2) if M * N < 4e6 else (1,))
+    mm.End()
+
+
+@pytest.mark.parametrize("shape", [(3713, 3216, 512), (3585, 1040, 128), (100, 400, 256)])
+def test_atomic_weight_only_tiles(ascq_gpu, oracle, shape):
+    """The weight-only tiles 256 x 192 (four chunks), 128 x 128 and a ring size"""
+    from test_gpu_gemv import make_weights
+
+    M, N, K = shape
+    rng = seeded(M)
+    w, scale, offset = make_weights(rng, K, N, O.INT4, 64)
+    mm = ascq_gpu.Matmul(ascq_gpu.F16, ascq_gpu.INT4, ascq_gpu.F16)
+    mm.SetOrgShape(M, N, K)
+    mm.SetTensorA(_dev(rng.standard_normal((M, K)).astype(np.float16)))
+    mm.SetTensorB(_dev(w))
+    mm.SetAntiQuantVector(_dev(offset), _dev(scale), 64)
+    _check(ascq_gpu, mm, O.F16, M, N, seed=M, ops=(1,))
+    mm.End()
+
+
+def test_atomic_calls_compose(ascq_gpu, oracle):
+    """Calls on two streams into one C of odd width (their words meet): every element gets each addition once"""
+    M, N, K, calls = 70, 131, 256, 6
+    one = torch.ones((M, K), dtype=torch.int8, device="cuda")
+    for c_type, dt in ((O.F16, torch.float16), (O.BF16, torch.bfloat16)):
+        mms = []
+        for _ in range(2):
+            mm = ascq_gpu.Matmul(ascq_gpu.INT8, ascq_gpu.INT8, c_type, ascq_gpu.INT32)
+            mm.SetOrgShape(M, N, K)
+            mm.SetTensorA(one)
+            mm.SetTensorB(torch.ones((N, K), dtype=torch.int8, device="cuda"), True)
+            mm.SetQuantScalar(int(np.float32(2.0 ** -8).view(np.uint32)))  # K ones x 2^-8 = 1
+            mms.append(mm)
+        c = torch.zeros((M, N), dtype=dt, device="cuda")
+        streams = [torch.cuda.Stream() for _ in mms]
+        torch.cuda.synchronize()
+        for _ in range(calls):
+            for mm, s in zip(mms, streams):
+                mm.IterateAll(c, ascq_gpu.ATOMIC_ADD, stream=s)
+        torch.cuda.synchronize()
+        assert bool((c == 2 * calls).all())
+
+
+@pytest.mark.parametrize("shape", [(3457, 1733, 64), (3301, 3805, 80), (200, 300, 256)])
+def test_fp8_c_on_pipelined_tiles(ascq_gpu, shape):
+    """A 1-byte C (the rolled epilogue) on two- and four-chunk tiles: e4m3 of exact sums x 2^-6"""
+    M, N, K = shape
+    g = torch.Generator().manual_seed(N)
+    A, B = torch.randint(-8, 9, (M, K), generator=g).float(), torch.randint(-8, 9, (N, K), generator=g).float()
+    mm = ascq_gpu.Matmul(ascq_gpu.FP8_E4M3, ascq_gpu.FP8_E4M3, ascq_gpu.FP8_E4M3)
+    mm.SetOrgShape(M, N, K)
+    mm.SetQuantScalar(int(np.float32(2.0 ** -6).view(np.uint32)))
+    mm.SetTensorA(A.to(torch.float8_e4m3fn).cuda())
+    mm.SetTensorB(B.to(torch.float8_e4m3fn).cuda(), True)
+    out = torch.zeros(M * N + 16, dtype=torch.float8_e4m3fn, device="cuda")
+    mm.IterateAll(out)
+    want = (A @ B.t() * 2.0 ** -6).clamp(-448, 448).to(torch.float8_e4m3fn)
+    got = out.view(torch.uint8).cpu()
+    assert not bool(got[M * N:].any())
+    same = (got[:M * N].view(M, N) & 0x7F) == (want.view(torch.uint8) & 0x7F)
+    assert bool(same.all()) and bool(((out[:M * N].view(M, N).float().cpu() == want.float())).all())
