@@ -128,6 +128,18 @@ __device__ __forceinline__ void stage_barrier()
     __builtin_amdgcn_sched_barrier(0);
 }
 
+// B [K, N] with long K and few tiles: 64 x 64 tiles on 64-row stages instead of the pipelined 64 x 128 ones, which take
+// 128 bytes of 128 K rows per stage and slow down where the row pitch is a multiple of 1024 (K = 16400, M = 1: N = 4608
+// 43 us, N = 5120 79; int8 and fp8 alike).  M = 1 / 64 / 128, 64 x 64 against pipelined, K = 8320: N = 5120 26 / 31 / 30
+// against 41 / 42 / 39, N = 8192 26 / 28 / 28 against 29 / 30 / 30, N = 2560 25 / 26 / 27 against 24 / 27 / 29; N = 1024,
+// M = 512 27 against 33; K = 16400, N = 1024, M = 256 50 against 61.  Not below: N = 2048, M = 128 26 against 24 (fp8 22), K = 6160, N = 4096 20 against 18; not
+// above 256 tiles: N = 9216, M = 128 49 against 37.
+inline bool few_long_kn(int64_t M, int64_t N, int64_t K)
+{
+    const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
+    return tiles <= 256 && ((K >= 6144 && N >= 4608) || (K >= 8192 && (N >= 2560 || tiles >= 128)) || (K >= 12288 && tiles >= 64));
+}
+
 // XCD-aware tile order: consecutive workgroup ids go to different XCDs; XCD x gets the ids [x*per, (x+1)*per)
 // of a grouped (GROUP_M tile rows at a time) raster, so the tiles one XCD runs together share A rows / B cols.
 __device__ __forceinline__ void tile_coords(int pid, int tiles_m, int tiles_n, int& tm, int& tn)

@@ -386,11 +386,17 @@ static hipError_t launch_f8_fmt(const GemmF8Args& a, bool ua, hipStream_t st)
                                 : launch_f8_tiled<32, 32, 1, 1, 4, false, 64, FMT, false, 4, true>(a, st);
     }
     if constexpr (ES == 1) {
-        // f32 C combined by enAtomic: what a CU exchanges per microsecond bounds it, so more, smaller tiles (M = 64, N = 256,
-        // K = 512: 14 us, 64 x 128 tiles 24)
-        if (a.atomic != C_STORE && a.c_type == DT_F32 && !(a.M >= 1024 && a.N >= 1024)) {
-            if (a.trans_b) return launch_f8_tiled<64, 64, 2, 2, 4, true, 64, FMT>(a, st);
-            if (b_tr_rows && a.K % 16 == 0) return launch_f8_tiled<64, 64, 2, 2, 4, false, 64, FMT, false, 1, true>(a, st);
+        // as the int8 Matmul, 64 x 64 tiles where 64 x 128 ones are too few: B [N, K], up to 128 of those, K to 4096
+        // (M = 64, N = 4096, K = 1040: 6.1 / 6.5 us) or rows off 128 bytes (M = 64, N = 8192, K = 4112: 14.3 / 17.8).
+        // f32 C combined by enAtomic: what a CU exchanges per microsecond bounds it, so more, smaller tiles (M = 64,
+        // N = 256, K = 512: 14 / 24)
+        if (!(a.M >= 1024 && a.N >= 1024)) {
+            const int64_t tiles = ((a.M + 63) / 64) * ((a.N + 127) / 128);
+            const bool f32_atomic = a.atomic != C_STORE && a.c_type == DT_F32;
+            if (a.trans_b && (f32_atomic || (a.atomic == C_STORE && tiles <= 128 && (a.K <= 4096 || a.K % 128 != 0))))
+                return launch_f8_tiled<64, 64, 2, 2, 4, true, 64, FMT>(a, st);
+            if (b_tr_rows && a.K % 16 == 0 && (f32_atomic || (a.atomic == C_STORE && few_long_kn(a.M, a.N, a.K))))
+                return launch_f8_tiled<64, 64, 2, 2, 4, false, 64, FMT, false, 1, true>(a, st);
         }
         return launch_gemm_f8_pipe(a, st);
     } else {  // (the bf16 operands of a hifloat8 Matmul are always K-contiguous)

@@ -430,6 +430,21 @@ static hipError_t launch_i8_split(GemmI8Args a, hipStream_t st)
     return hipGetLastError();
 }
 
+// Calls whose smallest pipelined tiles (64 x 128, stages of 128 K bytes) are too few or too short for them run 64 x 64
+// tiles (32 x 32: `tiny`) on 64-byte stages.  B [N, K], us against the pipelined tiles: up to 128 of those, K to 4096
+// (M = 64, N = 4096, K = 528: 4.7 / 5.7; M = 256, N = 1024, K = 4096: 12.3 / 12.3; above, 4 to 8 % slower) or rows off
+// 128 bytes (M = 64, N = 8192, K = 4112: 14.0 / 17.8); up to 192, K to 1040 (M = 128, N = 11008, K = 528: 5.6 / 6.3);
+// any number, K to 384 (M = 256, N = 11008, K = 272: 6.0 / 7.2).  B [K, N]: `tiny`, K to 1040 (M = N = 256, K = 528:
+// 5.0 / 5.5) or from 10240 on with N >= 2048 (M = 64, N = 2048 / 3072, K = 16400: 51 / 51 against 62 / 68).  int32 C combined by enAtomic: up to 16 rows and K to 1024 (M = 1, N = 1024, K = 512: 4.9 / 6.0).
+static bool i8_few(const GemmI8Args& a, bool tiny)
+{
+    if (a.M >= 1024 && a.N >= 1024) return false;
+    if (a.atomic != C_STORE) return a.epi == EPI_I32 && a.M <= 16 && a.K <= 1024;
+    if (!a.trans_b) return tiny && (a.K <= 1040 || (a.K >= 10240 && a.N >= 2048));
+    const int64_t tiles = ((a.M + 63) / 64) * ((a.N + 127) / 128);
+    return a.K <= 384 || (tiles <= 192 && a.K <= 1040) || (tiles <= 128 && (a.K <= 4096 || a.K % 128 != 0));
+}
+
 hipError_t launch_gemm_i8(const GemmI8Args& a, hipStream_t st)
 {
     const bool a_ok = !a.trans_a && a.lda % 16 == 0 && ((uintptr_t)a.A % 16 == 0) && a.lda * a.M < (1ll << 31);
@@ -478,6 +493,13 @@ hipError_t launch_gemm_i8(const GemmI8Args& a, hipStream_t st)
             return a.N >= 10240 ? launch_tiled<32, 64, 1, 1, 4, false, 64, true, 4>(a, st)
                    : m64x32   ? launch_tiled<64, 32, 1, 1, 4, false, 64, true, 4>(a, st)
                                 : launch_tiled<32, 32, 1, 1, 4, false, 64, true, 4>(a, st);
+        const bool b_tr = !a.trans_b && a.ldb % 16 == 0 && (uintptr_t)a.B % 16 == 0 && a.N % 4 == 0 && a.K % 16 == 0;
+        if (i8_few(a, tiny)) {
+            if (a.trans_b) return tiny ? launch_tiled<32, 32, 1, 1, 4, true>(a, st) : launch_tiled<64, 64, 2, 2, 4, true>(a, st);
+            if (tiny && b_tr) return launch_tiled<32, 32, 1, 1, 4, false, 64, true>(a, st);
+        }
+        if (b_tr && a.atomic == C_STORE && few_long_kn(a.M, a.N, a.K))
+            return launch_tiled<64, 64, 2, 2, 4, false, 64, true>(a, st);
         return launch_gemm_i8_pipe(a, st);
     }
     // K not a multiple of 16, or operands / leading dimensions not 16-byte (A, K-contiguous B) or 4-byte ([K, N] B)

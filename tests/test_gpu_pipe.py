@@ -35,11 +35,23 @@ def _bits(t):
 
 
 # odd N (odd pitches of C, a [K, N] B packed), and K of every remainder class of a chunk (operands packed): few rows too
+# aligned calls with few tiles or few stages, on the 32 x 32 and 64 x 64 tiles (which of the two layouts: in the comments)
+FEW = [
+    (70, 528, 528),       # both: 32 x 32 (int8); 64 x 64 (fp8, [N, K])
+    (70, 4112, 1040),     # [N, K]: 64 x 64, 66 tiles of 64 x 128
+    (130, 8000, 528),     # [N, K]: 64 x 64, 189 of them (int8)
+    (300, 6032, 272),     # [N, K]: 64 x 64, 240 of them (int8)
+    (65, 1040, 4112),     # [N, K]: 64 x 64, rows off 128 bytes
+    (40, 4624, 6160),     # [K, N]: 64 x 64 (few_long_kn), K its least
+    (130, 2576, 8208),    # [K, N]: 64 x 64
+    (33, 2064, 10256),    # [K, N]: 32 x 32 (int8)
+    (300, 848, 12304),    # [K, N]: 64 x 64
+]
 RAGGED = [(130, 1001, 2048), (300, 5003, 1040), (130, 1004, 2047), (1, 1030, 1009), (20, 515, 77), (33, 601, 1), (70, 130, 4095)]
 
 
 @pytest.mark.parametrize("trans_b", [False, True])
-@pytest.mark.parametrize("M,N,K", SHAPES + RAGGED)
+@pytest.mark.parametrize("M,N,K", SHAPES + RAGGED + FEW)
 def test_int8_pipe(ascq_gpu, oracle, M, N, K, trans_b):
     rng = seeded(M + N + K + trans_b)
     A = rng.integers(-128, 128, (M, K), dtype=np.int8)
@@ -71,7 +83,7 @@ def test_int8_pipe(ascq_gpu, oracle, M, N, K, trans_b):
 
 
 @pytest.mark.parametrize("trans_b", [False, True])
-@pytest.mark.parametrize("M,N,K", SHAPES + RAGGED)
+@pytest.mark.parametrize("M,N,K", SHAPES + RAGGED + FEW)
 def test_fp8_pipe(ascq_gpu, M, N, K, trans_b):
     g = torch.Generator().manual_seed(M + N + K + trans_b)
     A = torch.randint(-4, 5, (M, K), generator=g)
