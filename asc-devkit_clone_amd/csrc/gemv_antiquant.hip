@@ -1382,8 +1382,11 @@ hipError_t launch_antiquant_matmul(uint16_t* y, const uint16_t* x, const void* w
     // in one round, 0.54 in up to 320 blocks, 0.35 a round with two k-split waves; 128-row blocks 0.65 a round to 6
     // strips, 0.87 at 12.  Ring against tiles: 512 x 11008 x 4096 57 / 61 us, 256 x 4096 x 4096 21 / 39, 1024 x 11008 x
     // 4096 109 / 86, 2048 x 11008 x 4096 222 / 177, 1024 x 8192 x 8192 int8 303 / 147, 512 x 4096 x 11008 122 / 100.
-    // Groups of 64 (256 x 14336 x 4096, int8): 48 us, in 64-row passes of the kernels below 99.
-    if (M > 64 && K % KT == 0) {
+    // Groups of 64 (256 x 14336 x 4096, int8): 48 us, in 64-row passes of the kernels below 99
+    // ... but two passes for at most 96 rows, 128 where N leaves a pass in one round (96 x 4096 x 4096, int4, g = 64: 27 / 39
+    // us; 128 x 4096 x 11008: 84 / 98; 128 x 14336 x 4096: 46 / 40).
+    const bool passes = !cols_ok && M <= (N <= 8192 ? 128 : 96);
+    if (M > 64 && K % KT == 0 && !passes) {
         const int64_t rb64 = (M + 63) / 64, rb128 = (M + 127) / 128;
         auto blocks = [&](int smax, int64_t rb) { return aq_blocks(NBT, smax, (int)(rb < 256 ? 256 / rb : 1)); };
         const int c64 = blocks(6, rb64), c128 = blocks(12, rb128);

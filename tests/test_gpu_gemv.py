@@ -210,7 +210,11 @@ def test_prefill_gemm(ascq_gpu, oracle, w_type, with_offset, M, K, N, group):
 
 @pytest.mark.parametrize("w_type,with_offset", [("int4", True), ("int8", False), ("int4", False), ("int8", True)])
 @pytest.mark.parametrize("M,K,N,group", [
-    (65, 128, 16, 64),        # 64 x 128 tiles: two stages, one strip, one row in the second tile
+    (65, 128, 16, 64),        # two 64-row passes (up to 128 rows at this N), one row in the second
+    (128, 1152, 528, 64),     # two whole passes
+    (96, 384, 8208, 64),      # passes at wide N, up to 96 rows
+    (97, 384, 8208, 64),      # 64 x 128 tiles
+    (193, 128, 16, 64),       # 64 x 128 tiles: two stages, one strip, one row in the last tile
     (129, 640, 4112, 64),     # 64 x 128: one row and one strip in the last tiles
     (577, 2560, 4112, 64),    # 128 x 128
     (383, 4096, 11008, 64),   # 128 x 192: 64 columns in the last tile
@@ -219,7 +223,7 @@ def test_prefill_gemm(ascq_gpu, oracle, w_type, with_offset, M, K, N, group):
     (600, 2944, 4096, 2944),  # one group over all of K, 23 packed tiles
 ])
 def test_prefill_tiles(ascq_gpu, oracle, w_type, with_offset, M, K, N, group):
-    """M > 64 on the pipelined tiles of aq_gemm.hip (groups of 64 always; the others where they beat the ring kernel):
+    """M > 64 on the pipelined tiles of aq_gemm.hip (groups of 64 above 96 or 128 rows; the others where they beat the ring kernel):
     every output of sampled rows, both sides of each 64-row boundary among them, within the bound of check_close"""
     rng = seeded(M + K + N + group + with_offset)
     code = O.INT8 if w_type == "int8" else O.INT4
