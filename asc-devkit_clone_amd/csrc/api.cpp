@@ -455,10 +455,13 @@ ascq_status pack_byte_operands(ascq_matmul_s* h, hipStream_t st, int64_t m, int6
 {
     const PackPlan p = pack_plan(fp8, o, m, n, *k);
     if (!p.a && !p.b) return ASCQ_OK;
-    // (the smallest calls keep the element-wise kernel, which needs no workspace and which ASCQ_LOG names, though the
-    // copy and the GEMM would be faster: 32 x 32 x 40 in 17.1 us, 40 x 40 x 41 in 9.3)
-    if (fp8 && !o.trans_b && m * n * *k <= 32 * 32 * 40) return ASCQ_OK;
     if (h->no_alloc) return ASCQ_OK;
+    // the any-alignment tiles take 18 us per 1000 K and round of 128 tiles of 128 x 128, the copy and the aligned ones
+    // about 7, but two launches: K below 192 is faster in one (1000 x 1000 x 100: 5.8 / 7.3 us; at K = 200 8.0 / 7.9) up
+    // to some rounds.  fp8 with B [K, N] would run element by element (32 x 32 x 40: 17.1 / 6.5)
+    const int64_t rounds = (((m + 127) / 128) * ((n + 127) / 128) + 127) / 128;
+    const bool elementwise = fp8 && !o.trans_b;
+    if (!elementwise && *k < 192 && rounds <= 4) return ASCQ_OK;
     const size_t need = p.a_bytes + p.b_bytes;
     uint8_t* pa = nullptr;
     if (h->ws && !h->ws_owned) {
@@ -467,10 +470,7 @@ ascq_status pack_byte_operands(ascq_matmul_s* h, hipStream_t st, int64_t m, int6
         pa = (uint8_t*)h->ws + base;
         o.ws_end = base;
     } else {
-        // the any-alignment tiles take 18 us per 1000 K and round of 128 tiles of 128 x 128, the packed form about 7; fp8
-        // with B [K, N] would run element by element
-        const int64_t rounds = (((m + 127) / 128) * ((n + 127) / 128) + 127) / 128;
-        pa = pack_room(h, st, need, fp8 && !o.trans_b ? 1e9f : 0.011f * (float)*k * (float)rounds);
+        pa = pack_room(h, st, need, elementwise ? 1e9f : 0.011f * (float)*k * (float)rounds);
         if (!pa) return ASCQ_OK;
     }
     uint8_t* pb = pa + p.a_bytes;

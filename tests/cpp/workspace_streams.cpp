@@ -68,6 +68,27 @@ int main()
         }
         ascq_matmul_destroy(h);
     }
+    // a short K is not packed while the any-alignment tiles take few rounds; what would run element by element always is
+    const struct {
+        int64_t m, n, k;
+        int fp8, trans_b, packed;
+    } small[] = {{32, 32, 40, 0, 1, 0},    {32, 32, 40, 0, 0, 0},   {300, 1000, 190, 1, 1, 0}, {300, 1000, 200, 1, 1, 1},
+                 {2000, 4000, 100, 0, 1, 0}, {4000, 4000, 100, 0, 1, 1}, {32, 32, 40, 1, 0, 1},    {1, 64, 17, 1, 0, 1}};
+    for (const auto& c : small) {
+        ascq_matmul_t h = nullptr;
+        ascq_matmul_types t{ASCQ_DT_INT8, ASCQ_DT_INT8, ASCQ_DT_INT32, 0, 0, 0};
+        if (c.fp8) t.a_type = t.b_type = ASCQ_DT_FP8_E4M3, t.c_type = ASCQ_DT_F32;
+        if (ascq_matmul_create(&t, &h) != ASCQ_OK) return 1;
+        ascq_matmul_set_org_shape(h, c.m, c.n, c.k);
+        ascq_matmul_set_tensor_a(h, (void*)0x10000004, 0);
+        ascq_matmul_set_tensor_b(h, (void*)0x20000000, c.trans_b);
+        for (int call = 0; call < 2; ++call) {
+            used.clear();
+            EXPECT(ascq_matmul_iterate_all(h, (void*)0x30000000, 0, nullptr) == ASCQ_OK);
+        }
+        EXPECT(!used.empty() == (c.packed != 0));
+        ascq_matmul_destroy(h);
+    }
     std::printf("%d failure(s)\n", failures);
     return failures != 0;
 }

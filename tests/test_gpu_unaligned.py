@@ -161,9 +161,10 @@ ascq.quant_group_matmul(dev(x), dev(np.ones(64, np.float32)), dev(w), dev(np.one
                         dev(np.array([0, 30, 64], np.int64)), 0, False, torch.bfloat16)
 torch.cuda.synchronize()
 print("step group done", file=sys.stderr, flush=True)
-# fp8 Matmul with B given [K, N] and K = 40: the generic kernel
+# fp8 Matmul with B given [K, N], K = 40 and a workspace without room to pack the operands: the generic kernel
 mm = ascq.Matmul(ascq.FP8_E4M3, ascq.FP8_E4M3, ascq.F32)
 mm.SetOrgShape(32, 32, 40)
+mm.SetWorkspace(dev(np.zeros(16, np.uint8)), 16)
 mm.SetTensorA(dev(np.full((32, 40), 0x38, np.uint8)))
 mm.SetTensorB(dev(np.full((40, 32), 0x38, np.uint8)), False)
 c = torch.empty((32, 32), dtype=torch.float32, device="cuda")
