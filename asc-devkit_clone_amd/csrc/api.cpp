@@ -199,16 +199,6 @@ int64_t hif8_k_pad(int64_t K) { return (K + 7) / 8 * 8; }
 
 size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// int8 / fp8 B given [K, N] is read in place, but ascq_matmul_workspace_size keeps the N K bytes that it has always
-// reported at these sizes (earlier kernels transposed B there), and a handle holds them as before: callers' checks,
-// buffers and the scratch limit of the allocation-free form rely on the figure.
-bool bytes_reserves_b(const ascq_matmul_s* h)
-{
-    if (h->ty.b_format == ASCQ_FORMAT_NZ) return false;
-    if (kind_of(h->ty) == K_INT8 && h->N % 16 == 0 && (h->M < 1024 || h->N < 1024)) return false;
-    return !h->trans_b && h->M >= 512 && h->N % 16 == 0 && h->K % 16 == 0;
-}
-
 // int8 / fp8 A given [K, M] (isTransA): the whole org A is transposed to [M, K] in the workspace (the tiled
 // GEMM reads K-contiguous A rows only)
 bool bytes_transposes_a(const ascq_matmul_s* h) { return h->trans_a != 0; }
@@ -227,7 +217,6 @@ size_t bytes_operands(const ascq_matmul_s* h)
 // ... then, for decode-sized batches, the accumulators of the K split across workgroups
 size_t bytes_workspace(const ascq_matmul_s* h)
 {
-    if (bytes_reserves_b(h)) return align256((size_t)h->N * (size_t)h->K) + bytes_operands(h);  // (M >= 512: no split)
     const int tb = h->trans_b || bytes_nz_b(h);  // B as the GEMM sees it
     return bytes_operands(h) + align256(ascq::decode_split_ws_bytes(h->M, h->N, h->K, tb));
 }
@@ -307,7 +296,7 @@ ascq_status split_region(ascq_matmul_s* h, int64_t m, int64_t n, int64_t k, uint
     return ASCQ_OK;
 }
 
-// int8 / fp8 operands after the workspace transposes (bytes_transposes_a / _b): pointers, leading dimensions
+// int8 / fp8 operands after the copies to the workspace (bytes_transposes_a, bytes_nz_b) and the packing: pointers, leading dimensions
 // (org shape) and the layouts the GEMM sees
 struct ByteOperands {
     const uint8_t* A;
@@ -326,7 +315,7 @@ ascq_status prepare_byte_operands(ascq_matmul_s* h, hipStream_t st, ByteOperands
     o.trans_a = h->trans_a;
     o.trans_b = h->trans_b;
     const bool ta = bytes_transposes_a(h), nz = bytes_nz_b(h);
-    if (!ta && !nz && !bytes_reserves_b(h)) return ASCQ_OK;
+    if (!ta && !nz) return ASCQ_OK;
     ascq_status s = ensure_workspace(h);
     if (s != ASCQ_OK) return s;
     uint8_t* ws = (uint8_t*)h->ws;

@@ -700,7 +700,7 @@ def bench_fp8(torch, ascq, iters, trans_b=True):
     ms = _time_loop(torch, fn, iters, warmup=2)
     tf = 2 * M * N * K / (ms * 1e-3) / 1e12
     return dict(workload=f"fp8 e4m3 Matmul {M}x{N}x{K}, fp32 acc, per-channel QF322BF16_PRE -> bf16, B given "
-                         + ("[N,K] (isTransposeB)" if trans_b else "[K,N] (transposed into the workspace)"),
+                         + ("[N,K] (isTransposeB)" if trans_b else "[K,N]"),
                 ms=ms, value=tf, unit="TFLOPS", frac_of_peak=tf / FP8_PEAK_TFLOPS)
 
 

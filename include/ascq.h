@@ -153,7 +153,7 @@ uint64_t ascq_pack_quant_pre(float m1, int32_t offset9, int32_t sign_flag);
  *                               conversion pass into the workspace)
  *  fp8_e4m3|fp8_e5m2 (any mix), bf16|f32, f32 bias, with E8M0 scales -> MX-FP8 (matmul_mx.asc:90-244, bias
  *                               :99-116,199-201; K % 64 == 0)
- * int8 / fp8 A given [K, M] (isTransA) and a large [K, N] B are transposed into the workspace first.
+ * int8 / fp8 A given [K, M] (isTransA) is transposed into the workspace first; B [K, N] is read as it lies.
  * ------------------------------------------------------------------------------------------ */
 typedef struct ascq_matmul_s* ascq_matmul_t;
 
@@ -216,9 +216,14 @@ ascq_status ascq_matmul_set_antiquant_vector(ascq_matmul_t h, const void* offset
  * scaleA: [M, sK] (transpose: [sK/2, M, 2]); scaleB: [sK/2, N, 2] (transpose: [N, sK]); sK = ceil(K/64)*2. */
 ascq_status ascq_matmul_set_tensor_scale_a(ascq_matmul_t h, const uint8_t* scale_a, int32_t is_transpose_scale_a);
 ascq_status ascq_matmul_set_tensor_scale_b(ascq_matmul_t h, const uint8_t* scale_b, int32_t is_transpose_scale_b);
-/* Optional device workspace for handles that need one (int8 / fp8 with isTransA or a large [K,N] B; MX; hifloat8;
- * W4/W8 with ND B):
- * ascq_matmul_workspace_size() bytes.  Without it IterateAll allocates on first use. */
+/* Optional device workspace: ascq_matmul_workspace_size() bytes.  Handles that need one (int8 / fp8 with isTransA or an NZ
+ * B; int4; MX; hifloat8; W4/W8 with ND B) allocate it on first use when none is set.  Two parts of the figure are optional,
+ * and a caller's workspace without them is accepted: the partials of the K split at decode-sized batches, and room to pack
+ * int8 / fp8 operands whose rows or pointers are off their alignment (16 bytes; a [K, N] B 4) or whose K is not a multiple
+ * of 16 -- it depends on the pointers and the single shape set when the size is asked for.  Without the room such calls run
+ * on slower any-alignment kernels.  A handle without a caller's workspace allocates room for packing itself, per stream
+ * (four at most; from the second call on where one call would not repay it), but neither under stream capture nor in
+ * ascq_matmul_iterate_all_noalloc: give a handle a workspace to have its captured calls packed. */
 ascq_status ascq_matmul_workspace_size(ascq_matmul_t h, size_t* bytes);
 ascq_status ascq_matmul_set_workspace(ascq_matmul_t h, void* workspace, size_t bytes);
 /* IterateAll(GlobalTensor<C>, enAtomic) (matmul.h:255-265; matmul_impl.h:119-137).  en_atomic (ATOMIC_ADD / MAX /
@@ -235,10 +240,11 @@ ascq_status ascq_matmul_set_workspace(ascq_matmul_t h, void* workspace, size_t b
 ascq_status ascq_matmul_iterate_all(ascq_matmul_t h, void* c, uint8_t en_atomic, void* stream);
 /* IterateAll that allocates nothing -- no counterpart in the reference; for callers that cannot allocate device
  * memory (code under HIP graph capture, serving loops, harnesses that forbid hipMalloc).  Same arguments and
- * results as ascq_matmul_iterate_all, but a handle that needs a workspace (ascq_matmul_workspace_size > 0) uses
+ * results as ascq_matmul_iterate_all, but a handle that needs a workspace (or keeps K-split partials) uses
  * the library's static per-device scratch of ASCQ_NOALLOC_SCRATCH_BYTES instead of its own workspace or a
- * hipMalloc; a handle needing more is rejected with ASCQ_E_UNSUPPORTED before anything is launched.  Every call
+ * hipMalloc; a handle needing more is rejected with ASCQ_E_UNSUPPORTED before anything is launched.  Every such call
  * on one device shares that device's scratch: calls that overlap on a device (other streams, other threads) race.
+ * Operands off their alignment are not packed there (see above).
  * Nothing of the scratch's previous contents is read. */
 #define ASCQ_NOALLOC_SCRATCH_BYTES ((size_t)64 << 20)
 ascq_status ascq_matmul_iterate_all_noalloc(ascq_matmul_t h, void* c, uint8_t en_atomic, void* stream);

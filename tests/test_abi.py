@@ -422,16 +422,20 @@ def test_nz_argument_checks():
 
 def test_noalloc_iterate_all_rejects_oversized_workspace():
     """ascq_matmul_iterate_all_noalloc refuses, before launching anything, a handle whose workspace exceeds the
-    static scratch (int8 [K, N] B of 8192 x 16384 needs 128 MiB to be transposed), and checks its arguments"""
+    static scratch (an int8 A given [K, M], 8192 x 16384, needs 128 MiB to be transposed), and checks its arguments; a large
+    [K, N] B is read in place and needs none"""
     L = ascq.lib()
     h = ctypes.c_void_p()
     d = ctypes.c_void_p(0x1000)
     t = ascq._MatmulTypes(ascq.INT8, ascq.INT8, ascq.INT32, 0, 0, 0)
     _err(L.ascq_matmul_create(ctypes.byref(t), ctypes.byref(h)), ascq.OK)
-    _err(L.ascq_matmul_set_org_shape(h, 1024, 16384, 8192), ascq.OK)
+    _err(L.ascq_matmul_set_org_shape(h, 16384, 16384, 8192), ascq.OK)
     _err(L.ascq_matmul_set_tensor_a(h, d, 0), ascq.OK)
     _err(L.ascq_matmul_set_tensor_b(h, d, 0), ascq.OK)
     ws = ctypes.c_size_t()
+    _err(L.ascq_matmul_workspace_size(h, ctypes.byref(ws)), ascq.OK)
+    assert ws.value == 0
+    _err(L.ascq_matmul_set_tensor_a(h, d, 1), ascq.OK)
     _err(L.ascq_matmul_workspace_size(h, ctypes.byref(ws)), ascq.OK)
     assert ws.value > (64 << 20)
     _err(L.ascq_matmul_iterate_all_noalloc(h, d, 0, None), ascq.E_UNSUPPORTED)

@@ -34,7 +34,7 @@ def _bits(t):
 
 @pytest.mark.parametrize("trans_b", [False, True])
 def test_int8_deqf16_8192_sampled(ascq_gpu, oracle, trans_b):
-    """A int8 [8192, 8192], B int8 [K, N] (the benchmark's layout, transposed into the workspace first) or [N, K],
+    """A int8 [8192, 8192], B int8 [K, N] (the benchmark's layout, read in place) or [N, K],
     int32 bias, per-channel QUANT_PRE words -> f16; sampled rows bit-exact against the oracle."""
     rng = seeded(81 + trans_b)
     A = rng.integers(-127, 128, (S, S), dtype=np.int8)

@@ -1,6 +1,6 @@
 """ascq_matmul_iterate_all_noalloc (IterateAll with the workspace taken from the library's static per-device
 scratch, allocating nothing) against ascq_matmul_iterate_all, bit-exact, on two calls in a row -- the second with a
-smaller problem -- for each kind of handle that uses a workspace: int8 with a [K, N] B transposed into it, int8 at
+smaller problem -- for each kind of handle that uses a workspace: int8 with an A given [K, M] transposed into it, int8 at
 decode-sized batches keeping K-split partials in it, MX-FP4
 with its scales rearranged (and a [K, N] B transposed) into it, and int4 operands unpacked into it.  The handle
 keeps its own workspace across the allocation-free calls.  A fresh handle that only calls the allocation-free entry
@@ -42,9 +42,8 @@ def _same(c1, c2):
     assert torch.equal(a, b)
 
 
-def test_noalloc_int8_kn_b(ascq_gpu, oracle):
-    """int8 x int8 -> f16 (VDEQF16), B given [K, N] with M, N >= 1024 (the 256 x 256 tile sizes): B is transposed
-    into the workspace (smaller [K, N] problems read it in place with LDS transpose reads)"""
+def test_noalloc_int8_km_a(ascq_gpu, oracle):
+    """int8 x int8 -> f16 (VDEQF16), A given [K, M]: transposed into the workspace (B [K, N] is read in place)"""
     ascq = ascq_gpu
     mm = ascq.Matmul(ascq.INT8, ascq.INT8, ascq.F16, ascq.INT32)
     for i, (M, N, K) in enumerate([(1024, 1024, 512), (1024, 1024, 256)]):
@@ -57,7 +56,7 @@ def test_noalloc_int8_kn_b(ascq_gpu, oracle):
         mm.SetOrgShape(M, N, K)
         assert mm.WorkspaceSize() > 0
         mm.SetQuantVector(_dev(words.view(np.int64)))
-        mm.SetTensorA(_dev(A))
+        mm.SetTensorA(_dev(A.T), True)
         mm.SetTensorB(_dev(B), False)
         mm.SetBias(_dev(bias))
         c1, c2 = _both(ascq, mm, (M, N), torch.float16)
@@ -131,8 +130,8 @@ def test_noalloc_int4(ascq_gpu, oracle):
         mm.End()
 
 
-def _int8_kn_handle(ascq, M, N, K, seed):
-    """an int8 -> f16 handle with B given [K, N] (M, N >= 1024: B is transposed into the workspace) and its inputs"""
+def _int8_km_handle(ascq, M, N, K, seed):
+    """an int8 -> f16 handle with A given [K, M] (transposed into the workspace) and its inputs"""
     rng = seeded(seed)
     A = rng.integers(-127, 128, (M, K), dtype=np.int8)
     B = rng.integers(-127, 128, (K, N), dtype=np.int8)
@@ -140,7 +139,7 @@ def _int8_kn_handle(ascq, M, N, K, seed):
     mm = ascq.Matmul(ascq.INT8, ascq.INT8, ascq.F16, 0)
     mm.SetOrgShape(M, N, K)
     mm.SetQuantVector(_dev(words.view(np.int64)))
-    mm.SetTensorA(_dev(A))
+    mm.SetTensorA(_dev(A.T), True)
     mm.SetTensorB(_dev(B), False)
     return mm, A, B, words
 
@@ -150,12 +149,12 @@ def test_noalloc_fresh_handle_allocates_nothing(ascq_gpu, oracle):
     memory does not move (a workspace of its own would take >= 8 MiB); the first IterateAll on the same handle then
     allocates that workspace -- so the handle had none of its own before"""
     ascq = ascq_gpu
-    M, N, K = 1024, 2048, 4096
-    warm, _, _, _ = _int8_kn_handle(ascq, M, N, K, 330)  # loads the kernels and the scratch address first
+    M, N, K = 2048, 1024, 4096
+    warm, _, _, _ = _int8_km_handle(ascq, M, N, K, 330)  # loads the kernels and the scratch address first
     c = torch.empty((M, N), dtype=torch.float16, device="cuda")
     warm.IterateAllNoAlloc(c)
     torch.cuda.synchronize()
-    mm, A, B, words = _int8_kn_handle(ascq, M, N, K, 331)
+    mm, A, B, words = _int8_km_handle(ascq, M, N, K, 331)
     need = mm.WorkspaceSize()
     assert need >= 8 << 20
     free0 = torch.cuda.mem_get_info()[0]
@@ -176,13 +175,13 @@ def test_noalloc_fresh_handle_allocates_nothing(ascq_gpu, oracle):
 
 
 def test_noalloc_graph_capture_replays(ascq_gpu, oracle):
-    """IterateAllNoAlloc captured in a HIP graph (the transpose of B into the scratch and the GEMM: kernel nodes only,
+    """IterateAllNoAlloc captured in a HIP graph (the transpose of A into the scratch and the GEMM: kernel nodes only,
     no memset, no allocation): every replay, with eager allocation-free calls of another handle on the same scratch
     between the replays, equals the eager call bit for bit"""
     ascq = ascq_gpu
     M, N, K = 1024, 1024, 512
-    mm, A, B, words = _int8_kn_handle(ascq, M, N, K, 340)
-    other, _, _, _ = _int8_kn_handle(ascq, M, N, 256, 341)
+    mm, A, B, words = _int8_km_handle(ascq, M, N, K, 340)
+    other, _, _, _ = _int8_km_handle(ascq, M, N, 256, 341)
     eager = torch.empty((M, N), dtype=torch.float16, device="cuda")
     mm.IterateAllNoAlloc(eager)
     junk = torch.empty_like(eager)
