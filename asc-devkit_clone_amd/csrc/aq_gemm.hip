@@ -34,7 +34,7 @@ struct NoCols {};
 template <int BM, int BN, int WM, int WN, int FMT>
 __global__ __launch_bounds__(WM * WN * 64, 2) void aq_pipe_kernel(AqGemmArgs p)
 {
-    using T = GemmPipe<BM, BN, WM, WN, 2, OP_AQ, FMT>;
+    using T = GemmPipe<BM, BN, WM, WN, OP_AQ, FMT>;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem_aq[];
     int tm, tn;
     pipe_tile((int)blockIdx.x, (int)((p.M + BM - 1) / BM), (int)((p.N + BN - 1) / BN), tm, tn);
@@ -72,7 +72,7 @@ static hipError_t launch_aq_pipe(const AqGemmArgs& a, bool int4, hipStream_t st)
     const unsigned tiles = ((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
     auto go = [&](auto F) -> hipError_t {
         constexpr int FMT = decltype(F)::value;
-        using T = GemmPipe<BM, BN, WM, WN, 2, OP_AQ, FMT>;
+        using T = GemmPipe<BM, BN, WM, WN, OP_AQ, FMT>;
         constexpr auto kern = aq_pipe_kernel<BM, BN, WM, WN, FMT>;
         const hipError_t e = ensure_dynamic_lds<kern>((int)T::LDS_BYTES);
         if (e != hipSuccess) return e;

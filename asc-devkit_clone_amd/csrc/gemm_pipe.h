@@ -1,5 +1,5 @@
 // gemm_pipe.h -- the half-tile pipelined MFMA main loop of the medium and large int8 / fp8 / MX Matmuls (gfx950),
-// for K-contiguous operands with 128-byte multiples of K.
+// and of the weight-only Matmul: A [M, K] K-contiguous, B [N, K] the same or (int8, fp8) [K, N].
 //
 // What bounds a large tile is the feed from L2 / HBM into LDS.  GemmCore's two-stage loop waits for a whole stage
 // (64 KiB at 256 x 256) that was requested less than one stage of MFMAs earlier, and reads each k-step's fragments
@@ -7,13 +7,13 @@
 // bytes of every tile row) is four halves -- the upper and lower half of A's rows and of B's -- and the loop runs in
 // phases of a quarter stage.  A phase multiplies one A half by one B half (a quadrant of the wave's accumulators)
 // out of registers, reads the half that the phase after next needs first from LDS into registers, and requests one
-// half from memory into the slot whose half went to registers in the phase before.  Requests so run 4 ST - 2 phases
-// ahead of their reads (1.5 stages of MFMAs at ST = 2: 96 KiB in flight of a 128 KiB ring), no MFMA waits for an LDS
+// half from memory into the slot whose half went to registers in the phase before.  Requests so run six phases
+// ahead of their reads (1.5 stages of MFMAs: 96 KiB in flight of a 128 KiB ring of two stages), no MFMA waits for an LDS
 // read issued in front of it, and a barrier has MFMA operands ready in registers on its far side.
 //
 // Order of the halves: H(4k) = A0(k), H(4k+1) = B0(k), H(4k+2) = B1(k), H(4k+3) = A1(k).  Phase t = 4k + p:
 //   p = 0: A0 B0, p = 1: A0 B1, p = 2: A1 B1, p = 3: A1 B0 -- each half is read once and consecutive phases share one;
-//   it reads H(t + 2) and requests H(t + 1 + 4 ST).  Each wave's quadrant rows are (half) x (wave row) x 32-row blocks.
+//   it reads H(t + 2) and requests H(t + 9).  Each wave's quadrant rows are (half) x (wave row) x 32-row blocks.
 // B0(k + 1) is read while B0(k) is still multiplied: it goes to the registers B1(k) has left, so the two register sets
 // of B swap roles from stage to stage.
 //
@@ -35,7 +35,9 @@
 // MX-FP4: the E8M0 scales arrive stage-major, the eight of (stage, row) -- k-step s, block g of it -- at byte 2 g + s of
 // its eight, and each stage's go to one of four scale slots, requested three stages ahead, one copy per wave and stage;
 // a lane reads the two bytes of block g of its row and the MFMA's op_sel picks the k-step's.
-// K is a multiple of 16 bytes: a lane's chunks at or past the end of K are not read (zeros), nor are a [K, N] B's rows.
+// K: a lane's 16-byte chunks at or past the end of K are not read (zeros), nor are a [K, N] B's rows.  So K of K-contiguous
+// operands is a multiple of 16 bytes; with B [K, N] K is any, A's bytes from K to the end of its chunk lying within its
+// pitch (int8: any, they meet zeros; fp8: zeros, a NaN would not vanish).
 //
 // Weight-only antiquant (OP_AQ): A is f16 (a stage is 64 k), B the packed int4 / int8 weight.  A wave loads one 16-column
 // strip of a half per stage into registers (packed codes, the columns' scale and offset), six phases ahead, dequantises
@@ -80,7 +82,7 @@ struct PipeArgs {
     rsrc4_t a, b;       // A: [rows][lda] bytes; B: [columns][ldb] bytes, or (BTR) [K][ldb]; ranges end with the operand
     uint32_t lda, ldb;
     uint32_t a0, b0;    // byte offsets of the tile origin
-    int32_t kbytes;     // K, a multiple of 16
+    int32_t kbytes;     // K
     // MX: the stage-major scales ([stage][rows][8]) of both operands through one resource: byte offsets of the tile's
     // first row in stage 0, and the stage strides
     rsrc4_t aux;
@@ -95,14 +97,14 @@ struct PipeArgs {
 // B operand of the weight-only antiquant pipeline; FMT bit 0: int4 codes (else int8), bit 1: with offsets
 constexpr int OP_AQ = 16;
 
-template <int BM, int BN, int WM, int WN, int ST, int OP, int FMT = 0, bool BTR = false>
+template <int BM, int BN, int WM, int WN, int OP, int FMT = 0, bool BTR = false>
 struct GemmPipe {
+    static constexpr int ST = 2;  // stages of the ring
     static constexpr bool IS_F8 = OP == OP_F8;
     static constexpr bool IS_MX = OP == OP_MXFP4;
     static constexpr bool IS_AQ = OP == OP_AQ;
     static_assert(OP == OP_I8 || OP == OP_F8 || ((IS_MX || IS_AQ) && !BTR),
                   "int8, fp8, MX-FP4 with a K-contiguous B, or f16 with a packed weight");
-    static_assert(!IS_AQ || ST == 2, "weight registers by stage parity");
     static constexpr int CBSZ = IS_MX ? F8F6F4_E2M1 : FMT & 7;  // f8f6f4 formats of A and B
     static constexpr int BLGP = IS_MX ? F8F6F4_E2M1 : (FMT >> 3) & 7;
     static constexpr int TBM = BM, TBN = BN, TWN = WN;
@@ -131,7 +133,6 @@ struct GemmPipe {
     static_assert(hm(0) % (8 * NW) == 0 && hm(1) % (8 * NW) == 0 && hn(0) % (8 * NW) == 0 && hn(1) % (8 * NW) == 0,
                   "copies split evenly over the waves");
     static_assert(NW == 4 || NW == 8, "the swizzles of a lane's copies agree");
-    static_assert(ST == 2 || ST == 4, "the stage loop is unrolled by the ring");
     static_assert(A_REG <= 65536 && B_REG <= 65536, "LDS read offsets are 16 bits");
     static_assert(LDS_BYTES <= 160 * 1024, "LDS");
     static_assert(SCA + SCB <= NW, "one scale copy per wave");
@@ -560,16 +561,8 @@ struct GemmPipe {
         for (; kt + ST <= nk; kt += ST) {
             stage(I0{}, kt);
             stage(I1{}, kt + 1);
-            if constexpr (ST == 4) {
-                stage(I2{}, kt + 2);
-                stage(I3{}, kt + 3);
-            }
         }
         if (kt < nk) stage(I0{}, kt);
-        if constexpr (ST == 4) {
-            if (kt + 1 < nk) stage(I1{}, kt + 1);
-            if (kt + 2 < nk) stage(I2{}, kt + 2);
-        }
         // drain: no copy may still target LDS when the caller reuses it or the wave ends
         wait_vmcnt<0>();
     }
@@ -581,7 +574,7 @@ struct GemmPipe {
 // beyond its stages when all write at once (`tail`: first stage's latency, epilogue).  A CU runs c = ceil(tiles / 256)
 // tiles, one after the other or side by side (128 x 128 two at a time, 64 x 128 three: no gain per tile, so the same
 // sum), a fraction of the CUs one fewer.  E.g. K = 4096, N = 11008 (start: this layout's tiles before these kernels):
-// M = 2048 192 x 256 in 78 us against 91 (256 x 256), 84 (128 x 256), 88 (128 x 128); M = 512 128 x 192 in 25.0 against
+// M = 2048 256 x 192 in 78 us against 91 (256 x 256), 84 (128 x 256), 88 (128 x 128); M = 512 128 x 192 in 25.0 against
 // 25.6 (128 x 256), 27.8 (128 x 128), 30.2 (64 x 128); M = 256 128 x 128 in 16.6 against 20.3 (128 x 192), 20.6
 // (64 x 128); M = 128 64 x 128 in 12.5 against 16.0 (128 x 128).
 enum PipeTile { PIPE_256x256, PIPE_192x256, PIPE_256x192, PIPE_128x256, PIPE_128x192, PIPE_128x128, PIPE_64x128, PIPE_TILES };

@@ -1,15 +1,16 @@
 // gemm_pipe_f8.hip -- the fp8 Matmul on the pipelined tiles of gemm_pipe.h: the GEMM and epilogues of gemm_f8.hip for
-// A [M, K] and B [N, K] with 16-byte-aligned rows and K a multiple of 128.
+// A [M, K] with 16-byte-aligned rows and B [N, K] the same (K a multiple of 16), or B [K, N] with 4-byte-aligned rows (any
+// K, A zero-padded to a multiple of 16).
 #include "common.h"
 #include "gemm_pipe.h"
 #include "launch.h"
 
 namespace ascq {
 
-template <int BM, int BN, int WM, int WN, int ST, int FMT, bool BTR>
+template <int BM, int BN, int WM, int WN, int FMT, bool BTR>
 __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_f8_pipe_kernel(GemmF8Args p)
 {
-    using T = GemmPipe<BM, BN, WM, WN, ST, OP_F8, FMT, BTR>;
+    using T = GemmPipe<BM, BN, WM, WN, OP_F8, FMT, BTR>;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem_f8[];
     int tm, tn;
     pipe_tile((int)blockIdx.x, (int)((p.M + BM - 1) / BM), (int)((p.N + BN - 1) / BN), tm, tn);
@@ -68,15 +69,15 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_f8_pipe_kernel(GemmF8Arg
         });
 }
 
-template <int BM, int BN, int WM, int WN, int ST, int FMT, bool BTR>
+template <int BM, int BN, int WM, int WN, int FMT, bool BTR>
 static hipError_t launch_f8_pipe(const GemmF8Args& a, hipStream_t st)
 {
-    using T = GemmPipe<BM, BN, WM, WN, ST, OP_F8, FMT, BTR>;
+    using T = GemmPipe<BM, BN, WM, WN, OP_F8, FMT, BTR>;
     constexpr int LDS = (int)T::LDS_BYTES + ColLds::BYTES;
     const int tiles = (int)(((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN));
-    const hipError_t e = ensure_dynamic_lds<gemm_f8_pipe_kernel<BM, BN, WM, WN, ST, FMT, BTR>>(LDS);
+    const hipError_t e = ensure_dynamic_lds<gemm_f8_pipe_kernel<BM, BN, WM, WN, FMT, BTR>>(LDS);
     if (e != hipSuccess) return e;
-    launch_k((gemm_f8_pipe_kernel<BM, BN, WM, WN, ST, FMT, BTR>), dim3(tiles), dim3(T::NT), LDS, st, a);
+    launch_k((gemm_f8_pipe_kernel<BM, BN, WM, WN, FMT, BTR>), dim3(tiles), dim3(T::NT), LDS, st, a);
     return hipGetLastError();
 }
 
@@ -87,13 +88,13 @@ static hipError_t launch_f8_pipe_layout(const GemmF8Args& a, hipStream_t st)
     // on 128 x 128)
     const bool f32_atomic = a.atomic != C_STORE && a.c_type == DT_F32 && !(a.M >= 1024 && a.N >= 1024);
     switch (f32_atomic ? PIPE_64x128 : pick_pipe_tile(a.M, a.N, a.K)) {
-    case PIPE_256x256: return launch_f8_pipe<256, 256, 2, 4, 2, FMT, BTR>(a, st);
-    case PIPE_192x256: return launch_f8_pipe<192, 256, 2, 4, 2, FMT, BTR>(a, st);
-    case PIPE_256x192: return launch_f8_pipe<256, 192, 4, 2, 2, FMT, BTR>(a, st);
-    case PIPE_128x256: return launch_f8_pipe<128, 256, 2, 4, 2, FMT, BTR>(a, st);
-    case PIPE_128x192: return launch_f8_pipe<128, 192, 4, 2, 2, FMT, BTR>(a, st);
-    case PIPE_128x128: return launch_f8_pipe<128, 128, 2, 2, 2, FMT, BTR>(a, st);
-    default: return launch_f8_pipe<64, 128, 2, 2, 2, FMT, BTR>(a, st);
+    case PIPE_256x256: return launch_f8_pipe<256, 256, 2, 4, FMT, BTR>(a, st);
+    case PIPE_192x256: return launch_f8_pipe<192, 256, 2, 4, FMT, BTR>(a, st);
+    case PIPE_256x192: return launch_f8_pipe<256, 192, 4, 2, FMT, BTR>(a, st);
+    case PIPE_128x256: return launch_f8_pipe<128, 256, 2, 4, FMT, BTR>(a, st);
+    case PIPE_128x192: return launch_f8_pipe<128, 192, 4, 2, FMT, BTR>(a, st);
+    case PIPE_128x128: return launch_f8_pipe<128, 128, 2, 2, FMT, BTR>(a, st);
+    default: return launch_f8_pipe<64, 128, 2, 2, FMT, BTR>(a, st);
     }
 }
 template <int FMT>

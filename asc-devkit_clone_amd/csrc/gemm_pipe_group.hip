@@ -13,7 +13,7 @@ namespace ascq {
 template <int BM, int BN, int WM, int WN, bool BTR>
 __global__ __launch_bounds__(WM * WN * 64, 2) void group_gemm_pipe_kernel(GroupGemmArgs p)
 {
-    using T = GemmPipe<BM, BN, WM, WN, 2, OP_I8, 0, BTR>;
+    using T = GemmPipe<BM, BN, WM, WN, OP_I8, 0, BTR>;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     GroupTile tile;
     if (!find_group_tile<T::NT, BM, BN>(p, tile)) return;
@@ -56,7 +56,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void group_gemm_pipe_kernel(GroupG
 template <int BM, int BN, int WM, int WN, bool BTR>
 static hipError_t launch_group_pipe_tile(const GroupGemmArgs& a, hipStream_t st)
 {
-    using T = GemmPipe<BM, BN, WM, WN, 2, OP_I8, 0, BTR>;
+    using T = GemmPipe<BM, BN, WM, WN, OP_I8, 0, BTR>;
     constexpr int LDS = (int)T::LDS_BYTES + 2048;
     const int64_t upper = ((a.M + BM - 1) / BM + a.G) * ((a.N + BN - 1) / BN);  // tiles, at most
     const hipError_t e = ensure_dynamic_lds<group_gemm_pipe_kernel<BM, BN, WM, WN, BTR>>(LDS);

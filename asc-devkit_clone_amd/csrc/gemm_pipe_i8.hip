@@ -7,10 +7,10 @@
 
 namespace ascq {
 
-template <int BM, int BN, int WM, int WN, int ST, bool BTR>
+template <int BM, int BN, int WM, int WN, bool BTR>
 __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_i8_pipe_kernel(GemmI8Args p)
 {
-    using T = GemmPipe<BM, BN, WM, WN, ST, OP_I8, 0, BTR>;
+    using T = GemmPipe<BM, BN, WM, WN, OP_I8, 0, BTR>;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     int tm, tn;
     pipe_tile((int)blockIdx.x, (int)((p.M + BM - 1) / BM), (int)((p.N + BN - 1) / BN), tm, tn);
@@ -69,15 +69,15 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_i8_pipe_kernel(GemmI8Arg
         });
 }
 
-template <int BM, int BN, int WM, int WN, int ST, bool BTR>
+template <int BM, int BN, int WM, int WN, bool BTR>
 static hipError_t launch_i8_pipe(const GemmI8Args& a, hipStream_t st)
 {
-    using T = GemmPipe<BM, BN, WM, WN, ST, OP_I8, 0, BTR>;
+    using T = GemmPipe<BM, BN, WM, WN, OP_I8, 0, BTR>;
     constexpr int LDS = (int)T::LDS_BYTES + ColLds::BYTES;
     const int tiles = (int)(((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN));
-    const hipError_t e = ensure_dynamic_lds<gemm_i8_pipe_kernel<BM, BN, WM, WN, ST, BTR>>(LDS);
+    const hipError_t e = ensure_dynamic_lds<gemm_i8_pipe_kernel<BM, BN, WM, WN, BTR>>(LDS);
     if (e != hipSuccess) return e;
-    launch_k((gemm_i8_pipe_kernel<BM, BN, WM, WN, ST, BTR>), dim3(tiles), dim3(T::NT), LDS, st, a);
+    launch_k((gemm_i8_pipe_kernel<BM, BN, WM, WN, BTR>), dim3(tiles), dim3(T::NT), LDS, st, a);
     return hipGetLastError();
 }
 
@@ -85,13 +85,13 @@ template <bool BTR>
 static hipError_t launch_i8_pipe_layout(const GemmI8Args& a, hipStream_t st)
 {
     switch (pick_pipe_tile(a.M, a.N, a.K)) {
-    case PIPE_256x256: return launch_i8_pipe<256, 256, 2, 4, 2, BTR>(a, st);
-    case PIPE_192x256: return launch_i8_pipe<192, 256, 2, 4, 2, BTR>(a, st);
-    case PIPE_256x192: return launch_i8_pipe<256, 192, 4, 2, 2, BTR>(a, st);
-    case PIPE_128x256: return launch_i8_pipe<128, 256, 2, 4, 2, BTR>(a, st);
-    case PIPE_128x192: return launch_i8_pipe<128, 192, 4, 2, 2, BTR>(a, st);
-    case PIPE_128x128: return launch_i8_pipe<128, 128, 2, 2, 2, BTR>(a, st);
-    default: return launch_i8_pipe<64, 128, 2, 2, 2, BTR>(a, st);
+    case PIPE_256x256: return launch_i8_pipe<256, 256, 2, 4, BTR>(a, st);
+    case PIPE_192x256: return launch_i8_pipe<192, 256, 2, 4, BTR>(a, st);
+    case PIPE_256x192: return launch_i8_pipe<256, 192, 4, 2, BTR>(a, st);
+    case PIPE_128x256: return launch_i8_pipe<128, 256, 2, 4, BTR>(a, st);
+    case PIPE_128x192: return launch_i8_pipe<128, 192, 4, 2, BTR>(a, st);
+    case PIPE_128x128: return launch_i8_pipe<128, 128, 2, 2, BTR>(a, st);
+    default: return launch_i8_pipe<64, 128, 2, 2, BTR>(a, st);
     }
 }
 

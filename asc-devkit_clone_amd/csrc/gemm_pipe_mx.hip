@@ -13,7 +13,7 @@ template <int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__(WM * WN * 64, 2) void mx_pipe_kernel(MxGemmArgs p, const uint8_t* __restrict__ sa_sm,
                                                                   const uint8_t* __restrict__ sb_sm)
 {
-    using T = GemmPipe<BM, BN, WM, WN, 2, OP_MXFP4>;
+    using T = GemmPipe<BM, BN, WM, WN, OP_MXFP4>;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem_mx[];
     int tm, tn;
     pipe_tile((int)blockIdx.x, (int)((p.M + BM - 1) / BM), (int)((p.N + BN - 1) / BN), tm, tn);
@@ -101,7 +101,7 @@ __global__ __launch_bounds__(256) void mx_pipe_scale_kernel(MxScaleJob ja, MxSca
 template <int BM, int BN, int WM, int WN>
 static hipError_t launch_mx_pipe(const MxGemmArgs& a, const uint8_t* sa, const uint8_t* sb, hipStream_t st)
 {
-    using T = GemmPipe<BM, BN, WM, WN, 2, OP_MXFP4>;
+    using T = GemmPipe<BM, BN, WM, WN, OP_MXFP4>;
     constexpr int LDS = (int)T::LDS_BYTES + 1024;  // (bias only)
     const int tiles = (int)(((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN));
     const hipError_t e = ensure_dynamic_lds<mx_pipe_kernel<BM, BN, WM, WN>>(LDS);

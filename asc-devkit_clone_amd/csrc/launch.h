@@ -219,8 +219,7 @@ size_t mx_decode_split_ws_bytes(int64_t M, int64_t N, int64_t K);
 size_t fp6_q_plane_bytes(int64_t R, int64_t K);
 hipError_t launch_fp4_to_fp6_planes(uint8_t* P, uint8_t* Q, const uint8_t* src, int64_t R, int64_t K, bool e1m2,
                                     hipStream_t st);
-// transpose.hip: int8 [rows, cols] -> [cols, rows]; fp4 [K, N] -> [N, K] tiled fast path (returns false when
-// the shape / alignment does not allow it)
+// transpose.hip:
 // rows of any byte alignment [rows][ld] -> zero-padded 16-byte-aligned rows [rows][cols rounded up to 16]; two jobs in
 // one launch, a job with a null dst is none; sources below 2^31 bytes
 struct PackRows {
@@ -229,6 +228,8 @@ struct PackRows {
     int64_t rows, cols, ld;
 };
 hipError_t launch_pack_rows(const PackRows& a, const PackRows& b, hipStream_t st);
+// int8 [rows, cols] -> [cols, rows]; fp4 [K, N] -> [N, K] tiled fast path (returns false when the shape / alignment does
+// not allow it)
 hipError_t launch_transpose_i8(uint8_t* dst, const uint8_t* src, int64_t rows, int64_t cols, hipStream_t st);
 bool fp4_transpose_tiled(uint8_t* dst, const uint8_t* src, int64_t K, int64_t N, hipStream_t st, hipError_t* err);
 size_t mx_scale_workspace_bytes(int64_t M, int64_t N, int64_t K);
