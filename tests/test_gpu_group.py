@@ -231,3 +231,32 @@ def test_group_matmul_store_fallback(ascq_gpu, oracle, N, shift, w_trans):
     np.testing.assert_array_equal(got[shift:shift + M * N].reshape(M, N), ref)
     three = np.float16(3.0).view(np.uint16)
     assert (got[:shift] == three).all() and (got[shift + M * N:] == three).all()
+
+
+# (M, N, K, G): the tile shape pick_pipe_tile chooses (half a row tile more per group)
+@pytest.mark.parametrize("w_trans", [False, True])
+@pytest.mark.parametrize("M,N,K,G", [
+    (4124, 396, 288, 3),    # 128 x 128
+    (4056, 908, 416, 3),    # 128 x 192
+    (1607, 3272, 528, 8),   # 128 x 256
+    (3428, 1668, 64, 3),    # 192 x 256
+    (4460, 1296, 64, 3),    # 256 x 192
+    (4321, 3320, 80, 3),    # 256 x 256
+])
+def test_group_pipelined_tiles(ascq_gpu, oracle, M, N, K, G, w_trans):
+    """Every tile shape of the group matmul above decode size, in both weight layouts: uneven groups that end inside a
+    tile, an empty one, rows of no group behind them, partial last column tiles, K tails"""
+    rng = seeded(M + N + K + w_trans)
+    cuts = np.sort(rng.integers(0, M - 7, G - 1))
+    if G > 3:
+        cuts[1] = cuts[0]  # an empty group
+    counts = np.diff(np.concatenate([[0], cuts, [M - 7]])).astype(np.int64)
+    x = rng.integers(-127, 128, (M, K), dtype=np.int8)
+    w = rng.integers(-127, 128, (G, N, K) if w_trans else (G, K, N), dtype=np.int8)
+    pts = rng.normal(0, 0.01, M).astype(np.float32)
+    scale = rng.normal(0, 0.01, (G, N)).astype(np.float32)
+    y = torch.full((M, N), 3.0, dtype=torch.bfloat16, device="cuda")
+    ascq_gpu.quant_group_matmul(_dev(x), _dev(pts), _dev(w), _dev(scale), _dev(counts), 1, w_trans, torch.bfloat16, out=y)
+    y0 = torch.full((M, N), 3.0, dtype=torch.bfloat16).view(torch.int16).numpy().view(np.uint16).copy()
+    ref = O.group_matmul(x, pts, w, scale, counts, 1, G, M, K, N, O.BF16, w_trans, y=y0)
+    np.testing.assert_array_equal(y.cpu().view(torch.int16).numpy().view(np.uint16), ref)

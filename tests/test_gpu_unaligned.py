@@ -1,6 +1,8 @@
-"""GPU parity: the any-alignment MFMA tiles (K not a multiple of 16, operands at any byte offset) of the quantized
-group matmul, the int8 Matmul and the fp8 Matmul, against the oracle; and ASCQ_LOG=1 naming the generic kernel a
-launch falls back to.
+"""GPU parity of operands off their alignment (K not a multiple of 16, operands at any byte offset) against the oracle: the
+any-alignment MFMA tiles of the quantized group matmul, and for the int8 and fp8 Matmul both forms -- packed to aligned
+rows first (room == "own": the handle's own, the call made twice, since a first call may go without), and the any-alignment
+tiles (room == "none": a caller's workspace too small for packing); and ASCQ_LOG=1 naming the generic kernel a launch falls
+back to.
 
 Each operand is placed at a byte offset inside a larger device buffer whose other bytes hold 0x5A, so bytes read past
 K, past a row or past the operand would enter the sums unless the kernel zeroes them.  int8: int32 accumulators,
@@ -65,7 +67,12 @@ def test_group_matmul_any_alignment(ascq_gpu, oracle, w_trans, K, N, x_off, w_of
     np.testing.assert_array_equal(_bits(y.cpu()), ref)
 
 
-def _int8_mm(ascq, A, B, bias, words, trans_a, trans_b, a_off, b_off, M, N, K, single=None):
+def _no_room(mm):
+    """a caller's workspace that holds what the call cannot do without, but no room to pack operands"""
+    mm.SetWorkspace(torch.empty(256, dtype=torch.uint8, device="cuda"), 256)
+
+
+def _int8_mm(ascq, A, B, bias, words, trans_a, trans_b, a_off, b_off, M, N, K, single=None, room="own"):
     mm = ascq.Matmul(ascq.INT8, ascq.INT8, ascq.F16, ascq.INT32)
     mm.SetOrgShape(M, N, K)
     if single is not None:
@@ -74,19 +81,28 @@ def _int8_mm(ascq, A, B, bias, words, trans_a, trans_b, a_off, b_off, M, N, K, s
     mm.SetTensorA(_dev_at(A, a_off), trans_a)
     mm.SetTensorB(_dev_at(B, b_off), trans_b)
     mm.SetBias(_dev(bias))
-    c = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
-    mm.IterateAll(c)
+    if room == "none":
+        _no_room(mm)
+    first = None
+    for _ in range(2 if room == "own" else 1):
+        c = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
+        mm.IterateAll(c)
+        torch.cuda.synchronize()
+        bits = _bits(c.cpu())
+        assert first is None or np.array_equal(first, bits)
+        first = bits
     mm.End()
-    torch.cuda.synchronize()
-    return _bits(c.cpu())
+    return first
 
 
+@pytest.mark.parametrize("room", ["own", "none"])
 @pytest.mark.parametrize("trans_b", [False, True])
 @pytest.mark.parametrize("shape,a_off,b_off", [((77, 200, 99), 0, 0), ((300, 132, 1037), 3, 1), ((5, 7, 3), 1, 2),
-                                               ((1030, 1100, 333), 2, 0), ((2100, 2080, 77), 0, 3)])
-def test_int8_matmul_any_alignment(ascq_gpu, oracle, trans_b, shape, a_off, b_off):
-    """int8 Matmul, DEQF16 C with int32 bias and per-channel words, K % 16 != 0 and / or A, B at odd byte offsets
-    (64 x 64 and, for 2100 x 2080, 128 x 128 any-alignment tiles): bit-exact"""
+                                               ((1030, 1100, 333), 2, 0), ((2100, 2080, 77), 0, 3),
+                                               ((2100, 2080, 205), 1, 3)])
+def test_int8_matmul_any_alignment(ascq_gpu, oracle, trans_b, shape, a_off, b_off, room):
+    """int8 Matmul, DEQF16 C with int32 bias and per-channel words, K % 16 != 0 and / or A, B at odd byte offsets: packed from
+    K = 192 on where there is room, else 64 x 64 and, for 2100 x 2080, 128 x 128 any-alignment tiles; bit-exact"""
     M, N, K = shape
     rng = seeded(M + N + K + a_off + trans_b)
     A = rng.integers(-128, 128, (M, K), dtype=np.int8)
@@ -95,7 +111,7 @@ def test_int8_matmul_any_alignment(ascq_gpu, oracle, trans_b, shape, a_off, b_of
     sc = np.exp(rng.uniform(np.log(2.0 ** -20), np.log(2.0 ** -8), N)).astype(np.float32)
     words = sc.view(np.uint32).astype(np.uint64)
     got = _int8_mm(ascq_gpu, A, np.ascontiguousarray(Bkn.T) if trans_b else Bkn, bias, words, False, trans_b, a_off,
-                   b_off, M, N, K)
+                   b_off, M, N, K, room=room)
     ref = O.mm_dequant(O.matmul_i8(A, Bkn, bias), O.F16, qvec=words)
     np.testing.assert_array_equal(got, ref)
 
@@ -118,17 +134,23 @@ def test_int8_matmul_any_alignment_trans_a_single_shape(ascq_gpu, oracle):
     assert np.isnan(got[sm:].view(np.float16)).all() and np.isnan(got[:, sn:].view(np.float16)).all()
 
 
+def _fp8_of(v):
+    return torch.from_numpy(np.ascontiguousarray(v)).float().to(torch.float8_e4m3fn).view(torch.uint8).numpy()
+
+
 def _fp8_codes(rng, shape, t8):
     v = rng.integers(-4, 5, shape).astype(np.float32)
     return torch.from_numpy(v).to(t8).view(torch.uint8).numpy()
 
 
+@pytest.mark.parametrize("room", ["own", "none"])
 @pytest.mark.parametrize("fa,fb", [(O.FP8_E4M3, O.FP8_E4M3), (O.FP8_E5M2, O.FP8_E4M3)])
 @pytest.mark.parametrize("shape,a_off,b_off", [((96, 160, 150), 0, 0), ((300, 200, 77), 5, 3),
-                                               ((2100, 2080, 40), 1, 0)])
-def test_fp8_matmul_any_alignment(ascq_gpu, oracle, fa, fb, shape, a_off, b_off):
+                                               ((2100, 2080, 40), 1, 0), ((96, 160, 250), 3, 0), ((2100, 2080, 203), 1, 2)])
+def test_fp8_matmul_any_alignment(ascq_gpu, oracle, fa, fb, shape, a_off, b_off, room):
     """fp8 A [M, K], B [N, K] with K % 16 != 0 and / or at odd byte offsets, f32 bias, f32 C: integer-valued codes,
-    exact sums, bit-exact"""
+    exact sums, bit-exact; packed from K = 192 on where there is room, else the 64 x 64 and (2100 x 2080) 128 x 128
+    any-alignment tiles"""
     M, N, K = shape
     rng = seeded(M + K + fa + 3 * fb + a_off)
     tt = {O.FP8_E4M3: torch.float8_e4m3fn, O.FP8_E5M2: torch.float8_e5m2}
@@ -140,12 +162,77 @@ def test_fp8_matmul_any_alignment(ascq_gpu, oracle, fa, fb, shape, a_off, b_off)
     mm.SetTensorA(_dev_at(A, a_off))
     mm.SetTensorB(_dev_at(Bt, b_off), True)
     mm.SetBias(_dev(bias))
-    c = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
-    mm.IterateAll(c)
-    mm.End()
-    torch.cuda.synchronize()
+    if room == "none":
+        _no_room(mm)
     ref, _, _, _ = O.matmul_fp8(A, Bt, fa, fb, bias=bias, out_type=O.F32, trans_b=True)
-    np.testing.assert_array_equal(c.cpu().numpy(), ref)
+    for _ in range(2 if room == "own" else 1):
+        c = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+        mm.IterateAll(c)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(c.cpu().numpy(), ref)
+    mm.End()
+
+
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("kind", ["int8", "fp8"])
+def test_packed_calls(ascq_gpu, oracle, kind, trans_b):
+    """One handle whose operands are packed, through what can change between its calls: other pointers at other offsets, a
+    single shape and back, A given [K, M] with an odd K (a copy in the workspace is packed), enAtomic, a caller's workspace
+    of the reported size, End and a smaller shape.  Integer-valued operands, exact sums"""
+    ascq = ascq_gpu
+    M, N, K = 150, 333, 1201
+    rng = seeded(60 + trans_b)
+    fp8 = kind == "fp8"
+    code = _fp8_of if fp8 else (lambda v: v)
+    ints = lambda *shape: rng.integers(-4, 5, shape, dtype=np.int8)  # noqa: E731
+    A, A2, B, B2 = ints(M, K), ints(M, K), ints(K, N), ints(K, N)
+    lay = lambda b: np.ascontiguousarray(b.T) if trans_b else b  # noqa: E731
+    prod = lambda a, b: a.astype(np.int32) @ b.astype(np.int32)  # noqa: E731
+    dt = torch.float32 if fp8 else torch.int32
+    t = ascq.FP8_E4M3 if fp8 else ascq.INT8
+    mm = ascq.Matmul(t, t, ascq.F32 if fp8 else ascq.INT32)
+
+    def run(want, op=0, c0=0, calls=1, block=None):
+        m, n = block or (M, N)
+        c = torch.full((M, N), c0, dtype=dt, device="cuda")
+        for _ in range(calls):
+            mm.IterateAll(c, op)
+        got = c.cpu().numpy()
+        np.testing.assert_array_equal(got[:m, :n], want.astype(got.dtype))
+        assert (got[m:] == c0).all() and (got[:, n:] == c0).all()
+
+    mm.SetOrgShape(M, N, K)
+    mm.SetTensorA(_dev_at(code(A), 0))
+    mm.SetTensorB(_dev_at(code(lay(B)), 1), trans_b)
+    run(prod(A, B))
+    run(prod(A, B))
+    mm.SetTensorA(_dev_at(code(A2), 5))
+    run(prod(A2, B))
+    mm.SetTensorB(_dev_at(code(lay(B2)), 0), trans_b)
+    run(prod(A2, B2))
+    mm.SetSingleShape(70, 130, 501)
+    run(prod(A2[:70, :501], B2[:501, :130]), block=(70, 130))
+    mm.SetSingleShape(M, N, K)
+    run(3 + 2 * prod(A2, B2), op=ascq.ATOMIC_ADD, c0=3, calls=2)
+    mm.SetTensorA(_dev_at(code(np.ascontiguousarray(A.T)), 3), True)
+    run(prod(A, B2))
+    run(prod(A, B2))
+    mm.SetTensorA(_dev_at(code(A), 0))
+    nbytes = mm.WorkspaceSize()
+    assert nbytes >= M * K
+    ws = torch.full((nbytes + 64,), FILL, dtype=torch.uint8, device="cuda")
+    mm.SetWorkspace(ws[:nbytes], nbytes)
+    run(prod(A, B2))
+    assert bool((ws[nbytes:] == FILL).all()) and not bool((ws[:nbytes] == FILL).all())
+    mm.SetWorkspace(None, 0)
+    mm.End()
+    m, n, k = 33, 65, 257
+    mm.SetOrgShape(m, n, k)
+    mm.SetTensorA(_dev_at(code(np.ascontiguousarray(A[:m, :k])), 0))
+    mm.SetTensorB(_dev_at(code(lay(B[:k, :n])), 0), trans_b)
+    c = torch.zeros((m, n), dtype=dt, device="cuda")
+    mm.IterateAll(c)
+    np.testing.assert_array_equal(c.cpu().numpy().astype(np.int32), prod(A[:m, :k], B[:k, :n]))
 
 
 _LOG_SCRIPT = r"""
