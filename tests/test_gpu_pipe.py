@@ -20,8 +20,10 @@ SHAPES = [
     (3353, 536, 272),    # 128 x 128
     (4127, 932, 416),    # 128 x 192
     (1607, 3736, 528),   # 128 x 256
-    (3457, 1732, 64),    # 192 x 256
-    (3273, 1816, 144),   # 256 x 192
+    (3457, 1732, 64),    # 64 x 128, seven rounds of one partial stage
+    (3273, 1816, 144),   # 64 x 128
+    (3585, 2180, 144),   # 192 x 256
+    (4436, 1288, 144),   # 256 x 192
     (3301, 3804, 80),    # 256 x 256
 ]
 
@@ -144,7 +146,7 @@ def test_ragged_without_a_workspace(ascq_gpu, oracle):
 
 # (M, N, K): more than 128 tiles of 64 x 128, the tile pick_pipe_tile chooses; odd and even counts of half stages
 MX_SHAPES = [(513, 1900, 640), (1100, 2100, 384), (3353, 536, 640), (4127, 932, 896), (1607, 3736, 1152), (3457, 1732, 128),
-             (3273, 1816, 384), (3301, 3804, 128)]
+             (3273, 1816, 384), (3301, 3804, 128), (3394, 2308, 384), (4430, 1288, 384)]
 E2M1 = torch.tensor([0, 0.5, 1, 1.5, 2, 3, 4, 6, 0, -0.5, -1, -1.5, -2, -3, -4, -6], dtype=torch.float64)
 
 
