@@ -203,6 +203,15 @@ _current_device = getattr(torch._C, "_cuda_getDevice", None)
 _stream_ready = False
 
 
+def _forked() -> None:
+    """A forked child goes the public way again, which refuses a device that the parent initialised"""
+    global _stream_ready
+    _stream_ready = False
+
+
+os.register_at_fork(after_in_child=_forked)
+
+
 def _stream(stream) -> int | None:
     global _stream_ready
     if stream is None:

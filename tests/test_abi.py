@@ -510,3 +510,18 @@ def test_env_gated_host_log():
         r = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=120)
         assert r.returncode == 0, r.stderr
         assert ("ascq: error" in r.stderr and "null argument" in r.stderr) == expect, r.stderr
+
+
+def test_forked_child_asks_for_the_stream_the_public_way():
+    """The current stream's handle is read without torch's initialisation check once that check has passed; a forked child
+    must go through it again (it cannot use the parent's device)"""
+    before = ascq._stream_ready
+    ascq._stream_ready = True
+    try:
+        pid = os.fork()
+        if pid == 0:
+            os._exit(int(ascq._stream_ready))
+        assert os.waitstatus_to_exitcode(os.waitpid(pid, 0)[1]) == 0
+        assert ascq._stream_ready
+    finally:
+        ascq._stream_ready = before
