@@ -503,7 +503,8 @@ hipError_t launch_gemm_i8(const GemmI8Args& a, hipStream_t st)
         return launch_gemm_i8_pipe(a, st);
     }
     // K not a multiple of 16, or operands / leading dimensions not 16-byte (A, K-contiguous B) or 4-byte ([K, N] B)
-    // aligned, where the host layer had no workspace to pack them into: the any-alignment tiles (GemmCoreUA), 64 x 64 while that leaves fewer than 256 workgroups of 128 x 128
+    // aligned, where the host layer had no room to pack them or packing would not pay: the any-alignment tiles
+    // (GemmCoreUA), 64 x 64 while that leaves fewer than 256 workgroups of 128 x 128
     const int64_t a_span = a.lda * (a.M - 1) + a.K, b_span = a.trans_b ? a.ldb * (a.N - 1) + a.K : a.ldb * (a.K - 1) + a.N;
     const char* why = a.trans_a                            ? "A given [K, M]"
                       : (a_span >= (1ll << 31) - 16 || b_span >= (1ll << 31) - 16) ? "an operand spans 2^31 bytes"
