@@ -69,7 +69,8 @@ constexpr int op_of_fmt = (FMT == (FMT_BF16 | (FMT_BF16 << 3))) ? OP_BF16 : OP_F
 // range a whole number of KW RB units (shared out as evenly as p.splits allows), and stores the tile's fp32
 // accumulators in p.ws ([split][tile][fragment][lane]); 2 -- one wave per 32 x 32 fragment of a tile adds the
 // splits' accumulators of its fragment in split order (one fixed order, so the result does not vary between calls)
-// and stores it through the epilogue.
+// and stores it through the epilogue; 3 -- C combined by enAtomic: a kernel of its own, so that the compare-and-swap code
+// (half of the instructions) does not weigh on the schedule of the storing one.
 template <int BM, int BN, int WM, int WN, int ST, bool TB, int RB, int FMT, bool UA = false, int KW = 1, bool BTR = false,
           int PH = 0>
 __global__ __launch_bounds__(PH == 2 ? (BM / 32) * (BN / 32) * 64 : WM * WN * 64 * KW) void gemm_f8_kernel(GemmF8Args p)
@@ -81,7 +82,7 @@ __global__ __launch_bounds__(PH == 2 ? (BM / 32) * (BN / 32) * 64 : WM * WN * 64
                                         GemmCore<BM, BN, WM, WN, ST, TB, OP, RB, FMT, true, false, BTR>>::type;
     static_assert(KW == 1 || (WM == 1 && WN == 1 && (TB || BTR) && !UA),
                   "k-split waves run one-wave tiles of a K-contiguous or LDS-transposed B");
-    static_assert(PH == 0 || (WM == 1 && WN == 1 && !UA && ES == 1 && (PH == 2 || KW > 1)), "K split across workgroups");
+    static_assert(PH == 0 || PH == 3 || (WM == 1 && WN == 1 && !UA && ES == 1 && (PH == 2 || KW > 1)), "K split across workgroups");
     extern __shared__ __attribute__((aligned(16))) uint8_t smem_f8[];
     const int tiles_m = (int)((p.M + BM - 1) / BM), tiles_n = (int)((p.N + BN - 1) / BN);
     const int ntiles = tiles_m * tiles_n;
@@ -222,7 +223,7 @@ __global__ __launch_bounds__(PH == 2 ? (BM / 32) * (BN / 32) * 64 : WM * WN * 64
             }
         }
     };
-    if (KW == 1 && p.atomic != C_STORE) {  // enAtomic: f32 / f16 / bf16 C (the host layer refuses the others)
+    if constexpr (PH == 3) {  // enAtomic: f32 / f16 / bf16 C (the host layer refuses the others)
         // (acc + bias) x M1 of the column -- the store path's arithmetic
         auto v = [&](int cl, uint32_t a) {
             float x = __uint_as_float(a);
@@ -309,10 +310,16 @@ static hipError_t launch_f8_tiled(const GemmF8Args& a, hipStream_t st)
     static_assert(KW == 1 || (size_t)(KW - 1) * T::FM * T::FN * 64 * sizeof(typename T::acc_t) <= (size_t)LDS,
                   "k-split reduction");
     const int tiles = (int)(((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN));
-    const hipError_t e = ensure_dynamic_lds<gemm_f8_kernel<BM, BN, WM, WN, ST, TB, RB, FMT, UA, KW, BTR>>(LDS);
-    if (e != hipSuccess) return e;
-    launch_k((gemm_f8_kernel<BM, BN, WM, WN, ST, TB, RB, FMT, UA, KW, BTR>), dim3(tiles), dim3(T::NT * KW), LDS, st, a);
-    return hipGetLastError();
+    auto go = [&](auto PH) -> hipError_t {
+        constexpr auto kern = gemm_f8_kernel<BM, BN, WM, WN, ST, TB, RB, FMT, UA, KW, BTR, decltype(PH)::value>;
+        const hipError_t e = ensure_dynamic_lds<kern>(LDS);
+        if (e != hipSuccess) return e;
+        launch_k(kern, dim3(tiles), dim3(T::NT * KW), LDS, st, a);
+        return hipGetLastError();
+    };
+    if constexpr (KW == 1)  // (the K-split waves only store)
+        if (a.atomic != C_STORE) return go(std::integral_constant<int, 3>{});
+    return go(std::integral_constant<int, 0>{});
 }
 
 // the K split across workgroups of decode-sized batches (decode_splits): one-wave tiles of 32 or 64 rows (one row

@@ -31,7 +31,9 @@ using I8Core = typename std::conditional<UA, GemmCoreUA<BM, BN, WM, WN, TB, CT>,
 // PH (K split across workgroups, decode-sized batches): 1 -- workgroup b runs split b / tiles of tile b % tiles, its
 // K range a whole number of KW RB units (the units shared out as evenly as p.splits allows), and stores the tile's
 // accumulators in p.ws ([split][tile][fragment][lane]); 2 -- one wave per 32 x 32 fragment of a tile adds the
-// splits' accumulators of its fragment in split order (int32: exact) and stores it through the epilogue.
+// splits' accumulators of its fragment in split order (int32: exact) and stores it through the epilogue; 3 -- C combined by
+// enAtomic: a kernel of its own, so that the compare-and-swap code (half of the instructions) does not weigh on the
+// schedule of the storing one.
 template <int BM, int BN, int WM, int WN, int ST, bool TB, int RB = 64, bool BTR = false, int KW = 1, bool UA = false,
           int PH = 0>
 __global__ __launch_bounds__(PH == 2 ? (BM / 32) * (BN / 32) * 64 : WM * WN * 64 * KW) void gemm_i8_kernel(GemmI8Args p)
@@ -39,7 +41,7 @@ __global__ __launch_bounds__(PH == 2 ? (BM / 32) * (BN / 32) * 64 : WM * WN * 64
     using T = I8Core<BM, BN, WM, WN, ST, TB, RB, false, BTR, UA>;
     static_assert(!UA || KW == 1, "any-alignment tiles run whole K");
     static_assert(KW == 1 || (WM == 1 && WN == 1), "k-split waves run one-wave tiles");
-    static_assert(PH == 0 || (WM == 1 && WN == 1 && !UA && (PH == 2 || KW > 1)), "K split across workgroups");
+    static_assert(PH == 0 || PH == 3 || (WM == 1 && WN == 1 && !UA && (PH == 2 || KW > 1)), "K split across workgroups");
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int tiles_m = (int)((p.M + BM - 1) / BM), tiles_n = (int)((p.N + BN - 1) / BN);
     const int ntiles = tiles_m * tiles_n;
@@ -178,7 +180,7 @@ __global__ __launch_bounds__(PH == 2 ? (BM / 32) * (BN / 32) * 64 : WM * WN * 64
             }
         }
     };
-    if (KW == 1 && p.atomic != C_STORE) {  // enAtomic: int32 / f16 / bf16 C (the host layer refuses the others)
+    if constexpr (PH == 3) {  // enAtomic: int32 / f16 / bf16 C (the host layer refuses the others)
         // acc + bias (int32, wrapping), then x M1 of the column for f16 / bf16 -- the store path's arithmetic
         auto v = [&](int cl, uint32_t a) { return (int32_t)(a + (uint32_t)(p.bias ? p.bias[n0 + cl] : 0)); };
         auto m1 = [&](int cl) { return p.qvec ? quant_pre_m1(p.qvec[n0 + cl]) : mscalar; };
@@ -379,11 +381,16 @@ static hipError_t launch_tiled(const GemmI8Args& a, hipStream_t st)
     using T = I8Core<BM, BN, WM, WN, ST, TB, RB, false, BTR, UA>;
     const int tiles = (int)(((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN));
     constexpr size_t lds = T::LDS_BYTES * KW;
-    const hipError_t e = ensure_dynamic_lds<gemm_i8_kernel<BM, BN, WM, WN, ST, TB, RB, BTR, KW, UA>>((int)lds);
-    if (e != hipSuccess) return e;
-    launch_k((gemm_i8_kernel<BM, BN, WM, WN, ST, TB, RB, BTR, KW, UA>), dim3(tiles), dim3(T::NT * KW), (uint32_t)lds, st,
-             a);
-    return hipGetLastError();
+    auto go = [&](auto PH) -> hipError_t {
+        constexpr auto kern = gemm_i8_kernel<BM, BN, WM, WN, ST, TB, RB, BTR, KW, UA, decltype(PH)::value>;
+        const hipError_t e = ensure_dynamic_lds<kern>((int)lds);
+        if (e != hipSuccess) return e;
+        launch_k(kern, dim3(tiles), dim3(T::NT * KW), (uint32_t)lds, st, a);
+        return hipGetLastError();
+    };
+    if constexpr (KW == 1)  // (the K-split waves only store)
+        if (a.atomic != C_STORE) return go(std::integral_constant<int, 3>{});
+    return go(std::integral_constant<int, 0>{});
 }
 
 // the K split across workgroups of decode-sized batches: 32-row one-wave tiles, four K-split waves per workgroup,
