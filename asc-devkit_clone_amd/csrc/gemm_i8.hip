@@ -505,7 +505,10 @@ hipError_t launch_gemm_i8(const GemmI8Args& a, hipStream_t st)
             if (a.trans_b) return tiny ? launch_tiled<32, 32, 1, 1, 4, true>(a, st) : launch_tiled<64, 64, 2, 2, 4, true>(a, st);
             if (tiny && b_tr) return launch_tiled<32, 32, 1, 1, 4, false, 64, true>(a, st);
         }
-        if (b_tr && a.atomic == C_STORE && few_long_kn(a.M, a.N, a.K))
+        // (B [K, N] at short K: 64 x 64 tiles too, up to 896 of them, 512 from K = 336 to 384; us against the pipelined tiles:
+        // M = 256, N = 14336, K = 272 7.1 / 7.6, M = 512, N = 6144 6.5 / 7.1; M = 256, N = 14336, K = 384 8.0 / 7.3)
+        const bool short_kn = a.K <= 384 && t64 <= (a.K <= 320 ? 896 : 512) && a.M < 1024;
+        if (b_tr && a.atomic == C_STORE && (short_kn || few_long_kn(a.M, a.N, a.K)))
             return launch_tiled<64, 64, 2, 2, 4, false, 64, true>(a, st);
         return launch_gemm_i8_pipe(a, st);
     }

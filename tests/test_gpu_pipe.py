@@ -42,7 +42,7 @@ FEW = [
     (70, 528, 528),       # both: 32 x 32 (int8); 64 x 64 (fp8, [N, K])
     (70, 4112, 1040),     # [N, K]: 64 x 64, 66 tiles of 64 x 128
     (130, 8000, 528),     # [N, K]: 64 x 64, 189 of them (int8)
-    (300, 6032, 272),     # [N, K]: 64 x 64, 240 of them (int8)
+    (300, 6032, 272),     # both: 64 x 64 (int8)
     (65, 1040, 4112),     # [N, K]: 64 x 64, rows off 128 bytes
     (40, 4624, 6160),     # [K, N]: 64 x 64 (few_long_kn), K its least
     (130, 2576, 8208),    # [K, N]: 64 x 64
