@@ -304,6 +304,7 @@ struct ByteOperands {
     int64_t lda, ldb;
     int trans_a, trans_b;
     size_t ws_end = SIZE_MAX;  // the workspace up to the packed operands, if it holds any
+    bool bf16 = false;         // fp8 operands decoded to bf16 rows (lda, ldb in values)
 };
 
 ascq_status prepare_byte_operands(ascq_matmul_s* h, hipStream_t st, ByteOperands& o)
@@ -345,22 +346,34 @@ ascq_status prepare_byte_operands(ascq_matmul_s* h, hipStream_t st, ByteOperands
 // graph may hold and a mere pointer must not replace.  The room is optional: a caller's workspace without it, a stream
 // under capture (the graph would share the room with later eager calls), a fifth stream, a failed allocation or the
 // allocation-free form (whose scratch all handles share) leave the call to the any-alignment tiles.
+// fp8 with B [K, N] off its alignment is decoded to bf16 rows, A [M, K] and B [N, K], instead (every fp8 value is a bf16 value):
+// without room it runs element by element, its sums in fp32, which the fp8 MFMAs, dropping what lies 2^-13 below a group's
+// largest product, would not keep and the bf16 MFMAs do.  (From 512 rows on with N and K multiples of 16 such a B has always
+// been brought to the fp8 MFMAs; it is packed like the rest.)
 struct PackPlan {
-    bool a, b;
+    bool a, b, bf16;
     int64_t kp, pitch_b;  // bytes of a packed row of A (and of a K-contiguous B); of a packed row of B
     size_t a_bytes, b_bytes;
 };
-PackPlan pack_plan(bool fp8, const ByteOperands& o, int64_t m, int64_t n, int64_t k)
+PackPlan pack_plan(const ascq_matmul_s* h, const ByteOperands& o, int64_t m, int64_t n, int64_t k)
 {
     PackPlan p{};
     if (o.trans_a) return p;
-    const bool k16 = k % 16 == 0;
+    const bool k16 = k % 16 == 0, fp8 = kind_of(h->ty) == K_F8;
     p.kp = (k + 15) / 16 * 16;
+    p.pitch_b = o.trans_b ? p.kp : (n + 15) / 16 * 16;
     p.a = o.lda % 16 != 0 || (uintptr_t)o.A % 16 != 0 || (!k16 && (o.trans_b || fp8));
     p.b = o.trans_b ? o.ldb % 16 != 0 || (uintptr_t)o.B % 16 != 0 || !k16 : o.ldb % 4 != 0 || (uintptr_t)o.B % 4 != 0;
-    p.pitch_b = o.trans_b ? p.kp : (n + 15) / 16 * 16;
-    p.a_bytes = p.a ? align256((size_t)m * (size_t)p.kp) : 0;
-    p.b_bytes = p.b ? align256((size_t)(o.trans_b ? n : k) * (size_t)p.pitch_b) : 0;
+    if (fp8 && !o.trans_b && !(k16 && h->M >= 512 && h->N % 16 == 0 && h->K % 16 == 0)) {
+        p.bf16 = (p.a || p.b || n % 4 != 0) && h->N < (1ll << 21);
+        p.a = p.b = p.bf16;
+        p.kp = (k + 7) / 8 * 16;
+        p.a_bytes = p.bf16 ? align256((size_t)m * (size_t)p.kp) : 0;
+        p.b_bytes = p.bf16 ? align256((size_t)n * (size_t)p.kp) : 0;
+    } else {
+        p.a_bytes = p.a ? align256((size_t)m * (size_t)p.kp) : 0;
+        p.b_bytes = p.b ? align256((size_t)(o.trans_b ? n : k) * (size_t)p.pitch_b) : 0;
+    }
     if (p.a_bytes >= (1u << 31) || p.b_bytes >= (1u << 31)) return PackPlan{};
     return p;
 }
@@ -379,7 +392,7 @@ size_t pack_need(const ascq_matmul_s* h)
     if ((kind != K_INT8 && kind != K_F8) || h->M <= 0 || h->trans_a || bytes_nz_b(h)) return 0;
     const int64_t m = h->sm > 0 ? h->sm : h->M, n = h->sn > 0 ? h->sn : h->N, k = h->sk > 0 ? h->sk : h->K;
     const ByteOperands o{(const uint8_t*)h->a, (const uint8_t*)h->b, h->K, h->trans_b ? h->K : h->N, 0, h->trans_b};
-    const PackPlan p = pack_plan(kind == K_F8, o, m, n, k);
+    const PackPlan p = pack_plan(h, o, m, n, k);
     return p.a || p.b ? pack_base(h, m, n, k) + p.a_bytes + p.b_bytes : 0;
 }
 
@@ -439,18 +452,16 @@ uint8_t* pack_room(ascq_matmul_s* h, hipStream_t st, size_t bytes, float gain_us
     return (uint8_t*)r.p;
 }
 
-ascq_status pack_byte_operands(ascq_matmul_s* h, hipStream_t st, int64_t m, int64_t n, int64_t* k, bool fp8,
-                               ByteOperands& o, int* a_padded)
+ascq_status pack_byte_operands(ascq_matmul_s* h, hipStream_t st, int64_t m, int64_t n, int64_t* k, ByteOperands& o)
 {
-    const PackPlan p = pack_plan(fp8, o, m, n, *k);
+    const PackPlan p = pack_plan(h, o, m, n, *k);
     if (!p.a && !p.b) return ASCQ_OK;
     if (h->no_alloc) return ASCQ_OK;
     // the any-alignment tiles take 18 us per 1000 K and round of 128 tiles of 128 x 128, the copy and the aligned ones
     // about 7, but two launches: K below 192 is faster in one (1000 x 1000 x 100: 5.8 / 7.3 us; at K = 200 8.0 / 7.9) up
-    // to some rounds.  fp8 with B [K, N] would run element by element (32 x 32 x 40: 17.1 / 6.5)
+    // to some rounds.  (Decoded to bf16: the other way is element by element.)
     const int64_t rounds = (((m + 127) / 128) * ((n + 127) / 128) + 127) / 128;
-    const bool elementwise = fp8 && !o.trans_b;
-    if (!elementwise && *k < 192 && rounds <= 4) return ASCQ_OK;
+    if (!p.bf16 && *k < 192 && rounds <= 4) return ASCQ_OK;
     const size_t need = p.a_bytes + p.b_bytes;
     uint8_t* pa = nullptr;
     if (h->ws && !h->ws_owned) {
@@ -459,10 +470,23 @@ ascq_status pack_byte_operands(ascq_matmul_s* h, hipStream_t st, int64_t m, int6
         pa = (uint8_t*)h->ws + base;
         o.ws_end = base;
     } else {
-        pa = pack_room(h, st, need, elementwise ? 1e9f : 0.011f * (float)*k * (float)rounds);
+        pa = pack_room(h, st, need, p.bf16 ? 1e9f : 0.011f * (float)*k * (float)rounds);
         if (!pa) return ASCQ_OK;
     }
     uint8_t* pb = pa + p.a_bytes;
+    if (p.bf16) {
+        const int64_t ld = p.kp / 2;
+        hipError_t e = ascq::launch_byte_to_bf16((uint16_t*)pa, ld, o.A, o.lda, m, *k, f8f6f4_code(h->ty.a_type), 0, st);
+        if (e == hipSuccess)
+            e = ascq::launch_byte_to_bf16((uint16_t*)pb, ld, o.B, o.ldb, n, *k, f8f6f4_code(h->ty.b_type), 1, st);
+        if (e != hipSuccess) return hip_status(e, "fp8 -> bf16");
+        o.A = pa;
+        o.B = pb;
+        o.lda = o.ldb = *k = ld;
+        o.trans_b = 1;
+        o.bf16 = true;
+        return ASCQ_OK;
+    }
     const ascq::PackRows ja{p.a ? pa : nullptr, o.A, m, *k, o.lda};
     const ascq::PackRows jb = o.trans_b ? ascq::PackRows{p.b ? pb : nullptr, o.B, n, *k, o.ldb}
                                         : ascq::PackRows{p.b ? pb : nullptr, o.B, *k, n, o.ldb};
@@ -472,7 +496,6 @@ ascq_status pack_byte_operands(ascq_matmul_s* h, hipStream_t st, int64_t m, int6
     if (p.a) {
         o.A = pa;
         o.lda = p.kp;
-        *a_padded = 1;
     }
     if (p.b) {
         o.B = pb;
@@ -781,8 +804,7 @@ ascq_status ascq_matmul_iterate_all(ascq_matmul_t h, void* c, uint8_t en_atomic,
         }
         ByteOperands o;
         ascq_status s = prepare_byte_operands(h, st, o);
-        int padded = 0;
-        if (s == ASCQ_OK) s = pack_byte_operands(h, st, m, n, &g.K, false, o, &padded);
+        if (s == ASCQ_OK) s = pack_byte_operands(h, st, m, n, &g.K, o);
         if (s != ASCQ_OK) return s;
         g.A = (const int8_t*)o.A;
         g.B = (const int8_t*)o.B;
@@ -862,8 +884,11 @@ ascq_status ascq_matmul_iterate_all(ascq_matmul_t h, void* c, uint8_t en_atomic,
         if (s != ASCQ_OK) return s;
         uint16_t* a16 = (uint16_t*)h->ws;
         uint16_t* b16 = (uint16_t*)((uint8_t*)h->ws + align256((size_t)h->M * (size_t)kp * 2));
-        hipError_t e = ascq::launch_hif8_to_bf16(a16, kp, (const uint8_t*)h->a, h->M, h->K, h->trans_a, st);
-        if (e == hipSuccess) e = ascq::launch_hif8_to_bf16(b16, kp, (const uint8_t*)h->b, h->N, h->K, !h->trans_b, st);
+        hipError_t e = ascq::launch_byte_to_bf16(a16, kp, (const uint8_t*)h->a, h->trans_a ? h->M : h->K, h->M, h->K,
+                                                 ascq::FMT_HIF8, h->trans_a, st);
+        if (e == hipSuccess)
+            e = ascq::launch_byte_to_bf16(b16, kp, (const uint8_t*)h->b, h->trans_b ? h->K : h->N, h->N, h->K, ascq::FMT_HIF8,
+                                          !h->trans_b, st);
         if (e != hipSuccess) return hip_status(e, "hifloat8 -> bf16");
         ascq::GemmF8Args g{};
         g.A = (const uint8_t*)a16;
@@ -898,7 +923,7 @@ ascq_status ascq_matmul_iterate_all(ascq_matmul_t h, void* c, uint8_t en_atomic,
         ByteOperands o;
         ascq_status s = prepare_byte_operands(h, st, o);
         g.K = k;
-        if (s == ASCQ_OK) s = pack_byte_operands(h, st, m, n, &g.K, true, o, &g.a_padded);
+        if (s == ASCQ_OK) s = pack_byte_operands(h, st, m, n, &g.K, o);
         if (s != ASCQ_OK) return s;
         g.A = o.A;
         g.B = o.B;
@@ -915,9 +940,10 @@ ascq_status ascq_matmul_iterate_all(ascq_matmul_t h, void* c, uint8_t en_atomic,
         g.qscalar = h->qscalar;
         g.use_quant = h->quant_set ? 1 : 0;
         g.c_type = h->ty.c_type;  // ascq_dtype codes equal the device DT_* codes
-        g.fmt_a = f8f6f4_code(h->ty.a_type);
-        g.fmt_b = f8f6f4_code(h->ty.b_type);
+        g.fmt_a = o.bf16 ? ascq::FMT_BF16 : f8f6f4_code(h->ty.a_type);
+        g.fmt_b = o.bf16 ? ascq::FMT_BF16 : f8f6f4_code(h->ty.b_type);
         g.atomic = atomic;
+        if (o.bf16) return hip_status(ascq::launch_gemm_f8(g, st), "gemm_f8 (bf16 rows)");
         s = split_region(h, m, n, k, atomic, o.ws_end, &g.ws, &g.ws_bytes);
         if (s != ASCQ_OK) return s;
         return hip_status(ascq::launch_gemm_f8(g, st), "gemm_f8");

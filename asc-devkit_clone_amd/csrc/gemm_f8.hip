@@ -25,7 +25,8 @@
 // significand of at most 4 bits, 2^-22 .. 2^15, +-inf, NaN) is a bf16 value -- a normal one, where f16 would need
 // subnormals below 2^-14 -- so the host layer decodes both operands to bf16 K-contiguous rows in the workspace and
 // this kernel runs them through v_mfma_f32_32x32x16_bf16 (fmt code FMT_BF16, GemmCore OP_BF16) with the same fp32
-// accumulators and epilogue.  C may be hifloat8 for either operand kind
+// accumulators and epilogue.  It does the same with fp8 operands off their alignment and B [K, N], whose sums the
+// element-wise kernel keeps in fp32.  C may be hifloat8 for either operand kind
 // ((V)QF322HIF8_PRE, quant_processor_fixpipe.h:106-107: ties away from zero, saturating at +-32768, NaN -> 0 -- the
 // saturation-mode row of matrix_compute_move_out_interface_boundary_value_summary.md:68-70).
 #include "common.h"
@@ -426,7 +427,7 @@ hipError_t launch_gemm_f8(const GemmF8Args& a, hipStream_t st)
     const bool b_ok = a.trans_b ? ((a.ldb * es) % 16 == 0 && ((uintptr_t)a.B % 16 == 0) && a.ldb * es * a.N < (1ll << 31))
                                 : (a.ldb % 4 == 0 && ((uintptr_t)a.B % 4 == 0) && a.ldb * a.K < (1ll << 31));
     // the tiled epilogue addresses a 256-row output tile with 32-bit offsets
-    const bool tiled = a_ok && b_ok && ((a.K * es) % 16 == 0 || (!a.trans_b && a.a_padded)) && a.ldc < (1ll << 21);
+    const bool tiled = a_ok && b_ok && (a.K * es) % 16 == 0 && a.ldc < (1ll << 21);
     // otherwise fp8 with A [M, K] and B [N, K] (any alignment, any K) takes the any-alignment tiles
     const char* why = tiled ? nullptr
                       : bf ? "bf16 operands: K not a multiple of 8"

@@ -36,8 +36,8 @@
 // its eight, and each stage's go to one of four scale slots, requested three stages ahead, one copy per wave and stage;
 // a lane reads the two bytes of block g of its row and the MFMA's op_sel picks the k-step's.
 // K: a lane's 16-byte chunks at or past the end of K are not read (zeros), nor are a [K, N] B's rows.  So K of K-contiguous
-// operands is a multiple of 16 bytes; with B [K, N] K is any, A's bytes from K to the end of its chunk lying within its
-// pitch (int8: any, they meet zeros; fp8: zeros, a NaN would not vanish).
+// operands is a multiple of 16 bytes; with an int8 B [K, N] K is any, A's bytes from K to the end of its chunk lying within
+// its pitch (they meet zeros; an fp8 NaN would not vanish against them).
 //
 // Weight-only antiquant (OP_AQ): A is f16 (a stage is 64 k), B the packed int4 / int8 weight.  A wave loads one 16-column
 // strip of a half per stage into registers (packed codes, the columns' scale and offset), six phases ahead, dequantises

@@ -1,6 +1,5 @@
 // gemm_pipe_f8.hip -- the fp8 Matmul on the pipelined tiles of gemm_pipe.h: the GEMM and epilogues of gemm_f8.hip for
-// A [M, K] with 16-byte-aligned rows and B [N, K] the same (K a multiple of 16), or B [K, N] with 4-byte-aligned rows (any
-// K, A zero-padded to a multiple of 16).
+// A [M, K] with 16-byte-aligned rows and B [N, K] the same, or B [K, N] with 4-byte-aligned rows; K a multiple of 16.
 #include "common.h"
 #include "gemm_pipe.h"
 #include "launch.h"
@@ -17,7 +16,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_f8_pipe_kernel(GemmF8Arg
     const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
     const int rows = (int)(p.M - m0 < BM ? p.M - m0 : BM), cols = (int)(p.N - n0 < BN ? p.N - n0 : BN);
     PipeArgs c{};
-    c.a = make_rsrc4(p.A, (uint32_t)(p.lda * (p.M - 1) + (p.K + 15) / 16 * 16));  // (whole chunks: within the pitch)
+    c.a = make_rsrc4(p.A, (uint32_t)(p.lda * (p.M - 1) + p.K));
     c.b = make_rsrc4(p.B, (uint32_t)(BTR ? p.ldb * (p.K - 1) + (p.N + 3) / 4 * 4 : p.ldb * (p.N - 1) + p.K));
     c.lda = (uint32_t)p.lda;
     c.ldb = (uint32_t)p.ldb;

@@ -136,7 +136,7 @@ struct GemmF8Args {
     int use_quant;        // 1: multiply by M1 (SetQuantScalar / SetQuantVector was called)
     int c_type;           // DT_F16 / DT_BF16 / DT_F32; DT_INT8 / DT_UINT8 (QF322B8); DT_FP8_E4M3 / _E5M2 (QF322FP8);
                           // DT_HIF8 (QF322HIF8); DT_INT4 (QF322S4)
-    int fmt_a, fmt_b;     // f8f6f4 codes: 0 e4m3fn, 1 e5m2; FMT_BF16 in both: A / B are bf16 (a hifloat8 Matmul's
+    int fmt_a, fmt_b;     // f8f6f4 codes: 0 e4m3fn, 1 e5m2; FMT_BF16 in both: A / B are bf16 (a hifloat8 or decoded fp8 Matmul's
                           // operands decoded by the host layer; A [M, K] and B [N, K], K-contiguous, lda / ldb in
                           // elements)
     int trans_a, trans_b;
@@ -144,11 +144,10 @@ struct GemmF8Args {
     uint8_t* ws;          // decode-sized batches: room for the K-split partials (decode_split_ws_bytes), or null
     size_t ws_bytes;
     int splits;           // (set by the launcher) workgroups per tile of the K-split form
-    int a_padded;         // A's rows hold zeros from K up to a multiple of 16
 };
 hipError_t launch_gemm_f8(const GemmF8Args& a, hipStream_t st);
-// gemm_pipe_f8.hip: as gemm_pipe_i8.hip, but with B [K, N] and K not a multiple of 16 A's rows are zero-padded to one
-// (a_padded: a NaN or infinity past K would not vanish against B's zeros)
+// gemm_pipe_f8.hip: as gemm_pipe_i8.hip, but K a multiple of 16 (a NaN or infinity of A past K would not vanish against the
+// zeros of a [K, N] B)
 hipError_t launch_gemm_f8_pipe(const GemmF8Args& a, hipStream_t st);
 
 // group_gemm.hip
@@ -239,10 +238,11 @@ hipError_t launch_nz_to_nd(void* dst, const void* src, int esize, int64_t batch,
                            int transpose_out, hipStream_t st);
 hipError_t launch_nd_to_nz(void* dst, const void* src, int esize, int64_t batch, int64_t rows, int64_t cols,
                            hipStream_t st);
-// hifloat8 -> bf16 (exact): dst [R, ldd] bf16 (ldd % 8 == 0, columns C .. ldd - 1 zero, dst 16-byte aligned) from
-// src [R, C], or from src [C, R] with transpose
-hipError_t launch_hif8_to_bf16(uint16_t* dst, int64_t ldd, const uint8_t* src, int64_t R, int64_t C, int transpose,
-                              hipStream_t st);
+// hifloat8 (FMT_HIF8) or fp8 (0 e4m3, 1 e5m2) -> bf16 (exact): dst [R, ldd] bf16 (ldd % 8 == 0, columns C .. ldd - 1 zero,
+// dst 16-byte aligned) from src [R, C] of pitch lds, or from src [C, R] with transpose
+constexpr int FMT_HIF8 = 6;
+hipError_t launch_byte_to_bf16(uint16_t* dst, int64_t ldd, const uint8_t* src, int64_t lds, int64_t R, int64_t C, int fmt,
+                               int transpose, hipStream_t st);
 // int4 (two per byte, even element in the low nibble) -> int8, elementwise over `bytes` input bytes
 hipError_t launch_unpack_int4(int8_t* dst, const uint8_t* src, int64_t bytes, hipStream_t st);
 // transpose a [K, N] packed fp4 matrix (two per byte along N) into [N, K] (two per byte along K)

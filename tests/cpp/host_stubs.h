@@ -75,6 +75,12 @@ hipError_t launch_pack_rows(const PackRows& a, const PackRows& b, hipStream_t)
     if (b.dst) use(b.dst, (size_t)b.rows * ((b.cols + 15) / 16 * 16), "packed B");
     return hipSuccess;
 }
+hipError_t launch_byte_to_bf16(uint16_t* dst, int64_t ldd, const uint8_t*, int64_t, int64_t rows, int64_t, int, int transpose,
+                               hipStream_t)
+{
+    use(dst, (size_t)(rows * ldd) * 2, transpose ? "packed B (bf16)" : "packed A (bf16)");
+    return hipSuccess;
+}
 hipError_t launch_transpose_i8(uint8_t* dst, const uint8_t*, int64_t rows, int64_t cols, hipStream_t)
 {
     use(dst, (size_t)(rows * cols), "transposed A");

@@ -235,6 +235,55 @@ def test_packed_calls(ascq_gpu, oracle, kind, trans_b):
     np.testing.assert_array_equal(c.cpu().numpy().astype(np.int32), prod(A[:m, :k], B[:k, :n]))
 
 
+@pytest.mark.parametrize("room", ["own", "none"])
+@pytest.mark.parametrize("fa,fb", [(O.FP8_E4M3, O.FP8_E4M3), (O.FP8_E5M2, O.FP8_E4M3), (O.FP8_E4M3, O.FP8_E5M2)])
+@pytest.mark.parametrize("M,N,K,a_off,b_off", [(70, 200, 1003, 0, 0), (600, 100, 333, 1, 0), (33, 68, 512, 3, 0), (5, 66, 1024, 0, 2),
+                                               (1, 1, 17, 0, 0), (520, 272, 272, 1, 0)])
+def test_fp8_kn_off_alignment_sums_in_fp32(ascq_gpu, fa, fb, M, N, K, a_off, b_off, room):
+    """fp8 B [K, N] with a ragged K or N or off its alignment, f32 C: one product of 1 and small ones of 2^-15 in every group of
+    16 K.  fp32 sums keep them all (exactly: multiples of 2^-15 below 2^9); the fp8 MFMAs would drop them.  With 16-byte
+    multiples from 512 rows on (the last case) the call is on the fp8 MFMAs, aligned or not: their bound of 2^-13"""
+    t8 = {O.FP8_E4M3: torch.float8_e4m3fn, O.FP8_E5M2: torch.float8_e5m2}
+    a, b = torch.full((M, K), 2.0 ** -8), torch.full((K, N), 2.0 ** -7)
+    a[:, ::16], b[::16] = 1.0, 1.0
+    want = a.double() @ b.double()
+    mm = ascq_gpu.Matmul(fa, fb, ascq_gpu.F32)
+    mm.SetOrgShape(M, N, K)
+    code = lambda x, t: x.to(t).view(torch.uint8).numpy()  # noqa: E731
+    mm.SetTensorA(_dev_at(code(a, t8[fa]), a_off))
+    mm.SetTensorB(_dev_at(code(b, t8[fb]), b_off))
+    if room == "none":
+        _no_room(mm)
+    for _ in range(2):
+        c = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+        mm.IterateAll(c)
+        if M >= 512 and K % 16 == 0 and N % 16 == 0:
+            assert float((c.cpu().double() - want).abs().max()) <= 2.0 ** -13 * K
+        else:
+            assert torch.equal(c.cpu().double(), want)
+
+
+def test_fp8_kn_off_alignment_special_values(ascq_gpu):
+    """NaN and infinities (e5m2) of operands that are decoded to bf16 rows, and of the bytes around them"""
+    M, N, K = 40, 50, 77
+    g = torch.Generator().manual_seed(9)
+    a, b = torch.randn((M, K), generator=g).to(torch.float8_e5m2), torch.randn((K, N), generator=g).to(torch.float8_e5m2)
+    a[3, 5], a[7, 76], b[20, 9], b[76, 49] = float("nan"), float("inf"), float("-inf"), float("nan")
+    buf = torch.full((M * K + 33,), 0x7F, dtype=torch.uint8, device="cuda")
+    buf[1:1 + M * K] = a.view(torch.uint8).reshape(-1).cuda()
+    mm = ascq_gpu.Matmul(ascq_gpu.FP8_E5M2, ascq_gpu.FP8_E5M2, ascq_gpu.F32)
+    mm.SetOrgShape(M, N, K)
+    mm.SetTensorA(buf[1:1 + M * K])
+    mm.SetTensorB(b.cuda())
+    c = torch.zeros((M, N), device="cuda")
+    mm.IterateAll(c)
+    want = a.float() @ b.float()
+    got = c.cpu()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    f = want.isfinite()
+    np.testing.assert_allclose(got[f].numpy(), want[f].numpy(), rtol=1e-5, atol=1e-4)
+
+
 _LOG_SCRIPT = r"""
 import sys
 sys.path.insert(0, {pkg!r})
