@@ -296,8 +296,8 @@ ascq_status split_region(ascq_matmul_s* h, int64_t m, int64_t n, int64_t k, uint
     return ASCQ_OK;
 }
 
-// int8 / fp8 operands after the copies to the workspace (bytes_transposes_a, bytes_nz_b) and the packing: pointers, leading dimensions
-// (org shape) and the layouts the GEMM sees
+// int8 / fp8 operands after the copies to the workspace (bytes_transposes_a, bytes_nz_b) and the packing: pointers, leading
+// dimensions (org shape) and the layouts the GEMM sees
 struct ByteOperands {
     const uint8_t* A;
     const uint8_t* B;
