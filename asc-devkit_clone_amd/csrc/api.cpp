@@ -466,7 +466,8 @@ ascq_status pack_byte_operands(ascq_matmul_s* h, hipStream_t st, int64_t m, int6
     uint8_t* pa = nullptr;
     if (h->ws && !h->ws_owned) {
         const size_t base = pack_base(h, m, n, *k);
-        if (h->ws_bytes < base + need) return ASCQ_OK;
+        // (rows are packed 16 bytes at a time: not into a workspace off that alignment)
+        if (h->ws_bytes < base + need || (uintptr_t)h->ws % 16 != 0) return ASCQ_OK;
         pa = (uint8_t*)h->ws + base;
         o.ws_end = base;
     } else {

@@ -220,8 +220,9 @@ ascq_status ascq_matmul_set_tensor_scale_b(ascq_matmul_t h, const uint8_t* scale
  * B; int4; MX; hifloat8; W4/W8 with ND B) allocate it on first use when none is set.  Two parts of the figure are optional,
  * and a caller's workspace without them is accepted: the partials of the K split at decode-sized batches, and room to pack
  * int8 / fp8 operands whose rows or pointers are off their alignment (16 bytes; a [K, N] B 4) or whose K is not a multiple
- * of 16 (fp8 with B [K, N]: as bf16 rows, or N not a multiple of 4) -- it depends on the pointers and the single shape set when the size is asked for.  Without the room such calls run
- * on slower any-alignment kernels.  A handle without a caller's workspace allocates room for packing itself, per stream
+ * of 16 (fp8 with B [K, N]: as bf16 rows, or N not a multiple of 4) -- it depends on the pointers and the single shape set
+ * when the size is asked for.  Without the room, or with a workspace off 16 bytes itself, such calls run on slower
+ * any-alignment kernels.  A handle without a caller's workspace allocates room for packing itself, per stream
  * (four at most; from the second call on where one call would not repay it), but neither under stream capture nor in
  * ascq_matmul_iterate_all_noalloc: give a handle a workspace to have its captured calls packed. */
 ascq_status ascq_matmul_workspace_size(ascq_matmul_t h, size_t* bytes);

@@ -71,6 +71,7 @@ hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* s)
 namespace ascq {
 hipError_t launch_pack_rows(const PackRows& a, const PackRows& b, hipStream_t)
 {
+    if ((uintptr_t)a.dst % 16 != 0 || (uintptr_t)b.dst % 16 != 0) return hipErrorInvalidValue;  // (as the launcher does)
     if (a.dst) use(a.dst, (size_t)a.rows * ((a.cols + 15) / 16 * 16), "packed A");
     if (b.dst) use(b.dst, (size_t)b.rows * ((b.cols + 15) / 16 * 16), "packed B");
     return hipSuccess;
@@ -78,6 +79,7 @@ hipError_t launch_pack_rows(const PackRows& a, const PackRows& b, hipStream_t)
 hipError_t launch_byte_to_bf16(uint16_t* dst, int64_t ldd, const uint8_t*, int64_t, int64_t rows, int64_t, int, int transpose,
                                hipStream_t)
 {
+    if ((uintptr_t)dst % 16 != 0) return hipErrorInvalidValue;  // (as the launcher does)
     use(dst, (size_t)(rows * ldd) * 2, transpose ? "packed B (bf16)" : "packed A (bf16)");
     return hipSuccess;
 }

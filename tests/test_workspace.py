@@ -47,3 +47,9 @@ def test_allocation_free_calls_pack_nothing(tmp_path):
     """IterateAllNoAlloc with operands off their alignment does not pack them into the scratch that all handles share"""
     r = _run(tmp_path, "workspace_noalloc")
     assert r.returncode == 0, r.stdout[-3000:] + r.stderr[-2000:]
+
+
+def test_workspace_off_its_alignment_is_not_packed_into(tmp_path):
+    """A caller's workspace off 16 bytes: calls whose operands would be packed there run without, and none is refused"""
+    r = _run(tmp_path, "workspace_offset")
+    assert r.returncode == 0, r.stdout[-3000:] + r.stderr[-2000:]
